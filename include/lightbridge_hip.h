@@ -393,8 +393,8 @@ lbh_status lbh_moe_set_batch_tiles(lbh_moe *moe, int32_t tokens_per_chunk, int32
 
 /* Engine of the batched IQ2_S / IQ3_S streams (no counterpart in the reference,
  * whose batch is a loop over tokens).  Chunks of at least mx_min_tokens tokens
- * (1..16; default 4) run on the f16 matrix cores, one 16-row x 16-token product
- * per codebook step, with mx_rows_gate_up / mx_rows_down rows per workgroup
+ * (1..16; default 4) run on the int8 matrix cores, one 16-row x 16-token product
+ * per block, with mx_rows_gate_up / mx_rows_down rows per workgroup
  * (16, 32 or 64; 0: the defaults 16 and 32); smaller chunks run on the VALU
  * integer dots; mx_min_tokens = 0
  * keeps every chunk on the VALU.  Every choice gives the same bits.  Resets the
@@ -409,7 +409,8 @@ lbh_status lbh_moe_set_batch_engine(lbh_moe *moe, int32_t mx_min_tokens, int32_t
  * apart, so each step reads 16 pieces of 16 cache lines whose other pieces come
  * back in later steps.  This call gives the IQ2_S / IQ3_S gate, up and down
  * matrices (rows a multiple of 16) of the listed routed experts a second copy,
- * owned by the layer, with the 16 rows of every block adjacent.  The
+ * owned by the layer, with the 16 rows of every block adjacent (and a block's
+ * bytes in the order the streams' lanes read them).  The
  * matrix-core streams then read those copies; every other kernel keeps reading
  * the caller's matrices.  The results are the same bits.  The cost is a second
  * copy of those bytes in HBM (lbh_moe_batch_tile_copy_bytes).

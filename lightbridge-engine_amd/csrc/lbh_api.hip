@@ -854,6 +854,8 @@ struct lbh_moe {
     int tc, rt_gu_r, rt_gu_s, rt_d_r, rt_d_s;
     int mx_min;               // batched IQ chunks of >= mx_min tokens on the matrix cores (0: none)
     int mx_split_gu, mx_split_d;   // waves sharing a 16-row tile of those streams (1, 2, 4)
+    int mx_rows_gu, mx_rows_d;     // rows per workgroup at one wave per tile
+    int tile_copies;               // routed experts with tile copies: 0 none, 1 some, 2 all
     hipStream_t side;         // batched calls: second stream and fork/join events
     hipEvent_t ev[4];
     uint8_t *shared_gemm_mem; // MFMA-ready copies of a K-quant shared expert (batched calls)
@@ -884,6 +886,7 @@ constexpr int MX_MIN_DEFAULT = 4;
 void set_batch_defaults(lbh_moe *m, int mx_min) {
     m->mx_min = mx_min;
     m->mx_split_gu = 4, m->mx_split_d = 2;
+    m->mx_rows_gu = 64, m->mx_rows_d = 256;
     m->tc = mx_min > 0 ? 16 : 8;
     m->rt_gu_r = 64, m->rt_gu_s = 64, m->rt_d_r = 160, m->rt_d_s = 64;
 }
@@ -1579,6 +1582,9 @@ BatchArgs batch_args(const lbh_moe *m, const uint32_t *ids, const float *coefs, 
     a.mx_min = m->mx_min > 0 ? m->mx_min : BATCH_MAX_TC + 1;
     a.mx_split_gu = m->mx_split_gu;
     a.mx_split_d = m->mx_split_d;
+    a.mx_rows_gu = m->mx_rows_gu;
+    a.mx_rows_d = m->mx_rows_d;
+    a.mx_copies = m->tile_copies;
     a.vc = a.mx ? (a.tc < a.mx_min - 1 ? a.tc : a.mx_min - 1) : a.tc;
     if (a.vc < 1) a.vc = 1;
     return a;
@@ -1817,6 +1823,9 @@ lbh_status lbh_moe_make_batch_tile_copies(lbh_ctx *ctx, lbh_moe *m, const uint32
     m->tile_mem = mem;
     m->tile_bytes = total;
     m->experts_mx_dev = table;
+    size_t picked = 0;
+    for (size_t e = 0; e < m->n_experts; ++e) picked += pick[e] ? 1 : 0;
+    m->tile_copies = !table ? 0 : picked < m->n_experts ? 1 : 2;
     set_engine_for_copies(m, table != nullptr);
     return ok(err);
 }

@@ -39,11 +39,13 @@ constexpr int MB_WAVES = MB_THREADS / 64;
 constexpr int Q8L = 304;
 
 // Matrix-core operand copy of Q8_K rows, written beside the GGML bytes by the
-// quantize kernels: block k's 256 quants XOR 0x80 (as unsigned bytes, q + 128)
-// at q + 256 k, its scale at d[k].
+// quantize kernels: block k's 256 quants at q + 256 k, its scale at d[k].
+// split: in the order of the IQ3_S instructions (dword 2g + h of lane quarter
+// p holds elements 32g + 8p + 4h .. + 3), else in element order (IQ2_S).
 struct MxRows {
     uint8_t *q;
     float *d;
+    bool split;
 };
 
 __host__ __device__ constexpr int al16(int v) { return (v + 15) & ~15; }
@@ -423,8 +425,10 @@ __device__ __forceinline__ void quantize_rows_out(const float *x, long long nblo
     if (mx.q) {
         for (int k = lane; k < (int)cnt * 64; k += 64) {
             const int blk = k >> 6, w = k & 63;
-            const uint32_t v = *reinterpret_cast<const uint32_t *>(lds_wave + blk * 292 + 4 + 4 * w);
-            reinterpret_cast<uint32_t *>(mx.q)[(first + blk) * 64 + w] = v ^ 0x80808080u;
+            // w: destination dword, from source dword sw
+            const int sw = mx.split ? 8 * ((w >> 1) & 7) + 2 * (w >> 4) + (w & 1) : w;
+            reinterpret_cast<uint32_t *>(mx.q)[(first + blk) * 64 + w] =
+                *reinterpret_cast<const uint32_t *>(lds_wave + blk * 292 + 4 + 4 * sw);
         }
         if (lane < cnt) mx.d[first + lane] = *reinterpret_cast<const float *>(lds_wave + lane * 292);
     }
@@ -457,7 +461,7 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_prep(BatchArgs a) {
         const bool rm = a.has_shared && !a.shared_gemm && (a.shared.gate.type == T_Q4_K || a.shared.gate.type == T_Q5_K);
         if (first < nblocks)
             quantize_rows_out(a.x + first * 256, nblocks, first, a.q8x, rm ? a.q8x_rm : nullptr,
-                              smem + (tid >> 6) * 4 * 292, MxRows{a.mx ? a.xq_mx : nullptr, a.xd_mx});
+                              smem + (tid >> 6) * 4 * 292, MxRows{a.mx ? a.xq_mx : nullptr, a.xd_mx, false});
         return;
     }
     const int NE = a.n_experts, T = a.n_tokens, K = a.top_k, TC = a.tc;
@@ -647,12 +651,12 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_quant_h(BatchArgs a, int shar
     };
     if (chunk < br) {
         swiglu_blocks(a.g_r, a.u_r, chunk, br);
-        quantize_rows_out(&hbuf[wid][0], br, chunk, a.q8h_r, nullptr, lw, MxRows{a.mx ? a.hq_mx_r : nullptr, a.hd_mx_r});
+        quantize_rows_out(&hbuf[wid][0], br, chunk, a.q8h_r, nullptr, lw, MxRows{a.mx ? a.hq_mx_r : nullptr, a.hd_mx_r, a.type_down_r == T_IQ3_S});
     } else if (chunk >= brp && chunk - brp < bs) {
         const long long f = chunk - brp;
         swiglu_blocks(a.g_s, a.u_s, f, bs);
         quantize_rows_out(&hbuf[wid][0], bs, f, shared_mode == 1 ? nullptr : a.q8h_s, shared_mode == 1 ? a.q8h_s : nullptr,
-                          lw, MxRows{a.mx && shared_mode == 0 ? a.hq_mx_s : nullptr, a.hd_mx_s});
+                          lw, MxRows{a.mx && shared_mode == 0 ? a.hq_mx_s : nullptr, a.hd_mx_s, a.shared.down.type == T_IQ3_S});
     }
 }
 
@@ -707,320 +711,412 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_down(BatchArgs a) {
 
 // ==================================================== IQ streams on the matrix cores
 //
-// The IQ2_S / IQ3_S gate/up and down streams as f16 matrix-core products
-// (v_mfma_f32_16x16x32_f16), bit-identical to the dot4 streams above: per
-// (row, token, block) the integer block sum is formed exactly and folded in
-// the reference's order.
+// The IQ2_S / IQ3_S gate/up and down streams as int8 matrix-core products,
+// bit-identical to the dot4 streams above: per (row, token, block) the integer
+// block sum is formed exactly and folded in the reference's order.
 //
-// Wave tile: 16 rows x the chunk's tokens (up to 16) per block.  Lane l holds
-// row l % 16 of the A operand and token l % 16 of the B operand, both for the
-// block's elements 64 (l / 16) + 8 m .. + 7 in instruction m (m = 0..7): A and
-// B use the same (lane, slot) -> element map, so each instruction contracts 32
-// elements of the block whatever its internal k order.  The lane's slice of
-// its row is the four-lane part l / 16 of the unit (load_slice<TY, 4>).
-//   A: one codebook entry (IQ2_S: one 8-element grid entry; IQ3_S: two
-//      4-element entries) from LDS tables of f16 magnitudes, the eight sign
-//      bits applied by XOR with an f16 sign-mask table entry, times the
-//      entry's integer scale (IQ2_S 1 + 2 nibble per 16 elements, IQ3_S
-//      2 nibble + 1 per 32): |A| <= 43 * 31 = 1333 (IQ2_S), 15 * 31 = 465
-//      (IQ3_S), integers an f16 holds exactly.
-//   B: the Q8_K quants (|B| <= 128) from the operand copy of q + 128 as
-//      unsigned bytes: 0x6400 | (q + 128) is the f16 1024 + q + 128, and one
-//      packed f16 subtraction of 1152 leaves q exactly.
-// Every product is an integer below 2^18 and every partial sum of a chain of
-// instructions stays below 2^24 (IQ2_S: chains of three instructions, 96
-// elements, 96 * 1333 * 128 < 2^24; IQ3_S: the whole block, 256 * 465 * 128 <
-// 2^24), so the f32 accumulation is exact in any order; each chain converted
-// to int32 and summed gives the reference's integer block sum (q8_k.rs:337-364,
-// :380-428, integer additions, exact in any order).  The fold is the one of
+// Wave tile: the chunk's tokens (up to 16, operand A) x 16 weight rows
+// (operand B) per block.  Lane l = 16 q + c supplies token c of A and row c of
+// B for the same elements of the block, so an instruction contracts identical
+// elements whatever its internal k order; result i of the lane is (token
+// 4q + i, row c), so the row's d and scales are the lane's own.
+//   IQ2_S: v_mfma_i32_16x16x64_i8; instruction m contracts the lane's 16
+//     elements 64q + 16m .. + 15, one scale (half group).  The scaled weight
+//     +-{8, 25, 43} (1 + 2 nibble) is split as 256 hi + lo into two signed
+//     bytes, each a v_perm by the weight's code and sign from a table of the
+//     scale (16 entries x 16 bytes in LDS): two chains over the whole block,
+//     bsum = 256 sum_hi + sum_lo, no multiply per scale.
+//   IQ3_S: v_mfma_i32_16x16x32_i8; instruction g contracts group g (lane:
+//     elements 32g + 8q .. + 7), whose scale multiplies the 32-bit result
+//     (bsum += (2 nibble + 1) * result: 24-bit operands).  The signed bytes
+//     come from the 32 KiB signed table, one word per four weights.
+// The sums are int32 throughout, hence exact in any order, and equal the
+// reference's (q8_k.rs:337-364, :380-428).  The fold is the one of
 // lbh_rows.h: term = (d * d8) * (float)bsum, chain += term in block order,
 // IQ2_S result = 0.125 * chain.
+//
+// What bounds it: VALU issue (about 118 instructions per IQ2_S matrix, 16 rows
+// and block, 128 for IQ3_S; busy 72% and 62% of the time), beside the codebook
+// reads of the LDS.  As f16 products (v_mfma_f32_16x16x32_f16 on pre-scaled f16
+// weights) the same tile took about twice the VALU work: f16 signs and scales
+// for the weights, f16 conversions of the quants.  Measured on 192 experts of
+// hidden 4096, width 1536, top-8 Zipf(1.1), tile copies, kernel times:
+//   64 tokens   gate/up 159 -> 88 us, down 91 -> 61 us (step 417 -> 354 us)
+//   256 tokens  gate/up 375 -> 222 us, down 242 -> 143 us (step 832 -> 611 us)
 
-typedef _Float16 mx_h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 mx_h2 __attribute__((ext_vector_type(2)));
-typedef float mx_f4 __attribute__((ext_vector_type(4)));
-typedef uint32_t mx_u4 __attribute__((ext_vector_type(4)));
+typedef int mx_i4 __attribute__((ext_vector_type(4)));
 
 constexpr int MX_THREADS = 256;
 constexpr int MX_WAVES = MX_THREADS / 64;
+constexpr int MX_MAX_NB = 64;
 
+// IQ2_S scaled weights by scale nibble n: bytes 0-2 of {lo+, lo-, hi+, hi-} are
+// the split +-m (1 + 2n) = 256 hi + lo (lo signed) of m = 8, 25, 43.
+struct MxProducts {
+    uint32_t v[16][4];
+    constexpr MxProducts() : v{} {
+        const int mag[3] = {8, 25, 43};
+        for (int n = 0; n < 16; ++n)
+            for (int sg = 0; sg < 2; ++sg)
+                for (int c = 0; c < 3; ++c) {
+                    const int p = (sg ? -1 : 1) * mag[c] * (1 + 2 * n);
+                    const int low = p & 0xff, lo = low >= 128 ? low - 256 : low, hi = (p - lo) / 256;
+                    v[n][sg] |= (uint32_t)low << (8 * c);
+                    v[n][2 + sg] |= (uint32_t)(hi & 0xff) << (8 * c);
+                }
+    }
+};
+static __constant__ MxProducts c_mx_products = MxProducts();
 
-// LDS tables: the f16 magnitudes of every codebook entry (IQ2_S 1024 x 8, the
-// entry of index q | h << 8 at byte 2 * iq2s_code_addr(q, h); IQ3_S 512 x 4),
-// then for IQ3_S 256 sign masks of eight f16 (bit 15 of element i is bit i of
-// the sign byte); built at compile time, copied to LDS per workgroup.
+// LDS tables of a stream: IQ2_S the byte codes (GridLDS image) and the scaled
+// weights, IQ3_S the signed table.
 template <int TY>
 struct MxTab {
-    static constexpr int ENTRY = TY == T_IQ2_S ? 16 : 8;
-    static constexpr int GRID = (TY == T_IQ2_S ? 1024 : 512) * ENTRY;
-    static constexpr int SIGNS = TY == T_IQ3_S ? 256 * 16 : 0;
-    static constexpr int BYTES = GRID + SIGNS;
+    static constexpr int GRID = TY == T_IQ2_S ? GridLDS<T_IQ2_S>::BYTES : GridLDS<T_IQ3S_SGN>::BYTES;
+    static constexpr int BYTES = GRID + (TY == T_IQ2_S ? 256 : 0);
 };
-
-// f16 bits of a non-negative integer below 2048 (exact).
-constexpr uint32_t f16_bits_of(uint32_t v) {
-    if (v == 0) return 0;
-    int e = 0;
-    while ((v >> (e + 1)) != 0) ++e;
-    return ((uint32_t)(e + 15) << 10) | ((v << (10 - e)) & 0x3ffu);
-}
-
-constexpr uint64_t k_iq2s_vals[1024] = {LBH_IQ2S_GRID_VALUES};
-constexpr uint32_t k_iq3s_vals[512] = {LBH_IQ3S_GRID_VALUES};
-
-struct MxTables {
-    uint32_t iq2[1024][4];
-    uint32_t iq3[512][2];
-    uint32_t sign[256][4];
-};
-
-constexpr uint32_t f16_pair_of(uint32_t lo, uint32_t hi) { return f16_bits_of(lo) | (f16_bits_of(hi) << 16); }
-
-constexpr MxTables make_mx_tables() {
-    MxTables t{};
-    for (int i = 0; i < 1024; ++i)
-        for (int k = 0; k < 4; ++k)
-            t.iq2[iq2s_code_addr((uint32_t)i & 255u, (uint32_t)i >> 8) / 8][k] =
-                f16_pair_of((uint32_t)(k_iq2s_vals[i] >> (16 * k)) & 0xffu,
-                            (uint32_t)(k_iq2s_vals[i] >> (16 * k + 8)) & 0xffu);
-    for (int i = 0; i < 512; ++i)
-        for (int k = 0; k < 2; ++k)
-            t.iq3[i][k] = f16_pair_of((k_iq3s_vals[i] >> (16 * k)) & 0xffu, (k_iq3s_vals[i] >> (16 * k + 8)) & 0xffu);
-    for (uint32_t v = 0; v < 256; ++v)
-        for (int k = 0; k < 4; ++k)
-            t.sign[v][k] = (((v >> (2 * k)) & 1u) << 15) | (((v >> (2 * k + 1)) & 1u) << 31);
-    return t;
-}
-
-static __constant__ MxTables c_mx_tab = make_mx_tables();
-
-__device__ __forceinline__ uint32_t mx_bits(mx_h2 v) { return __builtin_bit_cast(uint32_t, v); }
-__device__ __forceinline__ mx_h2 mx_pair(uint32_t v) { return __builtin_bit_cast(mx_h2, v); }
 
 // Copies TY's tables into LDS (all threads; the caller synchronises).
 template <int TY>
 __device__ __forceinline__ void mx_fill(uint8_t *tab) {
-    const uint4 *g = reinterpret_cast<const uint4 *>(TY == T_IQ2_S ? &c_mx_tab.iq2[0][0] : &c_mx_tab.iq3[0][0]);
-    const uint4 *sg = reinterpret_cast<const uint4 *>(&c_mx_tab.sign[0][0]);
+    const uint4 *g = grid_image<TY == T_IQ2_S ? T_IQ2_S : T_IQ3S_SGN>();
     uint4 *o = reinterpret_cast<uint4 *>(tab);
-    for (int i = threadIdx.x; i < MxTab<TY>::GRID / 16; i += MX_THREADS) o[i] = g[i];
-    if constexpr (MxTab<TY>::SIGNS > 0)
-        for (int i = threadIdx.x; i < 256; i += MX_THREADS) o[MxTab<TY>::GRID / 16 + i] = sg[i];
+#pragma unroll
+    for (int i = 0; i < MxTab<TY>::GRID / 16 / MX_THREADS; ++i) o[threadIdx.x + i * MX_THREADS] = g[threadIdx.x + i * MX_THREADS];
+    if (TY == T_IQ2_S && threadIdx.x < 16)
+        o[MxTab<TY>::GRID / 16 + threadIdx.x] = reinterpret_cast<const uint4 *>(&c_mx_products.v[0][0])[threadIdx.x];
 }
 
-// Eight f16 magnitudes with their signs applied, times the integer scale ls.
-__device__ __forceinline__ mx_h8 mx_signed_scaled(uint4 mag, uint4 sgn, uint32_t ls) {
-    const _Float16 f = (_Float16)(float)ls;
-    const mx_h2 s = {f, f};
-    const mx_u4 r = {mx_bits(mx_pair(mag.x ^ sgn.x) * s), mx_bits(mx_pair(mag.y ^ sgn.y) * s),
-                     mx_bits(mx_pair(mag.z ^ sgn.z) * s), mx_bits(mx_pair(mag.w ^ sgn.w) * s)};
-    return __builtin_bit_cast(mx_h8, r);
-}
-
-// A operand of instruction m: the lane's slice holds sub-blocks 2p, 2p + 1;
-// m covers entry m % 4 of sub-block m / 4 (q8_k.rs:337-364 index, sign and
-// scale layout, read from the device encoding as slice_sum in lbh_dev.h).
-// The sign of weight 4t + i sits at bit t of byte i of the group's sign dword:
-// (b0, b0, b1, b1) << (7 - t) puts those of weights 4t, 4t + 1 at bits 15 and
-// 31, the sign bits of the f16 pair (b2, b2, b3, b3: weights 4t + 2, 4t + 3).
-__device__ __forceinline__ mx_h8 mx_a(const WSlice<T_IQ2_S, 4> &w, const uint8_t *tab, int m) {
-    const int g = m >> 2, lg = m & 3;
-    const Iq2sGroup q = iq2s_group(w, g);
-    const uint4 mag = *reinterpret_cast<const uint4 *>(tab + 2 * q.addr(lg));
-    const uint32_t p01 = perm(q.s, q.s, 0x01010000u), p23 = perm(q.s, q.s, 0x03030202u);
-    const int t0 = 2 * lg, t1 = 2 * lg + 1;
-    const uint4 sgn = make_uint4((p01 << (7 - t0)) & 0x80008000u, (p23 << (7 - t0)) & 0x80008000u,
-                                 (p01 << (7 - t1)) & 0x80008000u, (p23 << (7 - t1)) & 0x80008000u);
-    const uint32_t ls = 1u + 2u * ((byte_of(w.sc, g) >> (4 * (lg >> 1))) & 15u);
-    return mx_signed_scaled(mag, sgn, ls);
-}
-
-// IQ3_S (q8_k.rs:380-428): instruction m covers the two 4-element entries of
-// eighth m % 4 of sub-block m / 4, the sign byte's low nibble on the first.
-__device__ __forceinline__ mx_h8 mx_a(const WSlice<T_IQ3_S, 4> &w, const uint8_t *tab, int m) {
-    const int g = m >> 2, lg = m & 3;
-    const uint32_t h = byte_of(w.qh, g);
-    const uint32_t qq = w.qs[2 * g + (lg >> 1)];
-    const int sh = 16 * (lg & 1);
-    const uint32_t i1 = ((qq >> sh) & 0xffu) | ((h << (8 - 2 * lg)) & 0x100u);
-    const uint32_t i2 = ((qq >> (sh + 8)) & 0xffu) | ((h << (7 - 2 * lg)) & 0x100u);
-    const uint2 m1 = reinterpret_cast<const uint2 *>(tab)[i1], m2 = reinterpret_cast<const uint2 *>(tab)[i2];
-    const uint4 sgn = reinterpret_cast<const uint4 *>(tab + MxTab<T_IQ3_S>::GRID)[byte_of(w.sg[g], lg)];
-    const uint32_t ls = 2u * ((w.sc >> (4 * g)) & 15u) + 1u;
-    return mx_signed_scaled(make_uint4(m1.x, m1.y, m2.x, m2.y), sgn, ls);
-}
-
-// B operand: eight biased quants (two dwords) as f16.
-__device__ __forceinline__ mx_h8 mx_b(uint32_t x0, uint32_t x1) {
-    const mx_h2 off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    const mx_u4 r = {mx_bits(mx_pair(perm(0x64646464u, x0, 0x04010400u)) + off),
-                     mx_bits(mx_pair(perm(0x64646464u, x0, 0x04030402u)) + off),
-                     mx_bits(mx_pair(perm(0x64646464u, x1, 0x04010400u)) + off),
-                     mx_bits(mx_pair(perm(0x64646464u, x1, 0x04030402u)) + off)};
-    return __builtin_bit_cast(mx_h8, r);
-}
-
+// One lane's 64 weights of its row's block.
+//   IQ2_S  w: qs of its two groups, sg: their sign dwords, e: low nibble of
+//          byte j the groups' qh fields of lookup j; TILE: high nibble of byte
+//          j the scale nibble of half group j, else sc holds the four nibbles.
+//   IQ3_S  w: lookup bytes of four quads (below), sg: their sign dwords;
+//          qh, sc: the row's qh bytes and scale nibbles, all groups.
 template <int TY>
-constexpr int mx_chain() {
-    return TY == T_IQ2_S ? 3 : 8;   // instructions per exact f32 chain
-}
-
-// One wave step's inputs: the lane's slices of NM matrices and the block of
-// its token from the operand copy.
-template <int TY, int NM>
-struct MxStep {
-    WSlice<TY, 4> w[NM];
-    uint4 bq[4];
-    float d8;
+struct MxW;
+template <>
+struct MxW<T_IQ2_S> {
+    uint32_t w[2], sg[2], e, sc, d;
+};
+template <>
+struct MxW<T_IQ3_S> {
+    uint32_t w[4], sg[2], qh[2], sc, d;
 };
 
-// LDS of a matrix-core stream workgroup: the tables, then (split > 1) per
-// tile the per-block f32 terms [matrix][block][token][row].
-__host__ __device__ constexpr int mx_lds_bytes(int ty, int nm, int split, int nb) {
-    return (ty == T_IQ2_S ? MxTab<T_IQ2_S>::BYTES : MxTab<T_IQ3_S>::BYTES) +
-           (split > 1 ? (MX_WAVES / split) * nm * nb * 256 * 4 : 0);
+typedef uint32_t mx_u3 __attribute__((ext_vector_type(3)));
+
+// TILE: the matrix is a 16-row tile copy (k_units_to_tiles), whose lane slices
+// lie in lane order: u is the tile's first unit.  Else the row-major device
+// layout: u is the lane's unit.
+template <bool TILE>
+__device__ __forceinline__ void mx_load(const Planes &P, uint32_t u, int lane, MxW<T_IQ2_S> &o) {
+    const int q = lane >> 4;
+    if constexpr (TILE) {
+        const uint4 a = bld128(P, u * 64 + 16u * lane, 0);
+        o.w[0] = a.x, o.w[1] = a.y, o.sg[0] = a.z, o.sg[1] = a.w;
+        o.e = bld32(P, u * 16 + 4u * lane, 4 * P.U16);
+        o.d = bld16(P, u * 2 + 2u * (lane & 15), 5 * P.U16);
+        o.sc = 0;
+    } else {
+        const uint32_t u16 = u * 16, po = (uint32_t)(q >> 1) * P.U16 + 8u * (uint32_t)(q & 1);
+        const uint2 a = bld64(P, u16 + po, 0), c = bld64(P, u16 + po, 2 * P.U16);
+        o.w[0] = a.x, o.w[1] = a.y, o.sg[0] = c.x, o.sg[1] = c.y;
+        o.e = bld32(P, u16 + 4u * (uint32_t)(q >> 1), 4 * P.U16);
+        o.sc = bld16(P, u16 + 8u + 2u * (uint32_t)q, 4 * P.U16);
+        o.d = bld16(P, u * 2, 5 * P.U16);
+    }
+}
+template <bool TILE>
+__device__ __forceinline__ void mx_load(const Planes &P, uint32_t u, int lane, MxW<T_IQ3_S> &o) {
+    const int q = lane >> 4;
+    uint4 a;
+    uint2 s;
+    if constexpr (TILE) {
+        a = bld128(P, u * 64 + 16u * lane, 0);
+        s = bld64(P, u * 32 + 8u * lane, 4 * P.U16);
+        u += lane & 15;
+    } else {
+        a = bld128(P, u * 16 + (uint32_t)q * P.U16, 0);
+        s = bld64(P, u * 16 + (uint32_t)(q >> 1) * P.U16 + 8u * (uint32_t)(q & 1), 4 * P.U16);
+    }
+    const mx_u3 t = __builtin_bit_cast(mx_u3, __builtin_amdgcn_raw_buffer_load_b96(P.rsrc, u * 12, 6 * P.U16, WEIGHT_CPOL));
+    o.w[0] = a.x, o.w[1] = a.y, o.w[2] = a.z, o.w[3] = a.w;
+    o.sg[0] = s.x, o.sg[1] = s.y;
+    o.qh[0] = t.x, o.qh[1] = t.y, o.sc = t.z;
+    o.d = bld16(P, u * 2, 6 * P.U16 + 12 * P.U);
 }
 
-// Rows [r0, r1) (r1 - r0 <= 16 * MX_WAVES / S) of NM matrices (K = 256 nb)
-// against the chunk's tokens.  The workgroup holds MX_WAVES / S tiles of 16
-// rows; the S waves of a tile take its blocks j, j + S, ...: together they
-// read S consecutive blocks of each row (adjacent 16-byte pieces of the same
-// lines) per step.  With S > 1 each wave writes the f32 term
-// (d * d8) * (float)bsum of each (row, token, block) it computes to LDS;
-// after a workgroup barrier one thread per (tile, token, row) folds its terms
-// in block order (lbh_rows.h: chain = 0 + t_0 + t_1 + ...; IQ2_S result =
-// 0.125 * chain) and calls out(token column, row, values).  With S = 1 the
-// wave computes every block of its tile in order and each lane keeps the
-// chains of its four (row, token) results in registers (no term table, so
-// the workgroup's LDS is the tables alone).  Lane l's token column holds the
-// operand row bq / bd.  The first step's loads are issued before `prologue`
-// (table fill, ended by a workgroup barrier); then each step's loads are in
-// flight while the one before is computed.
-template <int TY, int NM, int S, class Prologue, class Out>
-__device__ __forceinline__ void mx_tiles(const MatView (&mv)[NM], int r0, int r1, int nb, const uint8_t *bq,
-                                         const float *bd, const uint8_t *tab, float *terms, Prologue prologue, Out out) {
+__device__ __forceinline__ void lanes32_swap(uint32_t &a, uint32_t &b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+__device__ __forceinline__ void lanes16_swap(uint32_t &a, uint32_t &b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+
+// Integer block sums bs[i] of (token 4q + i, row c) from the lane's weights
+// and its 64 quants of token c (tok[m]: 16 bytes).
+template <bool TILE>
+__device__ __forceinline__ void mx_block(const MxW<T_IQ2_S> &o, const uint4 (&tok)[4], const uint8_t *tab, int lane,
+                                         int32_t (&bs)[4]) {
+    const GridRef<T_IQ2_S> grid(tab);
+    // row-major: the lane's qh fields are fields 2 (q & 1), + 1 of its dword
+    const uint32_t e = TILE ? o.e : o.e >> (4 * ((lane >> 4) & 1));
+    mx_i4 lo = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const Iq2sGroup g = Iq2sGroup::make(o.w[m >> 1], e, m >> 1, o.sg[m >> 1]);
+        const uint32_t na = TILE ? (e >> (8 * m)) & 0xf0u
+                                 : (m == 0 ? o.sc << 4 : o.sc >> (4 * m - 4)) & 0xf0u;
+        const uint4 t = *reinterpret_cast<const uint4 *>(tab + MxTab<T_IQ2_S>::GRID + na);
+        mx_i4 bl, bh;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int lg = 2 * (m & 1) + k;
+            const uint2 code = grid.code_at(g.addr(lg));
+            const uint32_t s0 = g.sel(2 * lg) | code.x, s1 = g.sel(2 * lg + 1) | code.y;
+            bl[2 * k] = (int)perm(t.y, t.x, s0), bl[2 * k + 1] = (int)perm(t.y, t.x, s1);
+            bh[2 * k] = (int)perm(t.w, t.z, s0), bh[2 * k + 1] = (int)perm(t.w, t.z, s1);
+        }
+        const mx_i4 a = __builtin_bit_cast(mx_i4, tok[m]);
+        lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bl, lo, 0, 0, 0);
+        hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bh, hi, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bs[i] = (hi[i] << 8) + lo[i];
+}
+
+// IQ3_S quads: the lane's lookups are 2q and 2q + 1 of every group; quad 0 / 1
+// holds lookup 2q / 2q + 1 of groups 0, 1, 4, 5, quad 2 / 3 those of groups 2,
+// 3, 6, 7 (byte i: the i-th listed group).  Sign dword j: byte i the sign byte
+// q of the i-th group of quads 2j, 2j + 1.  A tile copy holds them so; the
+// row-major slice of lane q is groups 2q, 2q + 1 whole, and the four lanes of
+// a row exchange 4 x 4 pieces (v_permlane32_swap / 16_swap).
+__device__ __forceinline__ void mx_iq3_exchange(const MxW<T_IQ3_S> &o, uint32_t (&qd)[4], uint32_t (&sg)[2]) {
+    // t[j]: the lookups 2j, 2j + 1 of both groups, for the row's lane j
+    uint32_t t[4] = {perm(o.w[2], o.w[0], 0x05040100u), perm(o.w[2], o.w[0], 0x07060302u),
+                     perm(o.w[3], o.w[1], 0x05040100u), perm(o.w[3], o.w[1], 0x07060302u)};
+    lanes32_swap(t[0], t[2]);
+    lanes32_swap(t[1], t[3]);
+    lanes16_swap(t[0], t[1]);
+    lanes16_swap(t[2], t[3]);
+    qd[0] = perm(t[2], t[0], 0x06040200u), qd[1] = perm(t[2], t[0], 0x07050301u);
+    qd[2] = perm(t[3], t[1], 0x06040200u), qd[3] = perm(t[3], t[1], 0x07050301u);
+    uint32_t w0 = perm(o.sg[1], o.sg[0], 0x05010400u), w1 = perm(o.sg[1], o.sg[0], 0x07030602u);
+    lanes32_swap(w0, w1);
+    sg[0] = perm(w1, w0, 0x05040100u), sg[1] = perm(w1, w0, 0x07060302u);
+    lanes16_swap(sg[0], sg[1]);
+}
+
+template <bool TILE>
+__device__ __forceinline__ void mx_block(const MxW<T_IQ3_S> &o, const uint4 (&tok)[4], const uint8_t *tab, int lane,
+                                         int32_t (&bs)[4]) {
+    const Iq3SignedRef grid(tab);
+    uint32_t qd[4] = {o.w[0], o.w[1], o.w[2], o.w[3]}, sg[2] = {o.sg[0], o.sg[1]};
+    if constexpr (!TILE) mx_iq3_exchange(o, qd, sg);
+    // bits 0, 1 of byte i: the high index bits of lookups 2q, 2q + 1
+    const uint32_t ta = o.qh[0] >> (2 * (lane >> 4)), tb = o.qh[1] >> (2 * (lane >> 4));
+    const uint32_t hb[2] = {perm(tb, ta, 0x05040100u), perm(tb, ta, 0x07060302u)};
+    uint32_t word[2][8];   // [even, odd lookup][group]
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int j = k >> 1, odd = k & 1;
+        // iq3_signed_offset = x + 256 y per byte
+        const uint32_t h = (odd ? hb[j] << 1 : hb[j] << 2) & 0x04040404u;
+        const uint32_t s = (odd ? sg[j] >> 1 : sg[j] << 3) & 0x78787878u;
+        const uint32_t x = qd[k] & 0xfcfcfcfcu, y = (qd[k] & 0x03030303u) | h | s;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            word[odd][(i & 1) + 4 * (i >> 1) + 2 * j] = grid.word(perm(y, x, 0x0c0c0000u | ((4u + i) << 8) | (uint32_t)i));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bs[i] = 0;
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+        const uint4 v = tok[g >> 1];
+        const uint2 a = (g & 1) ? make_uint2(v.z, v.w) : make_uint2(v.x, v.y);
+        const uint2 b = make_uint2(word[0][g], word[1][g]);
+        const mx_i4 zero = {0, 0, 0, 0};
+        const mx_i4 r = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, a), __builtin_bit_cast(long, b),
+                                                              zero, 0, 0, 0);
+        const int32_t ls = (int32_t)(((g == 0 ? o.sc << 1 : o.sc >> (4 * g - 1)) & 0x1eu) | 1u);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            bs[i] += mul24(r[i], ls);
+            asm("" : "+v"(bs[i]));   // one v_mad_i32_i24 each, not two products and a three-way add
+        }
+    }
+}
+
+// One wave step's inputs: NM slices of the lane's rows and its quants of
+// token c.
+template <int TY, int NM>
+struct MxStep {
+    MxW<TY> w[NM];
+    uint4 tok[4];
+};
+
+// Dynamic LDS of a matrix-core stream workgroup (beside its static tables and
+// scales): with split > 1, per tile the f32 terms [matrix][block][token][row].
+__host__ __device__ constexpr int mx_dyn_lds(int nm, int split, int nb) {
+    return split > 1 ? (MX_WAVES / split) * nm * nb * 256 * 4 : 0;
+}
+__host__ __device__ constexpr int mx_lds_bytes(int ty, int nm, int split, int nb) {
+    return (ty == T_IQ2_S ? MxTab<T_IQ2_S>::BYTES : MxTab<T_IQ3_S>::BYTES) +
+           (split > 1 ? mx_dyn_lds(nm, split, nb) : MX_MAX_NB * 16 * 4);
+}
+
+// Rows [r0, r1) (multiples of 16 NM') of NM tiles per step against the chunk's
+// tokens: the NM matrices mv (gate and up), or, PAIR, NM adjacent 16-row tiles
+// of the one matrix mv[0], which share the step's token operands.
+//   S = 1: the waves take tiles r0 + RW wid, + 4 RW, ... (RW = 16 or 16 NM
+//     rows) to r1, computing every block of a tile in order, the chains of
+//     the lane's four (token, row) results in registers; s_d8[16 b + i] is the
+//     scale of token i's block b.
+//   S > 1: the workgroup holds MX_WAVES / S tiles, the S waves of a tile take
+//     its blocks j, j + S, ... and write the f32 term (d * d8) * (float)bsum of
+//     each (row, token, block) to LDS; after a workgroup barrier one thread
+//     per (tile, token, row) folds its terms in block order (lbh_rows.h: chain =
+//     0 + t_0 + t_1 + ...) and calls out(token column, row, values).  bd: the
+//     scales of the lane's tokens, d8_of(i)[b].
+// bq: the lane's token operand row.  The first step's loads are issued before
+// `prologue` (tables and scales to LDS, ended by a workgroup barrier); then
+// each step's loads are in flight while the one before is computed.
+template <int TY, int NM, int S, bool TILE, bool PAIR, class Prologue, class D8, class Out>
+__device__ __forceinline__ void mx_tiles(const MatView *mv, int r0, int r1, int nb, const uint8_t *bq, const uint8_t *tab,
+                                         const float *s_d8, float *terms, Prologue prologue, D8 d8_of, Out out) {
+    constexpr int NP = PAIR ? 1 : NM, RW = PAIR ? 16 * NM : 16;
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, q = lane >> 4;
     const int tl = wid / S, j = wid - tl * S;
-    const int rt0 = r0 + 16 * tl;
-    const int steps = rt0 < r1 && j < nb ? (nb - j + S - 1) / S : 0;
-    Planes P[NM];
-    uint32_t po[NM];
-    int32_t order[NM];   // wave-uniform: a tile copy (MAT_TILE16) or the row-major matrix
+    const int rt0 = r0 + RW * tl;
+    // steps of the wave: its blocks of one tile (S > 1), or its tiles' blocks (S = 1)
+    const int tiles = S > 1 ? 1 : (r1 - rt0 + RW * MX_WAVES - 1) / (RW * MX_WAVES);
+    const int steps = rt0 < r1 ? (S > 1 ? (j < nb ? (nb - j + S - 1) / S : 0) : tiles * nb) : 0;
+    Planes P[NP];
 #pragma unroll
-    for (int t = 0; t < NM; ++t) {
-        P[t] = make_planes(mv[t].planes, mv[t].units, mv[t].bytes);
-        po[t] = part_offset<TY, 4>(P[t], q);
-        order[t] = __builtin_amdgcn_readfirstlane(mv[t].order);
-    }
-    // Rows past r1 load the last row (every register defined; never output).
-    int r = rt0 + c;
-    r = r < r1 ? r : r1 - 1;
-    // The loads are unconditional: a step past the wave's last one reloads a
-    // block of the row (in bounds, never used), so the compiler's wait before
-    // a step's use counts exactly the younger step's loads.
-    auto issue = [&](int s, MxStep<TY, NM> &st) {
-        int b = j + S * (s < steps ? s : steps - 1);
-        b = b < 0 ? 0 : b < nb ? b : nb - 1;
+    for (int t = 0; t < NP; ++t) P[t] = make_planes(mv[t].planes, mv[t].units, mv[t].bytes);
+    const uint8_t *tp = bq + 64 * q;
+    // The loads are unconditional: a step past the wave's last one reloads the
+    // last (in bounds, never used), so the compiler's wait before a step's use
+    // counts exactly the younger step's loads.
+    int ir = rt0 < r1 ? rt0 : r0, ib = S > 1 ? (j < nb ? j : nb - 1) : 0;   // next tile row and block to load
+    auto issue = [&](MxStep<TY, NM> &st) {
 #pragma unroll
-        for (int t = 0; t < NM; ++t) load_slice(P[t], unit_index(order[t], r, b, nb), po[t], q, st.w[t]);
-        const uint4 *src = reinterpret_cast<const uint4 *>(bq + b * 256 + 64 * q);
+        for (int t = 0; t < NM; ++t) {
+            const int r = PAIR ? ir + 16 * t : ir;
+            const uint32_t u = TILE ? (uint32_t)(r * nb + 16 * ib) : (uint32_t)((r + c) * nb + ib);
+            mx_load<TILE>(P[PAIR ? 0 : t], u, lane, st.w[t]);
+        }
+        const uint4 *src = reinterpret_cast<const uint4 *>(tp + ib * 256);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) st.bq[k] = src[k];
-        st.d8 = bd[b];
+        for (int k = 0; k < 4; ++k) st.tok[k] = src[k];
+        if constexpr (S > 1) {
+            ib = ib + S < nb ? ib + S : ib;
+        } else if (++ib == nb) {
+            if (ir + RW * MX_WAVES < r1)
+                ir += RW * MX_WAVES, ib = 0;
+            else
+                ib = nb - 1;
+        }
     };
-    float *tt = S > 1 ? terms + tl * NM * nb * 256 : terms;   // S == 1: no term table
-    float chain[NM][4];   // S == 1: result i of the lane is (row 4q + i, token c)
+    float chain[NM][4];   // S == 1
 #pragma unroll
     for (int t = 0; t < NM; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) chain[t][i] = 0.0f;
-    auto process = [&](int s, const MxStep<TY, NM> &st) {
-        constexpr int CH = mx_chain<TY>();
-        const int b = j + S * s;
-        int32_t bs[NM][4];
-        mx_f4 acc[NM];
+    int pr = rt0, pb = S > 1 ? j : 0;   // tile row and block of the step being computed
+    auto process = [&](const MxStep<TY, NM> &st) {
+        float d8[4];
+        if constexpr (S == 1) {
+            const float4 v = *reinterpret_cast<const float4 *>(s_d8 + 16 * pb + 4 * q);
+            d8[0] = v.x, d8[1] = v.y, d8[2] = v.z, d8[3] = v.w;
+        } else {
 #pragma unroll
-        for (int t = 0; t < NM; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) bs[t][i] = 0;
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            const uint4 v = st.bq[m >> 1];
-            const mx_h8 bo = (m & 1) ? mx_b(v.z, v.w) : mx_b(v.x, v.y);
-#pragma unroll
-            for (int t = 0; t < NM; ++t) {
-                const mx_h8 ao = mx_a(st.w[t], tab, m);
-                const mx_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ao, bo, m % CH == 0 ? zero : acc[t], 0, 0, 0);
-                if (m % CH == CH - 1 || m == 7) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) bs[t][i] += (int32_t)acc[t][i];
-                }
-            }
+            for (int i = 0; i < 4; ++i) d8[i] = d8_of(4 * q + i)[pb];
         }
-        // Result i of the lane is (row 4q + i, token c); row 4q + i's d is in lane 4q + i.
 #pragma unroll
         for (int t = 0; t < NM; ++t) {
-            const float da = f16_to_f32(st.w[t].d);
-            float *o = tt + ((t * nb + b) * 16 + c) * 16 + 4 * q;
+            int32_t bs[4];
+            mx_block<TILE>(st.w[t], st.tok, tab, lane, bs);
+            const float d = f16_to_f32(st.w[t].d);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float dr = __shfl(da, 4 * q + i, 64);
-                const float term = __fmul_rn(__fmul_rn(dr, st.d8), (float)bs[t][i]);
+                const float term = __fmul_rn(__fmul_rn(d, d8[i]), (float)bs[i]);
                 if constexpr (S == 1)
                     chain[t][i] = __fadd_rn(chain[t][i], term);   // blocks in order
                 else
-                    o[i] = term;
+                    terms[((tl * NM + t) * nb + pb) * 256 + 16 * (4 * q + i) + c] = term;
             }
+        }
+        if constexpr (S > 1) {
+            pb += S;
+        } else if (++pb == nb) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float res[NM];
+#pragma unroll
+                for (int t = 0; t < NM; ++t) {
+                    res[t] = TY == T_IQ2_S ? __fmul_rn(0.125f, chain[t][i]) : chain[t][i];   // q8_k.rs:369
+                    chain[t][i] = 0.0f;
+                }
+                out(4 * q + i, pr + c, res);
+            }
+            pr += RW * MX_WAVES, pb = 0;
         }
     };
     MxStep<TY, NM> sa, sb;
-    issue(0, sa);
+    issue(sa);
     prologue();
     for (int s = 0; s < steps; s += 2) {
-        issue(s + 1, sb);
-        process(s, sa);
+        issue(sb);
+        process(sa);
         if (s + 1 >= steps) break;
-        issue(s + 2, sa);
-        process(s + 1, sb);
+        issue(sa);
+        process(sb);
     }
-    if constexpr (S == 1) {
-        if (rt0 >= r1) return;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
+    if constexpr (S > 1) {
+        __syncthreads();
+        for (int p = threadIdx.x; p < (MX_WAVES / S) * 256; p += MX_THREADS) {
+            const int ptl = p >> 8, cc = (p >> 4) & 15, row = p & 15;
+            const float *src = terms + ptl * NM * nb * 256 + cc * 16 + row;
             float res[NM];
 #pragma unroll
-            for (int t = 0; t < NM; ++t) res[t] = TY == T_IQ2_S ? __fmul_rn(0.125f, chain[t][i]) : chain[t][i];  // q8_k.rs:369
-            out(c, rt0 + 4 * q + i, res);
+            for (int t = 0; t < NM; ++t) {
+                float ch = 0.0f;
+                for (int b = 0; b < nb; ++b) ch = __fadd_rn(ch, src[(t * nb + b) * 256]);
+                res[t] = TY == T_IQ2_S ? __fmul_rn(0.125f, ch) : ch;  // q8_k.rs:369
+            }
+            out(cc, r0 + 16 * ptl + row, res);
         }
-        return;
-    }
-    __syncthreads();
-    for (int p = threadIdx.x; p < (MX_WAVES / S) * 256; p += MX_THREADS) {
-        const int ptl = p >> 8, cc = (p >> 4) & 15, row = p & 15;
-        const float *src = terms + ptl * NM * nb * 256 + cc * 16 + row;
-        float res[NM];
-#pragma unroll
-        for (int t = 0; t < NM; ++t) {
-            float ch = 0.0f;
-            for (int b = 0; b < nb; ++b) ch = __fadd_rn(ch, src[(t * nb + b) * 256]);
-            res[t] = TY == T_IQ2_S ? __fmul_rn(0.125f, ch) : ch;  // q8_k.rs:369
-        }
-        out(cc, r0 + 16 * ptl + row, res);
     }
 }
 
-// Gate/up + SwiGLU on the matrix cores (as k_mb_gate_up): workgroup (chunk, row tile).
-template <int TY, bool SHARED, int S>
+// Tables and token scales of a matrix-core workgroup into LDS.
+template <int TY, int S, class D8>
+__device__ __forceinline__ void mx_prologue(uint8_t *tab, float *s_d8, int n, int nb, D8 d8_of) {
+    mx_fill<TY>(tab);
+    if constexpr (S == 1)
+        for (int k = threadIdx.x; k < 16 * nb; k += MX_THREADS) {
+            const int i = k & 15;
+            s_d8[k] = i < n ? d8_of(i)[k >> 4] : 0.0f;
+        }
+    __syncthreads();
+}
+
+// Gate/up on the matrix cores (as k_mb_gate_up): workgroup (chunk, row tile).
+// TILE: the chunks whose expert has tile copies, else the others.
+template <int TY, bool SHARED, int S, bool TILE>
 __global__ void __launch_bounds__(MX_THREADS) k_mx_gate_up(BatchArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
-    uint8_t *tab = smem;
-    float *terms = reinterpret_cast<float *>(smem + MxTab<TY>::BYTES);
+    __shared__ __align__(16) uint8_t tab[MxTab<TY>::BYTES];
+    __shared__ __align__(16) float s_d8[S == 1 ? MX_MAX_NB * 16 : 4];
     if (a.plan[1]) return;
     const int nb = a.hidden / 256;
-    const int ffn = SHARED ? a.ffn_s : a.ffn_r, rt = 16 * MX_WAVES / S;
+    const int ffn = SHARED ? a.ffn_s : a.ffn_r, rt = S == 1 ? a.mx_rows_gu : 16 * MX_WAVES / S;
     const int tiles = (ffn + rt - 1) / rt;
     const int ci = blockIdx.x / tiles, tile = blockIdx.x - ci * tiles;
     const int r0 = tile * rt, r1 = r0 + rt < ffn ? r0 + rt : ffn;
@@ -1036,18 +1132,18 @@ __global__ void __launch_bounds__(MX_THREADS) k_mx_gate_up(BatchArgs a) {
         const ExpertDev &E = a.experts_mx[a.chunk_expert[ci]];
         mv[0] = E.gate, mv[1] = E.up;
     }
-    if (n < a.mx_min) return;
-    const int c = (int)(threadIdx.x & 15) < n ? (int)(threadIdx.x & 15) : n - 1;
-    const long long tok = SHARED ? (long long)(p0 + c) : (long long)a.pair_token[p0 + c];
+    if (n < a.mx_min || (mv[0].order == MAT_TILE16) != TILE) return;
+    auto token = [&](int i) {
+        i = i < n ? i : n - 1;
+        return SHARED ? (long long)(p0 + i) : (long long)a.pair_token[p0 + i];
+    };
+    auto d8_of = [&](int i) { return a.xd_mx + token(i) * nb; };
     float *g = SHARED ? a.g_s : a.g_r, *u = SHARED ? a.u_s : a.u_r;
-    mx_tiles<TY, 2, S>(
-        mv, r0, r1, nb, a.xq_mx + tok * nb * 256, a.xd_mx + tok * nb, tab, terms,
-        [&]() {
-            mx_fill<TY>(tab);
-            __syncthreads();
-        },
+    mx_tiles<TY, 2, S, TILE, false>(
+        mv, r0, r1, nb, a.xq_mx + token(threadIdx.x & 15) * nb * 256, tab, s_d8, reinterpret_cast<float *>(smem),
+        [&]() { mx_prologue<TY, S>(tab, s_d8, n, nb, d8_of); }, d8_of,
         [&](int i, int r, const float *res) {
-            if (i < n && r < r1) {
+            if (i < n) {
                 const long long o = (long long)(p0 + i) * ffn + r;
                 g[o] = res[0];
                 u[o] = res[1];
@@ -1055,15 +1151,16 @@ __global__ void __launch_bounds__(MX_THREADS) k_mx_gate_up(BatchArgs a) {
         });
 }
 
-// Down on the matrix cores (as k_mb_down).
-template <int TY, bool SHARED, int S>
+// Down on the matrix cores (as k_mb_down); with S = 1 each wave takes two
+// adjacent 16-row tiles a step, which share the token operands.
+template <int TY, bool SHARED, int S, bool TILE>
 __global__ void __launch_bounds__(MX_THREADS) k_mx_down(BatchArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
-    uint8_t *tab = smem;
-    float *terms = reinterpret_cast<float *>(smem + MxTab<TY>::BYTES);
+    __shared__ __align__(16) uint8_t tab[MxTab<TY>::BYTES];
+    __shared__ __align__(16) float s_d8[S == 1 ? MX_MAX_NB * 16 : 4];
     if (a.plan[1]) return;
     const int nb = (SHARED ? a.ffn_s : a.ffn_r) / 256;
-    const int rt = 16 * MX_WAVES / S;
+    const int rt = S == 1 ? a.mx_rows_d : 16 * MX_WAVES / S;
     const int tiles = (a.hidden + rt - 1) / rt;
     const int ci = blockIdx.x / tiles, tile = blockIdx.x - ci * tiles;
     const int r0 = tile * rt, r1 = r0 + rt < a.hidden ? r0 + rt : a.hidden;
@@ -1078,20 +1175,21 @@ __global__ void __launch_bounds__(MX_THREADS) k_mx_down(BatchArgs a) {
         p0 = a.chunk_p0[ci], n = a.chunk_n[ci];
         mv[0] = a.experts_mx[a.chunk_expert[ci]].down;
     }
-    if (n < a.mx_min) return;
+    if (n < a.mx_min || (mv[0].order == MAT_TILE16) != TILE) return;
+    const uint8_t *hq = SHARED ? a.hq_mx_s : a.hq_mx_r;
+    const float *hd = SHARED ? a.hd_mx_s : a.hd_mx_r;
     const int c = (int)(threadIdx.x & 15) < n ? (int)(threadIdx.x & 15) : n - 1;
-    const long long row = p0 + c;
-    const uint8_t *bq = (SHARED ? a.hq_mx_s : a.hq_mx_r) + row * nb * 256;
-    const float *bd = (SHARED ? a.hd_mx_s : a.hd_mx_r) + row * nb;
+    auto d8_of = [&](int i) { return hd + (long long)(p0 + (i < n ? i : n - 1)) * nb; };
     float *d = SHARED ? a.d_s : a.d_r;
-    mx_tiles<TY, 1, S>(
-        mv, r0, r1, nb, bq, bd, tab, terms,
-        [&]() {
-            mx_fill<TY>(tab);
-            __syncthreads();
-        },
+    constexpr int NM = S == 1 ? 2 : 1;
+    mx_tiles<TY, NM, S, TILE, true>(
+        mv, r0, r1, nb, hq + (long long)(p0 + c) * nb * 256, tab, s_d8, reinterpret_cast<float *>(smem),
+        [&]() { mx_prologue<TY, S>(tab, s_d8, n, nb, d8_of); }, d8_of,
         [&](int i, int r, const float *res) {
-            if (i < n && r < r1) d[(long long)(p0 + i) * a.hidden + r] = res[0];
+            if (i < n) {
+#pragma unroll
+                for (int t = 0; t < NM; ++t) d[(long long)(p0 + i) * a.hidden + r + 16 * t] = res[t];
+            }
         });
 }
 
@@ -1178,11 +1276,10 @@ static hipError_t allow_lds(K kernel, int lds) {
     return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
 }
 
-// lds: the stage's LDS footprint; the VALU kernels hold the codebook
-// statically, the rest is dynamic.
+// The VALU kernels hold the codebook statically, the rest is dynamic.
 template <int TY, bool SHARED>
-static hipError_t gate_up_typed(const BatchArgs &a, int lds, hipStream_t s) {
-    lds -= al16(GridLDS<TY>::BYTES);
+static hipError_t gate_up_typed(const BatchArgs &a, hipStream_t s) {
+    const int lds = stream_lds<TY, 2>(valu_cap(a, TY), a.hidden / 256, 2) - al16(GridLDS<TY>::BYTES);
     const int grid = SHARED ? cdiv(a.n_tokens, a.tc) * cdiv(a.ffn_s, a.rt_gu_s) : a.max_chunks * cdiv(a.ffn_r, a.rt_gu_r);
     // Routed IQ chunks left to the VALU beside the matrix cores: one-token
     // chunks in their own launch, then the rest (measured on MI355X at the
@@ -1206,8 +1303,8 @@ static hipError_t gate_up_typed(const BatchArgs &a, int lds, hipStream_t s) {
 }
 
 template <int TY, bool SHARED>
-static hipError_t down_typed(const BatchArgs &a, int lds, hipStream_t s) {
-    lds -= al16(GridLDS<TY>::BYTES);
+static hipError_t down_typed(const BatchArgs &a, hipStream_t s) {
+    const int lds = stream_lds<TY, 1>(valu_cap(a, TY), (SHARED ? a.ffn_s : a.ffn_r) / 256, 2) - al16(GridLDS<TY>::BYTES);
     const int grid = SHARED ? cdiv(a.n_tokens, a.tc) * cdiv(a.hidden, a.rt_d_s) : a.max_chunks * cdiv(a.hidden, a.rt_d_r);
     // Routed IQ downs beside the matrix cores taking every chunk of 2+ tokens:
     // the VALU chunks all hold one token and run the fused rows (measured on
@@ -1228,29 +1325,45 @@ static hipError_t down_typed(const BatchArgs &a, int lds, hipStream_t s) {
     return hipGetLastError();
 }
 
-// An IQ stream with the matrix cores on: the matrix-core launch when some
-// chunk can reach mx_min tokens, then the VALU launch when some chunk can stay
-// below it (each kernel returns early on the other's chunks).
+template <int TY, bool SHARED, int S, bool TILE>
+static hipError_t mx_gate_up_launch(const BatchArgs &a, hipStream_t s) {
+    const int lds = mx_dyn_lds(2, S, a.hidden / 256), rows = S == 1 ? a.mx_rows_gu : 16 * MX_WAVES / S;
+    const hipError_t e = allow_lds(k_mx_gate_up<TY, SHARED, S, TILE>, lds);
+    if (e != hipSuccess) return e;
+    const int grid = (SHARED ? cdiv(a.n_tokens, a.tc) : a.max_chunks) * cdiv(SHARED ? a.ffn_s : a.ffn_r, rows);
+    hipLaunchKernelGGL((k_mx_gate_up<TY, SHARED, S, TILE>), dim3(grid), dim3(MX_THREADS), lds, s, a);
+    return hipGetLastError();
+}
+
+template <int TY, bool SHARED, int S, bool TILE>
+static hipError_t mx_down_launch(const BatchArgs &a, hipStream_t s) {
+    const int nb = (SHARED ? a.ffn_s : a.ffn_r) / 256;
+    const int lds = mx_dyn_lds(1, S, nb), rows = S == 1 ? a.mx_rows_d : 16 * MX_WAVES / S;
+    const hipError_t e = allow_lds(k_mx_down<TY, SHARED, S, TILE>, lds);
+    if (e != hipSuccess) return e;
+    const int grid = (SHARED ? cdiv(a.n_tokens, a.tc) : a.max_chunks) * cdiv(a.hidden, rows);
+    hipLaunchKernelGGL((k_mx_down<TY, SHARED, S, TILE>), dim3(grid), dim3(MX_THREADS), lds, s, a);
+    return hipGetLastError();
+}
+
+// One launch for the experts with tile copies, one for the others (a layer
+// with copies of some experts only needs both).
 template <int TY, bool SHARED, int S>
 static hipError_t mx_gate_up_split(const BatchArgs &a, hipStream_t s) {
-    const int nb = a.hidden / 256;
-    const int lds = mx_lds_bytes(TY, 2, S, nb);
-    hipError_t e = allow_lds(k_mx_gate_up<TY, SHARED, S>, lds);
-    if (e != hipSuccess) return e;
-    const int grid = (SHARED ? cdiv(a.n_tokens, a.tc) : a.max_chunks) * cdiv(SHARED ? a.ffn_s : a.ffn_r, 16 * MX_WAVES / S);
-    hipLaunchKernelGGL((k_mx_gate_up<TY, SHARED, S>), dim3(grid), dim3(MX_THREADS), lds, s, a);
-    return hipGetLastError();
+    hipError_t e = hipSuccess;
+    if (SHARED || a.mx_copies != 2) e = mx_gate_up_launch<TY, SHARED, S, false>(a, s);
+    if constexpr (!SHARED)
+        if (e == hipSuccess && a.mx_copies) e = mx_gate_up_launch<TY, SHARED, S, true>(a, s);
+    return e;
 }
 
 template <int TY, bool SHARED, int S>
 static hipError_t mx_down_split(const BatchArgs &a, hipStream_t s) {
-    const int nb = (SHARED ? a.ffn_s : a.ffn_r) / 256;
-    const int lds = mx_lds_bytes(TY, 1, S, nb);
-    hipError_t e = allow_lds(k_mx_down<TY, SHARED, S>, lds);
-    if (e != hipSuccess) return e;
-    const int grid = (SHARED ? cdiv(a.n_tokens, a.tc) : a.max_chunks) * cdiv(a.hidden, 16 * MX_WAVES / S);
-    hipLaunchKernelGGL((k_mx_down<TY, SHARED, S>), dim3(grid), dim3(MX_THREADS), lds, s, a);
-    return hipGetLastError();
+    hipError_t e = hipSuccess;
+    if (SHARED || a.mx_copies != 2) e = mx_down_launch<TY, SHARED, S, false>(a, s);
+    if constexpr (!SHARED)
+        if (e == hipSuccess && a.mx_copies) e = mx_down_launch<TY, SHARED, S, true>(a, s);
+    return e;
 }
 
 // An IQ stream with the matrix cores on: the matrix-core launch when some
@@ -1258,46 +1371,46 @@ static hipError_t mx_down_split(const BatchArgs &a, hipStream_t s) {
 // below it (each kernel returns early on the other's chunks).  mx_split_* is
 // the number of waves that share a 16-row tile (1, 2 or 4).
 template <int TY, bool SHARED>
-static hipError_t mx_gate_up_typed(const BatchArgs &a, int lds, hipStream_t s_mx, hipStream_t s_valu) {
+static hipError_t mx_gate_up_typed(const BatchArgs &a, hipStream_t s_mx, hipStream_t s_valu) {
     if (a.mx_min <= a.tc) {
         const hipError_t e = a.mx_split_gu == 4   ? mx_gate_up_split<TY, SHARED, 4>(a, s_mx)
                              : a.mx_split_gu == 2 ? mx_gate_up_split<TY, SHARED, 2>(a, s_mx)
                                                   : mx_gate_up_split<TY, SHARED, 1>(a, s_mx);
         if (e != hipSuccess) return e;
     }
-    return a.mx_min > 1 ? gate_up_typed<TY, SHARED>(a, lds, s_valu) : hipSuccess;
+    return a.mx_min > 1 ? gate_up_typed<TY, SHARED>(a, s_valu) : hipSuccess;
 }
 
 template <int TY, bool SHARED>
-static hipError_t mx_down_typed(const BatchArgs &a, int lds, hipStream_t s_mx, hipStream_t s_valu) {
+static hipError_t mx_down_typed(const BatchArgs &a, hipStream_t s_mx, hipStream_t s_valu) {
     if (a.mx_min <= a.tc) {
         const hipError_t e = a.mx_split_d == 4   ? mx_down_split<TY, SHARED, 4>(a, s_mx)
                              : a.mx_split_d == 2 ? mx_down_split<TY, SHARED, 2>(a, s_mx)
                                                  : mx_down_split<TY, SHARED, 1>(a, s_mx);
         if (e != hipSuccess) return e;
     }
-    return a.mx_min > 1 ? down_typed<TY, SHARED>(a, lds, s_valu) : hipSuccess;
+    return a.mx_min > 1 ? down_typed<TY, SHARED>(a, s_valu) : hipSuccess;
 }
 
 // The matrix-core part of an IQ stream goes to s_mx, its VALU part to s_valu.
 template <bool SHARED>
-static hipError_t gate_up_any(int ty, const BatchArgs &a, int lds, hipStream_t s_mx, hipStream_t s_valu) {
+static hipError_t gate_up_any(int ty, const BatchArgs &a, hipStream_t s_mx, hipStream_t s_valu) {
     const hipStream_t s = s_valu;
     switch (ty) {
     case T_IQ2_S:
-        return a.mx ? mx_gate_up_typed<T_IQ2_S, SHARED>(a, lds, s_mx, s_valu) : gate_up_typed<T_IQ2_S, SHARED>(a, lds, s);
-    case T_Q4_K: return gate_up_typed<T_Q4_K, SHARED>(a, lds, s);
+        return a.mx ? mx_gate_up_typed<T_IQ2_S, SHARED>(a, s_mx, s_valu) : gate_up_typed<T_IQ2_S, SHARED>(a, s);
+    case T_Q4_K: return gate_up_typed<T_Q4_K, SHARED>(a, s);
     default: return hipErrorInvalidValue;
     }
 }
 
 template <bool SHARED>
-static hipError_t down_any(int ty, const BatchArgs &a, int lds, hipStream_t s_mx, hipStream_t s_valu) {
+static hipError_t down_any(int ty, const BatchArgs &a, hipStream_t s_mx, hipStream_t s_valu) {
     const hipStream_t s = s_valu;
     switch (ty) {
-    case T_IQ2_S: return a.mx ? mx_down_typed<T_IQ2_S, SHARED>(a, lds, s_mx, s_valu) : down_typed<T_IQ2_S, SHARED>(a, lds, s);
-    case T_IQ3_S: return a.mx ? mx_down_typed<T_IQ3_S, SHARED>(a, lds, s_mx, s_valu) : down_typed<T_IQ3_S, SHARED>(a, lds, s);
-    case T_Q5_K: return down_typed<T_Q5_K, SHARED>(a, lds, s);
+    case T_IQ2_S: return a.mx ? mx_down_typed<T_IQ2_S, SHARED>(a, s_mx, s_valu) : down_typed<T_IQ2_S, SHARED>(a, s);
+    case T_IQ3_S: return a.mx ? mx_down_typed<T_IQ3_S, SHARED>(a, s_mx, s_valu) : down_typed<T_IQ3_S, SHARED>(a, s);
+    case T_Q5_K: return down_typed<T_Q5_K, SHARED>(a, s);
     default: return hipErrorInvalidValue;
     }
 }
@@ -1352,10 +1465,10 @@ hipError_t launch_moe_batch(const BatchArgs &a, hipStream_t s, const BatchStream
         gm.mat[1] = a.su;
         if ((e = launch_prep_b(a.q8x, a.n_tokens, nbh, a.bx, s2)) != hipSuccess) return e;
         if ((e = launch_kq_gemm(gm, s2)) != hipSuccess) return e;
-    } else if (a.has_shared && (e = gate_up_any<true>(tsg, a, lds[2], s2, s2)) != hipSuccess) {
+    } else if (a.has_shared && (e = gate_up_any<true>(tsg, a, s2, s2)) != hipSuccess) {
         return e;
     }
-    if ((e = gate_up_any<false>(a.type_gate_r, a, lds[1], s2, s)) != hipSuccess) return e;
+    if ((e = gate_up_any<false>(a.type_gate_r, a, s2, s)) != hipSuccess) return e;
     if ((e = join(0)) != hipSuccess) return e;
 
     const bool rm = tsd == T_Q4_K || tsd == T_Q5_K;
@@ -1377,10 +1490,10 @@ hipError_t launch_moe_batch(const BatchArgs &a, hipStream_t s, const BatchStream
         gm.mat[0] = a.sd;
         if ((e = launch_prep_b(a.q8h_s, a.n_tokens, nbs, a.bh, s2)) != hipSuccess) return e;
         if ((e = launch_kq_gemm(gm, s2)) != hipSuccess) return e;
-    } else if (a.has_shared && (e = down_any<true>(tsd, a, lds[4], s2, s2)) != hipSuccess) {
+    } else if (a.has_shared && (e = down_any<true>(tsd, a, s2, s2)) != hipSuccess) {
         return e;
     }
-    if ((e = down_any<false>(a.type_down_r, a, lds[3], s2, s)) != hipSuccess) return e;
+    if ((e = down_any<false>(a.type_down_r, a, s2, s)) != hipSuccess) return e;
     if ((e = join(1)) != hipSuccess) return e;
 
     const long long total = (long long)a.n_tokens * a.hidden;

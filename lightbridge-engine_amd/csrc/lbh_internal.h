@@ -19,12 +19,6 @@ struct DevStatus {
 
 enum : int32_t { MAT_ROW_MAJOR = 0, MAT_TILE16 = 1 };
 
-// Unit of (row r, block b) of a matrix with nb blocks per row stored in unit
-// order `order` (MAT_TILE16 needs rows % 16 == 0).
-__host__ __device__ inline uint32_t unit_index(int32_t order, uint32_t r, uint32_t b, uint32_t nb) {
-    return order == MAT_TILE16 ? (((r >> 4) * nb + b) << 4) + (r & 15u) : r * nb + b;
-}
-
 // A matrix in the device layout (lbh_layout.h).
 struct MatView {
     const uint8_t *planes;
@@ -33,7 +27,8 @@ struct MatView {
     int32_t rows;
     // Unit order of the planes: MAT_ROW_MAJOR (u = r * nb + b) everywhere
     // except the batched matrix-core streams' tile copies, MAT_TILE16
-    // (u = ((r / 16) * nb + b) * 16 + r % 16: the 16 rows of a block adjacent).
+    // (u = ((r / 16) * nb + b) * 16 + r % 16: the 16 rows of a block adjacent,
+    // and their chunk bytes in lane order, k_units_to_tiles).
     int32_t order;
     long long units;   // rows * nb
     long long bytes;   // size of the planes allocation
@@ -218,11 +213,14 @@ struct BatchArgs {
     float *g_s, *u_s;           // [n_tokens][ffn_s]
     uint8_t *bx, *bh;           // GEMM activation tiles of x and of the shared h
     // mx = 1: chunks of at least mx_min tokens of the IQ2_S / IQ3_S streams run
-    // on the f16 matrix cores (mx_split_* waves share each 16-row tile) and read the
-    // operand copies of the Q8_K rows (quants XOR 0x80 at 256 bytes a block,
-    // scales apart) of x and of the routed and shared h; the VALU streams take the smaller chunks
-    // and stage vc = min(tc, mx_min - 1) tokens (tc when mx = 0).
+    // on the int8 matrix cores (mx_split_* waves share each 16-row tile; split 1:
+    // mx_rows_* rows per workgroup) and read the operand copies of the Q8_K rows
+    // (quants at 256 bytes a block, scales apart) of x and of the routed and
+    // shared h; the VALU streams take the smaller chunks and stage vc = min(tc,
+    // mx_min - 1) tokens (tc when mx = 0).  mx_copies: tile copies of no routed
+    // expert (0), some (1) or all (2).
     int32_t mx, mx_min, mx_split_gu, mx_split_d, vc;
+    int32_t mx_rows_gu, mx_rows_d, mx_copies;
     int32_t residual;           // y[t][r] += delta (as MoeArgs::residual)
     // The matrix-core streams' routed views [n_experts]: an expert's 16-row
     // tile copies where lbh_moe_make_batch_tile_copies made them, else its
@@ -296,8 +294,8 @@ hipError_t launch_repack(int ty, const uint8_t *ggml, uint8_t *planes, long long
                          hipStream_t s);
 hipError_t launch_repack_range(int ty, const uint8_t *src, uint8_t *dst, long long U, long long u0, long long n,
                                hipStream_t s);
-// Copy of an IQ2_S / IQ3_S matrix (rows % 16 == 0) with its units in
-// MAT_TILE16 order at dst (m.bytes bytes).
+// Copy of an IQ2_S / IQ3_S matrix (rows % 16 == 0) in MAT_TILE16 order at dst
+// (m.bytes bytes).
 hipError_t launch_units_to_tiles(const MatView &m, uint8_t *dst, hipStream_t s);
 hipError_t launch_validate_scales(int ty, const uint8_t *ggml, long long units,
                                   unsigned long long *first, hipStream_t s);

@@ -179,3 +179,37 @@ def test_tile_copies_async_device_routed_and_residual(be, oracle, small):
             assert _same(got_h[t], w), f"token {t}"
     finally:
         small.moe.make_batch_tile_copies([])
+
+
+@pytest.mark.parametrize("hidden,ffn,down", [(256, 768, IQ3_S), (768, 256, IQ3_S), (1280, 256, IQ2_S), (512, 1280, IQ3_S)])
+@pytest.mark.parametrize("copied", [None, [0, 2], "all"])
+def test_int8_streams_at_the_edges(be, oracle, hidden, ffn, down, copied):
+    """The int8 matrix-core streams at block counts below, at and off the wave
+    split (1, 2, 3, 5 blocks a row), chunks of 1, 2 or 3, 15 and 16 tokens, weights
+    whose codes, signs and scales are all 0, all ones or random, and inputs
+    that quantize to +-127: the largest integer sums, over the matrices as
+    uploaded, with copies of some experts and of all, at every wave split."""
+    def edge(e, *mats):
+        for m in mats:
+            b = m.reshape(-1, 110 if m is mats[2] and down == IQ3_S else 82)
+            b[e % 3::3, 2:], b[(e + 1) % 3::3, 2:] = 0xff, 0
+
+    shared = (Q4_K, Q5_K) if down == IQ3_S else (IQ2_S, IQ2_S)
+    layer = Layer(be, oracle, 4, hidden, ffn, 256, (IQ2_S, down, *shared), seed=181, scale=edge)
+    moe, rng = layer.moe, np.random.default_rng(hidden + ffn)
+    n = 17
+    moe.reserve_batch(n, 3)
+    if copied:
+        moe.make_batch_tile_copies(None if copied == "all" else copied)
+    ids = np.array([[0, 1, 2]] * 15 + [[0, 1, 2], [0, 2, 3]], np.uint32)   # 17, 16, 17 and 1 tokens
+    ids[0] = [0, 1, 3]                                                     # ... 2: 16, 3: 2
+    ids[1] = [0, 1, 3] if hidden == 256 else ids[1]                        # ... 2: 15, 3: 3
+    coefs = rng.random((n, 3)).astype(np.float32)
+    xs = np.sign(rng.standard_normal((n, hidden))).astype(np.float32)
+    xs[1::2] *= rng.random((8, hidden)).astype(np.float32)
+    want = oracle_batch(oracle, layer, ids, coefs, xs)
+    for engine in ((1, 64, 64), (1, 32, 32), (1, 16, 16), (2, 64, 16)):
+        moe.set_batch_engine(*engine)
+        got = run_checked(be, layer, ids, coefs, xs)
+        bad = [t for t in range(n) if not _same(got[t], want[t])]
+        assert not bad, f"engine {engine}: tokens {bad}"
