@@ -393,13 +393,12 @@ lbh_status lbh_moe_set_batch_tiles(lbh_moe *moe, int32_t tokens_per_chunk, int32
 
 /* Engine of the batched IQ2_S / IQ3_S streams (no counterpart in the reference,
  * whose batch is a loop over tokens).  Chunks of at least mx_min_tokens tokens
- * (1..16; default 4) run on the int8 matrix cores, one 16-row x 16-token product
- * per block, with mx_rows_gate_up / mx_rows_down rows per workgroup
- * (16, 32 or 64; 0: the defaults 16 and 32); smaller chunks run on the VALU
- * integer dots; mx_min_tokens = 0
- * keeps every chunk on the VALU.  Every choice gives the same bits.  Resets the
- * tokens per chunk (16 with the matrix cores, 8 without) and the VALU row tiles
- * to their defaults. */
+ * (1..16; 1 until this is called) run on the int8 matrix cores, one 16-row x
+ * 16-token product per block, with mx_rows_gate_up / mx_rows_down rows per
+ * workgroup (16, 32 or 64; 0: the defaults 64 and 256); smaller chunks run on
+ * the VALU integer dots; mx_min_tokens = 0 keeps every chunk on the VALU.
+ * Every choice gives the same bits.  Resets the tokens per chunk (16 with the
+ * matrix cores, 8 without) and the VALU row tiles to their defaults. */
 lbh_status lbh_moe_set_batch_engine(lbh_moe *moe, int32_t mx_min_tokens, int32_t mx_rows_gate_up,
                                     int32_t mx_rows_down);
 
@@ -420,11 +419,8 @@ lbh_status lbh_moe_set_batch_engine(lbh_moe *moe, int32_t mx_min_tokens, int32_t
  *   before it hold the released copies' addresses: capture them again. The
  *   same holds after lbh_moe_reserve_batch.
  * The copies are taken at this call: call it again after an expert's bytes
- * change.  Until lbh_moe_set_batch_engine is called, the layer's engine follows
- * the copies.  With copies, chunks of 2+ tokens run on the matrix cores, one wave
- * per 16-row tile.  Without, chunks of 4+ tokens run on the split tiles.  Each
- * measured fastest in its case.  Layers over an expert cache have no static
- * expert table and return LBH_INVALID_PARAMETER. */
+ * change.  Layers over an expert cache have no static expert table and return
+ * LBH_INVALID_PARAMETER. */
 lbh_status lbh_moe_make_batch_tile_copies(lbh_ctx *ctx, lbh_moe *moe, const uint32_t *experts, size_t n_experts,
                                           lbh_error *err);
 

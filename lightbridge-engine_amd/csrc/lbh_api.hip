@@ -853,13 +853,12 @@ struct lbh_moe {
     int32_t *plan_host;       // pinned
     int tc, rt_gu_r, rt_gu_s, rt_d_r, rt_d_s;
     int mx_min;               // batched IQ chunks of >= mx_min tokens on the matrix cores (0: none)
-    int mx_split_gu, mx_split_d;   // waves sharing a 16-row tile of those streams (1, 2, 4)
-    int mx_rows_gu, mx_rows_d;     // rows per workgroup at one wave per tile
+    int mx_rows_gu, mx_rows_d;     // rows per workgroup of those streams
     int tile_copies;               // routed experts with tile copies: 0 none, 1 some, 2 all
     hipStream_t side;         // batched calls: second stream and fork/join events
     hipEvent_t ev[4];
-    uint8_t *shared_gemm_mem; // MFMA-ready copies of a K-quant shared expert (batched calls)
-    size_t gemm_off[3];       // A offsets of gate, up, down in shared_gemm_mem
+    uint8_t *shared_kt_mem;   // tile copies of a K-quant shared expert (batched calls)
+    size_t kt_off[3];         // offsets of gate, up, down in shared_kt_mem
     // Single-token decode with a shared expert: its gate/up and down run on
     // side1 beside the routed experts (fork / join events); d_shared holds its
     // raw down rows for the routed launch's combine.
@@ -874,34 +873,22 @@ struct lbh_moe {
     uint8_t *tile_mem;
     size_t tile_bytes;
     ExpertDev *experts_mx_dev;
-    int engine_set;           // lbh_moe_set_batch_engine was called: the copies leave the engine alone
 };
 
 namespace {
 
-// Batched launch shapes measured on MI355X at the configs[3] shapes (64 tokens,
-// hidden 4096, routed ffn 1536): with the matrix cores on, chunks of 16 tokens
-// (one instruction's width); the VALU streams alone do best with chunks of 8.
-constexpr int MX_MIN_DEFAULT = 4;
+// Batched launch shapes (measured on MI355X, 192 experts of hidden 4096, width
+// 1536, top-8): with the matrix cores on, chunks of 16 tokens (one instruction's
+// width), from one token up, 64 gate/up rows (a 16-row tile per wave) and 256
+// down rows per workgroup (1, 5, 16, 64 and 256 tokens; 128 and 256 gate/up rows
+// 3-25% slower, 128 and 512 down rows 0-4%).  The VALU streams alone do best with
+// chunks of 8.
+constexpr int MX_MIN_DEFAULT = 1;
 void set_batch_defaults(lbh_moe *m, int mx_min) {
     m->mx_min = mx_min;
-    m->mx_split_gu = 4, m->mx_split_d = 2;
     m->mx_rows_gu = 64, m->mx_rows_d = 256;
     m->tc = mx_min > 0 ? 16 : 8;
     m->rt_gu_r = 64, m->rt_gu_s = 64, m->rt_d_r = 160, m->rt_d_s = 64;
-}
-// With the tile copies (lbh_moe_make_batch_tile_copies) a step's 16 rows of a
-// block are two whole lines, so one wave per 16-row tile and chunks from two
-// tokens on the matrix cores measured fastest, the VALU keeping the one-token
-// chunks (configs[3]: 360-362 us; 369-371 from three tokens, 379 from four;
-// without copies the split tiles and 4-token chunks stay the defaults: 430 us
-// there against 477-555 us for these settings).
-constexpr int MX_MIN_TILED = 2;
-void set_engine_for_copies(lbh_moe *m, bool copies) {
-    if (m->engine_set) return;
-    m->mx_min = copies ? MX_MIN_TILED : MX_MIN_DEFAULT;
-    m->mx_split_gu = copies ? 1 : 4;
-    m->mx_split_d = copies ? 1 : 2;
 }
 
 void free_moe(lbh_moe *m) {
@@ -910,7 +897,7 @@ void free_moe(lbh_moe *m) {
     if (m->experts_dev) (void)hipFree(m->experts_dev);
     delete[] m->experts_host;
     if (m->batch_mem) (void)hipFree(m->batch_mem);
-    if (m->shared_gemm_mem) (void)hipFree(m->shared_gemm_mem);
+    if (m->shared_kt_mem) (void)hipFree(m->shared_kt_mem);
     if (m->tile_mem) (void)hipFree(m->tile_mem);
     if (m->experts_mx_dev) (void)hipFree(m->experts_mx_dev);
     if (m->plan_host) (void)hipHostFree(m->plan_host);
@@ -1580,13 +1567,12 @@ BatchArgs batch_args(const lbh_moe *m, const uint32_t *ids, const float *coefs, 
     a.type_down_r = m->type_down_r;
     a.mx = m->mx_min > 0 ? 1 : 0;
     a.mx_min = m->mx_min > 0 ? m->mx_min : BATCH_MAX_TC + 1;
-    a.mx_split_gu = m->mx_split_gu;
-    a.mx_split_d = m->mx_split_d;
     a.mx_rows_gu = m->mx_rows_gu;
-    a.mx_rows_d = m->mx_rows_d;
+    a.mx_rows_d = (m->mx_rows_d + 31) / 32 * 32;   // the down streams take 32 rows a wave over tile copies
     a.mx_copies = m->tile_copies;
     a.vc = a.mx ? (a.tc < a.mx_min - 1 ? a.tc : a.mx_min - 1) : a.tc;
     if (a.vc < 1) a.vc = 1;
+    a.valu = !a.mx || a.mx_min > 1;
     return a;
 }
 
@@ -1639,13 +1625,13 @@ lbh_status lbh_moe_reserve_batch(lbh_moe *m, size_t max_tokens, size_t top_k, lb
     const size_t o_xqm = take(T * nbh * 256), o_xdm = take(T * nbh * 4);
     const size_t o_hqr = take(P * nbr * 256), o_hdr = take(P * nbr * 4);
     const size_t o_hqs = take(T * nbs * 256), o_hds = take(T * nbs * 4);
-    // A K-quant shared expert runs on the matrix cores: gate/up outputs and the
-    // GEMM activation tiles of x and of the shared h.
-    const bool sgemm = m->has_shared && is_kquant(m->shared.gate.type) && is_kquant(m->shared.down.type);
-    size_t o_bx = 0, o_bh = 0;
-    if (sgemm) {
-        o_bx = take(gemm_b_bytes((int)T, (int)nbh));
-        o_bh = take(gemm_b_bytes((int)T, (int)nbs));
+    // A K-quant shared expert runs on the matrix cores: operand tiles of x and
+    // of the shared h.
+    const bool kt = m->has_shared && m->shared.gate.type == LBH_Q4_K && m->shared.down.type == LBH_Q5_K;
+    size_t o_ktx = 0, o_kth = 0;
+    if (kt) {
+        o_ktx = take(kt_token_bytes((int)T, (int)nbh));
+        o_kth = take(kt_token_bytes((int)T, (int)nbs));
     }
     hipError_t e = hipMalloc(&m->batch_mem, off);
     if (e == hipSuccess) e = hipMemset(m->batch_mem, 0, off);
@@ -1688,36 +1674,31 @@ lbh_status lbh_moe_reserve_batch(lbh_moe *m, size_t max_tokens, size_t top_k, lb
     a.hd_mx_s = reinterpret_cast<float *>(b + o_hds);
     m->batch_ids = reinterpret_cast<uint32_t *>(b + o_ids);
     m->batch_coefs = reinterpret_cast<float *>(b + o_coefs);
-    a.shared_gemm = sgemm ? 1 : 0;
-    if (sgemm) {
-        a.bx = b + o_bx;
-        a.bh = b + o_bh;
-        if (!m->shared_gemm_mem) {
-            // MFMA-ready copies of the shared gate, up and down (built once).
-            const MatView v[3] = {m->shared.gate, m->shared.up, m->shared.down};
-            size_t so = 0, oa[3];
+    a.shared_kt = kt ? 1 : 0;
+    if (kt) {
+        a.kt_x = b + o_ktx;
+        a.kt_h = b + o_kth;
+        const MatView v[3] = {m->shared.gate, m->shared.up, m->shared.down};
+        if (!m->shared_kt_mem) {
+            // Tile copies of the shared gate, up and down (built once).
+            size_t so = 0;
             for (int i = 0; i < 3; ++i) {
-                oa[i] = so;
-                so += (gemm_a_bytes(v[i].rows, v[i].nb) + 255) & ~(size_t)255;
+                m->kt_off[i] = so;
+                so += (kt_weight_bytes(v[i].type, v[i].rows, v[i].nb) + 255) & ~(size_t)255;
             }
-            e = hipMalloc(&m->shared_gemm_mem, so);
-            for (int i = 0; i < 3 && e == hipSuccess; ++i) e = launch_prep_a(v[i], m->shared_gemm_mem + oa[i], nullptr);
+            e = hipMalloc(&m->shared_kt_mem, so);
+            for (int i = 0; i < 3 && e == hipSuccess; ++i) e = launch_kt_pack(v[i], m->shared_kt_mem + m->kt_off[i], nullptr);
             if (e == hipSuccess) e = hipDeviceSynchronize();
             if (e != hipSuccess) {
-                if (m->shared_gemm_mem) (void)hipFree(m->shared_gemm_mem);
-                m->shared_gemm_mem = nullptr;
+                if (m->shared_kt_mem) (void)hipFree(m->shared_kt_mem);
+                m->shared_kt_mem = nullptr;
                 (void)hipFree(m->batch_mem);
                 m->batch_mem = nullptr;
                 m->cap_tokens = m->cap_k = 0;
                 return hip_fail(err, e);
             }
-            m->gemm_off[0] = oa[0], m->gemm_off[1] = oa[1], m->gemm_off[2] = oa[2];
         }
-        uint8_t *g = m->shared_gemm_mem;
-        const int ffs = (int)ffn_s, hid = (int)m->hidden;
-        a.sg = MatGemm{g + m->gemm_off[0], a.g_s, ffs, ffs};
-        a.su = MatGemm{g + m->gemm_off[1], a.u_s, ffs, ffs};
-        a.sd = MatGemm{g + m->gemm_off[2], a.d_s, hid, hid};
+        for (int i = 0; i < 3; ++i) a.kt_w[i] = m->shared_kt_mem + m->kt_off[i];
     }
     m->cap_tokens = max_tokens;
     m->cap_k = top_k;
@@ -1750,15 +1731,14 @@ lbh_status lbh_moe_set_batch_engine(lbh_moe *m, int32_t mx_min_tokens, int32_t m
         return LBH_INVALID_PARAMETER;
     const lbh_moe saved = *m;
     set_batch_defaults(m, mx_min_tokens);
-    if (mx_rows_gate_up) m->mx_split_gu = 64 / mx_rows_gate_up;
-    if (mx_rows_down) m->mx_split_d = 64 / mx_rows_down;
+    if (mx_rows_gate_up) m->mx_rows_gu = mx_rows_gate_up;
+    if (mx_rows_down) m->mx_rows_d = mx_rows_down;
     const BatchArgs probe = batch_args(m, nullptr, nullptr, 1, 1, nullptr, nullptr);
     for (int st = 0; st < 5; ++st)
         if (batch_lds_bytes(probe, st) > 160 * 1024) {
             *m = saved;
             return LBH_UNSUPPORTED_SHAPE;
         }
-    m->engine_set = 1;
     return LBH_OK;
 }
 
@@ -1826,7 +1806,6 @@ lbh_status lbh_moe_make_batch_tile_copies(lbh_ctx *ctx, lbh_moe *m, const uint32
     size_t picked = 0;
     for (size_t e = 0; e < m->n_experts; ++e) picked += pick[e] ? 1 : 0;
     m->tile_copies = !table ? 0 : picked < m->n_experts ? 1 : 2;
-    set_engine_for_copies(m, table != nullptr);
     return ok(err);
 }
 
@@ -1840,7 +1819,6 @@ static lbh_status forward_batch(lbh_ctx *ctx, lbh_moe *m, const uint32_t *ids, c
     DeviceGuard g(ctx->device);
     BatchArgs a = batch_args(m, ids, coefs, n_tokens, top_k, x, y);
     a.residual = residual;
-    a.gemm_shape = ctx->gemm_shape;
     const BatchStreams bs = batch_streams(m);
     if (launch_moe_batch(a, ctx->stream, &bs) != hipSuccess) return LBH_HIP_ERROR;
     return LBH_OK;
@@ -1895,7 +1873,6 @@ lbh_status lbh_moe_routed_by_id_batch_into(lbh_ctx *ctx, lbh_moe *m, const uint3
     HIP_TRY(hipMemcpyAsync(m->batch_ids, ids, n_tokens * top_k * 4, hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(hipMemcpyAsync(m->batch_coefs, coefs, n_tokens * top_k * 4, hipMemcpyHostToDevice, ctx->stream));
     BatchArgs a = batch_args(m, m->batch_ids, m->batch_coefs, n_tokens, top_k, input, output);
-    a.gemm_shape = ctx->gemm_shape;
     const BatchStreams bs = batch_streams(m);
     HIP_TRY(launch_moe_batch(a, ctx->stream, &bs));
     HIP_TRY(hipMemcpyAsync(m->plan_host, a.plan, 8, hipMemcpyDeviceToHost, ctx->stream));

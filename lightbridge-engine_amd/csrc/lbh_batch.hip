@@ -8,23 +8,32 @@
 // are decoded once into registers for all of them:
 //
 //   k_mb_prep     counting sort of the pairs by expert (ascending token order
-//                 inside an expert) into a chunk table; Q8_K of every token;
-//   k_mb_gate_up  per (chunk, row tile): the chunk's Q8_K activations staged
-//                 in LDS, gate and up rows decoded once, integer dots against
-//                 every staged token, per-(row, token) folds in the
-//                 reference's block order, SwiGLU -> h;
-//   k_mb_quant_h  Q8_K of every h row (the down projections' inputs,
-//                 gemv.rs:161-163);
-//   k_mb_down     per (chunk, row tile): the down rows against every staged h;
+//                 inside an expert) into a chunk table; Q8_K of every token and
+//                 its matrix-core operands;
+//   k_mx_gate_up  per (chunk, row tile) on the int8 matrix cores: gate and up
+//                 rows against the chunk's tokens, folded in the reference's
+//                 block order; the same launch holds the shared expert's
+//                 K-quant gate and up (lbh_kt.h);
+//   k_mb_quant_h  SwiGLU and the Q8_K operands of every h row (the down
+//                 projections' inputs, gemv.rs:161-163);
+//   k_mx_down     per (chunk, row tile): the down rows against the chunk's h,
+//                 and the shared expert's down;
 //   k_mb_combine  per token and output row, in the reference's order:
 //                 y = ((0 + c_0 d_0) + c_1 d_1) + ... + 1.0 * d_shared.
 //
-// The shared expert is one more "expert" that every token selects.
+// k_mb_gate_up / k_mb_down are the same streams on the VALU integer dots, for
+// the chunks below a caller's matrix-core threshold
+// (lbh_moe_set_batch_engine).  By default every chunk runs on the matrix cores,
+// also those of one token: a 16-token tile decodes its weights at the VALU cost
+// of a one-token dot (measured, 192 experts of hidden 4096, width 1536, top-8:
+// 64 tokens with tile copies 255 us per step, 295 with the one-token chunks on
+// the VALU beside; 5 tokens without copies 112 and 143 us).
 //
 // Several workgroups read the same expert rows (one per chunk of its tokens),
 // so the weight loads keep the default cache policy here.
 #define LBH_WEIGHT_CPOL 0
 #include "lbh_internal.h"
+#include "lbh_kt.h"
 #include "lbh_math.h"
 #include "lbh_router.h"
 #include "lbh_rows.h"
@@ -39,9 +48,10 @@ constexpr int MB_WAVES = MB_THREADS / 64;
 constexpr int Q8L = 304;
 
 // Matrix-core operand copy of Q8_K rows, written beside the GGML bytes by the
-// quantize kernels: block k's 256 quants at q + 256 k, its scale at d[k].
-// split: in the order of the IQ3_S instructions (dword 2g + h of lane quarter
-// p holds elements 32g + 8p + 4h .. + 3), else in element order (IQ2_S).
+// quantize kernels: block k's 256 quants at q + 256 k, its scale at d[k].  Dword
+// 16 m + 4 p + i is dword 4 m + i of lane quarter p, so that the four lanes of a
+// token read 64 contiguous bytes at a time: elements 64 p + 16 m + 4 i .. + 3 for
+// IQ2_S, for IQ3_S (split) elements 32 g + 8 p + 4 h .. + 3 with 2 g + h = 4 m + i.
 struct MxRows {
     uint8_t *q;
     float *d;
@@ -414,10 +424,12 @@ constexpr int mb_lpu() {
 // Sort of the batch's pairs by expert (workgroup 0) and Q8_K of every token
 // (the other workgroups, four blocks per wave).
 __device__ __forceinline__ void quantize_rows_out(const float *x, long long nblocks, long long first, uint8_t *plain,
-                                                  uint8_t *rm, uint8_t *lds_wave, MxRows mx = MxRows{}) {
-    // Blocks [first, first + 4) (x points at block `first`) into the wave's
-    // LDS, then out to global memory: the GGML bytes, (rm != NULL) the copy
-    // with residue-major qs, and (mx.q != NULL) the matrix-core operand copy.
+                                                  uint8_t *rm, uint8_t *lds_wave, MxRows mx, uint8_t *kt, int nb) {
+    // Blocks [first, first + 4) (x points at block `first`) of rows of nb
+    // blocks into the wave's LDS, then out to global memory: (plain != NULL)
+    // the GGML bytes, (rm != NULL) the copy with residue-major qs, (mx.q !=
+    // NULL) the matrix-core operand copy, (kt != NULL) the f16 operand tiles of
+    // the K-quant rows (lbh_kt.h).
     const int lane = threadIdx.x & 63;
     const long long cnt = nblocks - first < 4 ? nblocks - first : 4;
     quantize_blocks_wave(x, lds_wave, 0, cnt);
@@ -426,11 +438,23 @@ __device__ __forceinline__ void quantize_rows_out(const float *x, long long nblo
         for (int k = lane; k < (int)cnt * 64; k += 64) {
             const int blk = k >> 6, w = k & 63;
             // w: destination dword, from source dword sw
-            const int sw = mx.split ? 8 * ((w >> 1) & 7) + 2 * (w >> 4) + (w & 1) : w;
+            const int p = (w >> 2) & 3, o = 4 * (w >> 4) + (w & 3);   // quarter p, its dword o
+            const int sw = mx.split ? 8 * (o >> 1) + 2 * p + (o & 1) : 16 * p + o;
             reinterpret_cast<uint32_t *>(mx.q)[(first + blk) * 64 + w] =
                 *reinterpret_cast<const uint32_t *>(lds_wave + blk * 292 + 4 + 4 * sw);
         }
         if (lane < cnt) mx.d[first + lane] = *reinterpret_cast<const float *>(lds_wave + lane * 292);
+    }
+    if (kt) {
+        for (int k = lane; k < (int)cnt * KT_STORE_PIECES; k += 64) {
+            const int blk = k / KT_STORE_PIECES;
+            const long long g = first + blk, t = g / nb;
+            kt_store_piece(kt, t, (int)(g - t * nb), nb, lds_wave + blk * 292, k - blk * KT_STORE_PIECES);
+        }
+    }
+    if (!plain && !rm) {
+        wave_sync();
+        return;
     }
     const int dw = (int)cnt * 73;
     for (int k = lane; k < dw; k += 64) {
@@ -458,10 +482,11 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_prep(BatchArgs a) {
         const int nb = a.hidden / 256;
         const long long nblocks = (long long)a.n_tokens * nb;
         const long long first = ((long long)(blockIdx.x - 1) * MB_WAVES + (tid >> 6)) * 4;
-        const bool rm = a.has_shared && !a.shared_gemm && (a.shared.gate.type == T_Q4_K || a.shared.gate.type == T_Q5_K);
+        const bool rm = a.has_shared && !a.shared_kt && (a.shared.gate.type == T_Q4_K || a.shared.gate.type == T_Q5_K);
         if (first < nblocks)
-            quantize_rows_out(a.x + first * 256, nblocks, first, a.q8x, rm ? a.q8x_rm : nullptr,
-                              smem + (tid >> 6) * 4 * 292, MxRows{a.mx ? a.xq_mx : nullptr, a.xd_mx, false});
+            quantize_rows_out(a.x + first * 256, nblocks, first, a.valu ? a.q8x : nullptr, rm ? a.q8x_rm : nullptr,
+                              smem + (tid >> 6) * 4 * 292, MxRows{a.mx ? a.xq_mx : nullptr, a.xd_mx, false},
+                              a.shared_kt ? a.kt_x : nullptr, nb);
         return;
     }
     const int NE = a.n_experts, T = a.n_tokens, K = a.top_k, TC = a.tc;
@@ -625,7 +650,7 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_gate_up(BatchArgs a) {
 // apart, so no exp runs inside their weight loops (its table load would wait
 // for every weight load in flight).  shared_mode 0: the shared copy is GGML
 // bytes plus the matrix-core operand copy (IQ down); 1: residue-major qs only
-// (VALU K-quant down); 2: GGML bytes (K-quant GEMM down).
+// (VALU K-quant down); 2: the f16 operand tiles (matrix-core K-quant down).
 __global__ void __launch_bounds__(MB_THREADS) k_mb_quant_h(BatchArgs a, int shared_mode) {
     __shared__ __align__(16) uint8_t lds[MB_WAVES * 4 * 292];
     __shared__ __align__(16) float hbuf[MB_WAVES][4 * 256];
@@ -651,12 +676,14 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_quant_h(BatchArgs a, int shar
     };
     if (chunk < br) {
         swiglu_blocks(a.g_r, a.u_r, chunk, br);
-        quantize_rows_out(&hbuf[wid][0], br, chunk, a.q8h_r, nullptr, lw, MxRows{a.mx ? a.hq_mx_r : nullptr, a.hd_mx_r, a.type_down_r == T_IQ3_S});
+        quantize_rows_out(&hbuf[wid][0], br, chunk, a.valu ? a.q8h_r : nullptr, nullptr, lw,
+                          MxRows{a.mx ? a.hq_mx_r : nullptr, a.hd_mx_r, a.type_down_r == T_IQ3_S}, nullptr, nbr);
     } else if (chunk >= brp && chunk - brp < bs) {
         const long long f = chunk - brp;
         swiglu_blocks(a.g_s, a.u_s, f, bs);
-        quantize_rows_out(&hbuf[wid][0], bs, f, shared_mode == 1 ? nullptr : a.q8h_s, shared_mode == 1 ? a.q8h_s : nullptr,
-                          lw, MxRows{a.mx && shared_mode == 0 ? a.hq_mx_s : nullptr, a.hd_mx_s, a.shared.down.type == T_IQ3_S});
+        quantize_rows_out(&hbuf[wid][0], bs, f, shared_mode == 0 ? a.q8h_s : nullptr, shared_mode == 1 ? a.q8h_s : nullptr,
+                          lw, MxRows{a.mx && shared_mode == 0 ? a.hq_mx_s : nullptr, a.hd_mx_s, a.shared.down.type == T_IQ3_S},
+                          shared_mode == 2 ? a.kt_h : nullptr, nbs);
     }
 }
 
@@ -787,17 +814,20 @@ __device__ __forceinline__ void mx_fill(uint8_t *tab) {
         o[MxTab<TY>::GRID / 16 + threadIdx.x] = reinterpret_cast<const uint4 *>(&c_mx_products.v[0][0])[threadIdx.x];
 }
 
-// One lane's 64 weights of its row's block.
-//   IQ2_S  w: qs of its two groups, sg: their sign dwords, e: low nibble of
-//          byte j the groups' qh fields of lookup j; TILE: high nibble of byte
-//          j the scale nibble of half group j, else sc holds the four nibbles.
-//   IQ3_S  w: lookup bytes of four quads (below), sg: their sign dwords;
-//          qh, sc: the row's qh bytes and scale nibbles, all groups.
+// One lane's 64 weights of its row's block, in the order of the tile copies:
+//   IQ2_S  w: qs of its two groups, sg: their sign dwords, e: byte j the
+//          groups' qh fields of lookup j (low nibble) and the scale nibble of
+//          half group j (high nibble).
+//   IQ3_S  w: lookup bytes of four quads: the lane's lookups are 2q and 2q + 1 of
+//          every group; quad 0 / 1 holds lookup 2q / 2q + 1 of groups 0, 1, 4, 5,
+//          quad 2 / 3 those of groups 2, 3, 6, 7 (byte i: the i-th listed
+//          group).  sg[j] byte i: the sign byte q of the i-th group of quads
+//          2j, 2j + 1.  qh, sc: the row's qh bytes and scale nibbles.
 template <int TY>
 struct MxW;
 template <>
 struct MxW<T_IQ2_S> {
-    uint32_t w[2], sg[2], e, sc, d;
+    uint32_t w[2], sg[2], e, d;
 };
 template <>
 struct MxW<T_IQ3_S> {
@@ -806,71 +836,128 @@ struct MxW<T_IQ3_S> {
 
 typedef uint32_t mx_u3 __attribute__((ext_vector_type(3)));
 
-// TILE: the matrix is a 16-row tile copy (k_units_to_tiles), whose lane slices
-// lie in lane order: u is the tile's first unit.  Else the row-major device
-// layout: u is the lane's unit.
-template <bool TILE>
-__device__ __forceinline__ void mx_load(const Planes &P, uint32_t u, int lane, MxW<T_IQ2_S> &o) {
-    const int q = lane >> 4;
-    if constexpr (TILE) {
-        const uint4 a = bld128(P, u * 64 + 16u * lane, 0);
-        o.w[0] = a.x, o.w[1] = a.y, o.sg[0] = a.z, o.sg[1] = a.w;
-        o.e = bld32(P, u * 16 + 4u * lane, 4 * P.U16);
-        o.d = bld16(P, u * 2 + 2u * (lane & 15), 5 * P.U16);
-        o.sc = 0;
-    } else {
-        const uint32_t u16 = u * 16, po = (uint32_t)(q >> 1) * P.U16 + 8u * (uint32_t)(q & 1);
-        const uint2 a = bld64(P, u16 + po, 0), c = bld64(P, u16 + po, 2 * P.U16);
-        o.w[0] = a.x, o.w[1] = a.y, o.sg[0] = c.x, o.sg[1] = c.y;
-        o.e = bld32(P, u16 + 4u * (uint32_t)(q >> 1), 4 * P.U16);
-        o.sc = bld16(P, u16 + 8u + 2u * (uint32_t)q, 4 * P.U16);
-        o.d = bld16(P, u * 2, 5 * P.U16);
-    }
-}
-template <bool TILE>
-__device__ __forceinline__ void mx_load(const Planes &P, uint32_t u, int lane, MxW<T_IQ3_S> &o) {
-    const int q = lane >> 4;
-    uint4 a;
-    uint2 s;
-    if constexpr (TILE) {
-        a = bld128(P, u * 64 + 16u * lane, 0);
-        s = bld64(P, u * 32 + 8u * lane, 4 * P.U16);
-        u += lane & 15;
-    } else {
-        a = bld128(P, u * 16 + (uint32_t)q * P.U16, 0);
-        s = bld64(P, u * 16 + (uint32_t)(q >> 1) * P.U16 + 8u * (uint32_t)(q & 1), 4 * P.U16);
-    }
+// The row's own bytes of unit u: d, and for IQ3_S qh and the scales.
+__device__ __forceinline__ void mx_load_row(const Planes &P, uint32_t u, MxW<T_IQ2_S> &o) { o.d = bld16(P, u * 2, 5 * P.U16); }
+__device__ __forceinline__ void mx_load_row(const Planes &P, uint32_t u, MxW<T_IQ3_S> &o) {
     const mx_u3 t = __builtin_bit_cast(mx_u3, __builtin_amdgcn_raw_buffer_load_b96(P.rsrc, u * 12, 6 * P.U16, WEIGHT_CPOL));
-    o.w[0] = a.x, o.w[1] = a.y, o.w[2] = a.z, o.w[3] = a.w;
-    o.sg[0] = s.x, o.sg[1] = s.y;
     o.qh[0] = t.x, o.qh[1] = t.y, o.sc = t.z;
     o.d = bld16(P, u * 2, 6 * P.U16 + 12 * P.U);
 }
 
-__device__ __forceinline__ void lanes32_swap(uint32_t &a, uint32_t &b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    a = r[0], b = r[1];
+__device__ __forceinline__ void mx_set_row(MxW<T_IQ2_S> &o, const MxW<T_IQ2_S> &r) { o.d = r.d; }
+__device__ __forceinline__ void mx_set_row(MxW<T_IQ3_S> &o, const MxW<T_IQ3_S> &r) {
+    o.qh[0] = r.qh[0], o.qh[1] = r.qh[1], o.sc = r.sc, o.d = r.d;
 }
-__device__ __forceinline__ void lanes16_swap(uint32_t &a, uint32_t &b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-    a = r[0], b = r[1];
+
+// Slice of a tile copy (k_units_to_tiles): u is the tile's first unit.
+__device__ __forceinline__ void mx_load(const Planes &P, uint32_t u, int lane, MxW<T_IQ2_S> &o) {
+    const uint4 a = bld128(P, u * 64 + 16u * lane, 0);
+    o.w[0] = a.x, o.w[1] = a.y, o.sg[0] = a.z, o.sg[1] = a.w;
+    o.e = bld32(P, u * 16 + 4u * lane, 4 * P.U16);
+    mx_load_row(P, u + (lane & 15), o);
+}
+__device__ __forceinline__ void mx_load(const Planes &P, uint32_t u, int lane, MxW<T_IQ3_S> &o) {
+    const uint4 a = bld128(P, u * 64 + 16u * lane, 0);
+    const uint2 s = bld64(P, u * 32 + 8u * lane, 4 * P.U16);
+    o.w[0] = a.x, o.w[1] = a.y, o.w[2] = a.z, o.w[3] = a.w;
+    o.sg[0] = s.x, o.sg[1] = s.y;
+    mx_load_row(P, u + (lane & 15), o);
+}
+
+// Row-major matrices: lane (q, c) reads whole block b0 + q of row c (u: its
+// unit), so each load covers 64 contiguous bytes of 16 rows; the four lanes of a
+// row exchange quarters for blocks (v_permlane32_swap / 16_swap, a 4 x 4
+// transposition), after which slice j is block b0 + j in the order above.
+// Eight blocks at a time: load set h gives lane (q, c) block b0 + 2q + c / 8 of
+// row 8h + c % 8, 128 contiguous bytes of eight rows; lanes c and c ^ 8 swap
+// across the sets (mx_rows8), set p then holds block b0 + 2q + p of row c and
+// its slice j block b0 + 2j + p.
+template <int TY>
+struct MxRaw {
+    uint32_t v[TY == T_IQ2_S ? 20 : 24];   // IQ2_S qs, signs, qh, scales; IQ3_S qs, signs
+};
+template <int TY>
+__device__ __forceinline__ void mx_load_raw(const Planes &P, uint32_t u, MxRaw<TY> &o) {
+#pragma unroll
+    for (int k = 0; k < (TY == T_IQ2_S ? 5 : 6); ++k) {
+        const uint4 a = bld128(P, u * 16, k * P.U16);
+        o.v[4 * k] = a.x, o.v[4 * k + 1] = a.y, o.v[4 * k + 2] = a.z, o.v[4 * k + 3] = a.w;
+    }
+}
+
+__device__ __forceinline__ void mx_rows8(uint32_t &a, uint32_t &b) {
+    const int x = (int)a, y = (int)b;   // row_ror:8 into lanes 8-15 / 0-7 of each row of 16
+    a = (uint32_t)__builtin_amdgcn_update_dpp(x, y, 0x128, 0xf, 0xc, false);
+    b = (uint32_t)__builtin_amdgcn_update_dpp(y, x, 0x128, 0xf, 0x3, false);
+}
+// t[k] of lane quarter q becomes t[q] of lane quarter k.
+__device__ __forceinline__ void mx_exchange(uint32_t &t0, uint32_t &t1, uint32_t &t2, uint32_t &t3) {
+    auto r = __builtin_amdgcn_permlane32_swap(t0, t2, false, false);
+    t0 = r[0], t2 = r[1];
+    r = __builtin_amdgcn_permlane32_swap(t1, t3, false, false);
+    t1 = r[0], t3 = r[1];
+    r = __builtin_amdgcn_permlane16_swap(t0, t1, false, false);
+    t0 = r[0], t1 = r[1];
+    r = __builtin_amdgcn_permlane16_swap(t2, t3, false, false);
+    t2 = r[0], t3 = r[1];
+}
+// 4 x 4 byte transposition: byte i of o[k] = byte k of (a, b, c, d)[i].
+__device__ __forceinline__ void mx_bytes4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t (&o)[4]) {
+    const uint32_t ab0 = perm(b, a, 0x05010400u), ab1 = perm(b, a, 0x07030602u);   // a0 b0 a1 b1, a2 b2 a3 b3
+    const uint32_t cd0 = perm(d, c, 0x05010400u), cd1 = perm(d, c, 0x07030602u);
+    o[0] = perm(cd0, ab0, 0x05040100u), o[1] = perm(cd0, ab0, 0x07060302u);
+    o[2] = perm(cd1, ab1, 0x05040100u), o[3] = perm(cd1, ab1, 0x07060302u);
+}
+__device__ __forceinline__ void mx_slices(const MxRaw<T_IQ2_S> &r, MxW<T_IQ2_S> (&o)[4]) {
+    uint32_t e[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {   // quarter k of the lane's block
+        const uint32_t qh = (r.v[16 + (k >> 1)] >> (4 * (k & 1))) & 0x0f0f0f0fu;
+        const uint32_t sc = perm(0u, r.v[18 + (k >> 1)], k & 1 ? 0x03030202u : 0x01010000u);
+        e[k] = qh | (((sc << 4) & 0x00f000f0u) | (sc & 0xf000f000u));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        uint32_t w[4] = {r.v[i], r.v[2 + i], r.v[4 + i], r.v[6 + i]};
+        uint32_t s[4] = {r.v[8 + i], r.v[10 + i], r.v[12 + i], r.v[14 + i]};
+        mx_exchange(w[0], w[1], w[2], w[3]);
+        mx_exchange(s[0], s[1], s[2], s[3]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j].w[i] = w[j], o[j].sg[i] = s[j];
+    }
+    mx_exchange(e[0], e[1], e[2], e[3]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j].e = e[j];
+}
+__device__ __forceinline__ void mx_slices(const MxRaw<T_IQ3_S> &r, MxW<T_IQ3_S> (&o)[4]) {
+    // qs bytes of group g: v[2g], v[2g + 1]; lane quarter k takes bytes 2k, 2k + 1
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int g0 = 4 * j / 2;   // quads 2j, 2j + 1: groups 2j, 2j + 1, 2j + 4, 2j + 5
+        uint32_t lo[4], hi[4], s[4], q0[4], q1[4];
+        mx_bytes4(r.v[2 * g0], r.v[2 * g0 + 2], r.v[2 * g0 + 8], r.v[2 * g0 + 10], lo);       // lookups 0-3
+        mx_bytes4(r.v[2 * g0 + 1], r.v[2 * g0 + 3], r.v[2 * g0 + 9], r.v[2 * g0 + 11], hi);   // lookups 4-7
+        mx_bytes4(r.v[16 + g0], r.v[17 + g0], r.v[20 + g0], r.v[21 + g0], s);
+        q0[0] = lo[0], q0[1] = lo[2], q0[2] = hi[0], q0[3] = hi[2];   // even lookups of quarters 0-3
+        q1[0] = lo[1], q1[1] = lo[3], q1[2] = hi[1], q1[3] = hi[3];
+        mx_exchange(q0[0], q0[1], q0[2], q0[3]);
+        mx_exchange(q1[0], q1[1], q1[2], q1[3]);
+        mx_exchange(s[0], s[1], s[2], s[3]);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) o[b].w[2 * j] = q0[b], o[b].w[2 * j + 1] = q1[b], o[b].sg[j] = s[b];
+    }
 }
 
 // Integer block sums bs[i] of (token 4q + i, row c) from the lane's weights
 // and its 64 quants of token c (tok[m]: 16 bytes).
-template <bool TILE>
-__device__ __forceinline__ void mx_block(const MxW<T_IQ2_S> &o, const uint4 (&tok)[4], const uint8_t *tab, int lane,
+__device__ __forceinline__ void mx_block(const MxW<T_IQ2_S> &o, const uint4 (&tok)[4], const uint8_t *tab, int,
                                          int32_t (&bs)[4]) {
     const GridRef<T_IQ2_S> grid(tab);
-    // row-major: the lane's qh fields are fields 2 (q & 1), + 1 of its dword
-    const uint32_t e = TILE ? o.e : o.e >> (4 * ((lane >> 4) & 1));
     mx_i4 lo = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-        const Iq2sGroup g = Iq2sGroup::make(o.w[m >> 1], e, m >> 1, o.sg[m >> 1]);
-        const uint32_t na = TILE ? (e >> (8 * m)) & 0xf0u
-                                 : (m == 0 ? o.sc << 4 : o.sc >> (4 * m - 4)) & 0xf0u;
-        const uint4 t = *reinterpret_cast<const uint4 *>(tab + MxTab<T_IQ2_S>::GRID + na);
+        const Iq2sGroup g = Iq2sGroup::make(o.w[m >> 1], o.e, m >> 1, o.sg[m >> 1]);
+        const uint4 t = *reinterpret_cast<const uint4 *>(tab + MxTab<T_IQ2_S>::GRID + ((o.e >> (8 * m)) & 0xf0u));
         mx_i4 bl, bh;
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
@@ -888,34 +975,9 @@ __device__ __forceinline__ void mx_block(const MxW<T_IQ2_S> &o, const uint4 (&to
     for (int i = 0; i < 4; ++i) bs[i] = (hi[i] << 8) + lo[i];
 }
 
-// IQ3_S quads: the lane's lookups are 2q and 2q + 1 of every group; quad 0 / 1
-// holds lookup 2q / 2q + 1 of groups 0, 1, 4, 5, quad 2 / 3 those of groups 2,
-// 3, 6, 7 (byte i: the i-th listed group).  Sign dword j: byte i the sign byte
-// q of the i-th group of quads 2j, 2j + 1.  A tile copy holds them so; the
-// row-major slice of lane q is groups 2q, 2q + 1 whole, and the four lanes of
-// a row exchange 4 x 4 pieces (v_permlane32_swap / 16_swap).
-__device__ __forceinline__ void mx_iq3_exchange(const MxW<T_IQ3_S> &o, uint32_t (&qd)[4], uint32_t (&sg)[2]) {
-    // t[j]: the lookups 2j, 2j + 1 of both groups, for the row's lane j
-    uint32_t t[4] = {perm(o.w[2], o.w[0], 0x05040100u), perm(o.w[2], o.w[0], 0x07060302u),
-                     perm(o.w[3], o.w[1], 0x05040100u), perm(o.w[3], o.w[1], 0x07060302u)};
-    lanes32_swap(t[0], t[2]);
-    lanes32_swap(t[1], t[3]);
-    lanes16_swap(t[0], t[1]);
-    lanes16_swap(t[2], t[3]);
-    qd[0] = perm(t[2], t[0], 0x06040200u), qd[1] = perm(t[2], t[0], 0x07050301u);
-    qd[2] = perm(t[3], t[1], 0x06040200u), qd[3] = perm(t[3], t[1], 0x07050301u);
-    uint32_t w0 = perm(o.sg[1], o.sg[0], 0x05010400u), w1 = perm(o.sg[1], o.sg[0], 0x07030602u);
-    lanes32_swap(w0, w1);
-    sg[0] = perm(w1, w0, 0x05040100u), sg[1] = perm(w1, w0, 0x07060302u);
-    lanes16_swap(sg[0], sg[1]);
-}
-
-template <bool TILE>
 __device__ __forceinline__ void mx_block(const MxW<T_IQ3_S> &o, const uint4 (&tok)[4], const uint8_t *tab, int lane,
                                          int32_t (&bs)[4]) {
     const Iq3SignedRef grid(tab);
-    uint32_t qd[4] = {o.w[0], o.w[1], o.w[2], o.w[3]}, sg[2] = {o.sg[0], o.sg[1]};
-    if constexpr (!TILE) mx_iq3_exchange(o, qd, sg);
     // bits 0, 1 of byte i: the high index bits of lookups 2q, 2q + 1
     const uint32_t ta = o.qh[0] >> (2 * (lane >> 4)), tb = o.qh[1] >> (2 * (lane >> 4));
     const uint32_t hb[2] = {perm(tb, ta, 0x05040100u), perm(tb, ta, 0x07060302u)};
@@ -925,8 +987,8 @@ __device__ __forceinline__ void mx_block(const MxW<T_IQ3_S> &o, const uint4 (&to
         const int j = k >> 1, odd = k & 1;
         // iq3_signed_offset = x + 256 y per byte
         const uint32_t h = (odd ? hb[j] << 1 : hb[j] << 2) & 0x04040404u;
-        const uint32_t s = (odd ? sg[j] >> 1 : sg[j] << 3) & 0x78787878u;
-        const uint32_t x = qd[k] & 0xfcfcfcfcu, y = (qd[k] & 0x03030303u) | h | s;
+        const uint32_t s = (odd ? o.sg[j] >> 1 : o.sg[j] << 3) & 0x78787878u;
+        const uint32_t x = o.w[k] & 0xfcfcfcfcu, y = (o.w[k] & 0x03030303u) | h | s;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             word[odd][(i & 1) + 4 * (i >> 1) + 2 * j] = grid.word(perm(y, x, 0x0c0c0000u | ((4u + i) << 8) | (uint32_t)i));
@@ -950,175 +1012,235 @@ __device__ __forceinline__ void mx_block(const MxW<T_IQ3_S> &o, const uint4 (&to
     }
 }
 
-// One wave step's inputs: NM slices of the lane's rows and its quants of
-// token c.
+// LDS of a matrix-core stream workgroup: the tables and the token scales.
+__host__ __device__ constexpr int mx_lds_bytes(int ty) {
+    return (ty == T_IQ2_S ? MxTab<T_IQ2_S>::BYTES : MxTab<T_IQ3_S>::BYTES) + MX_MAX_NB * 16 * 4;
+}
+
+// The wave's f32 chains of one tile: the lane's four (token 4q + i, row c)
+// results of NM matrices (or row tiles), blocks added in order.
 template <int TY, int NM>
-struct MxStep {
-    MxW<TY> w[NM];
-    uint4 tok[4];
+struct MxChains {
+    float c[NM][4];
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int t = 0; t < NM; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c[t][i] = 0.0f;
+    }
+    __device__ __forceinline__ void add(int t, const MxW<TY> &w, const uint4 (&tok)[4], const float4 &d8, const uint8_t *tab,
+                                        int lane) {
+        int32_t bs[4];
+        mx_block(w, tok, tab, lane, bs);
+        const float d = f16_to_f32(w.d), e[4] = {d8.x, d8.y, d8.z, d8.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[t][i] = __fadd_rn(c[t][i], __fmul_rn(__fmul_rn(d, e[i]), (float)bs[i]));
+    }
+    template <class Out>
+    __device__ __forceinline__ void finish(int q, int row, Out &out) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float res[NM];
+#pragma unroll
+            for (int t = 0; t < NM; ++t) res[t] = TY == T_IQ2_S ? __fmul_rn(0.125f, c[t][i]) : c[t][i];   // q8_k.rs:369
+            out(4 * q + i, row, res);
+        }
+        clear();
+    }
 };
 
-// Dynamic LDS of a matrix-core stream workgroup (beside its static tables and
-// scales): with split > 1, per tile the f32 terms [matrix][block][token][row].
-__host__ __device__ constexpr int mx_dyn_lds(int nm, int split, int nb) {
-    return split > 1 ? (MX_WAVES / split) * nm * nb * 256 * 4 : 0;
-}
-__host__ __device__ constexpr int mx_lds_bytes(int ty, int nm, int split, int nb) {
-    return (ty == T_IQ2_S ? MxTab<T_IQ2_S>::BYTES : MxTab<T_IQ3_S>::BYTES) +
-           (split > 1 ? mx_dyn_lds(nm, split, nb) : MX_MAX_NB * 16 * 4);
-}
-
-// Rows [r0, r1) (multiples of 16 NM') of NM tiles per step against the chunk's
+// Rows [r0, r1) (a multiple of 16) of NM tiles per step against the chunk's
 // tokens: the NM matrices mv (gate and up), or, PAIR, NM adjacent 16-row tiles
-// of the one matrix mv[0], which share the step's token operands.
-//   S = 1: the waves take tiles r0 + RW wid, + 4 RW, ... (RW = 16 or 16 NM
-//     rows) to r1, computing every block of a tile in order, the chains of
-//     the lane's four (token, row) results in registers; s_d8[16 b + i] is the
-//     scale of token i's block b.
-//   S > 1: the workgroup holds MX_WAVES / S tiles, the S waves of a tile take
-//     its blocks j, j + S, ... and write the f32 term (d * d8) * (float)bsum of
-//     each (row, token, block) to LDS; after a workgroup barrier one thread
-//     per (tile, token, row) folds its terms in block order (lbh_rows.h: chain =
-//     0 + t_0 + t_1 + ...) and calls out(token column, row, values).  bd: the
-//     scales of the lane's tokens, d8_of(i)[b].
-// bq: the lane's token operand row.  The first step's loads are issued before
-// `prologue` (tables and scales to LDS, ended by a workgroup barrier); then
-// each step's loads are in flight while the one before is computed.
-template <int TY, int NM, int S, bool TILE, bool PAIR, class Prologue, class D8, class Out>
+// of the one matrix mv[0], which share the step's token operands.  The waves
+// take tiles r0 + RW wid, + 4 RW, ... (RW = 16 or 16 NM rows) to r1, every
+// block of a tile in order; s_d8[16 b + i] is the scale of token i's block b,
+// bq the lane's token operand row.  out(token column, row, values) is called
+// once per (token, row).  The first loads are issued before `prologue` (tables
+// and scales to LDS, ended by a workgroup barrier); then a step's loads are in
+// flight while the one before is computed.
+//   TILE: tile copies, one block per step.
+//   else: row-major matrices, four blocks (IQ2_S) or eight (IQ3_S, whose rows
+//   are short) per load step, exchanged into slices (mx_slices).  Loading 16
+//   bytes of each line at a time, block by block, took 1.5 to 2 times the tile
+//   copies' time; four blocks still fetch half of the lines twice from beyond
+//   L2, and eight with no spare registers to load ahead measured slower (64
+//   tokens, gate/up: 231 us with four, 265 us with eight).
+template <int TY, int NM, bool TILE, bool PAIR, class Prologue, class Out>
 __device__ __forceinline__ void mx_tiles(const MatView *mv, int r0, int r1, int nb, const uint8_t *bq, const uint8_t *tab,
-                                         const float *s_d8, float *terms, Prologue prologue, D8 d8_of, Out out) {
-    constexpr int NP = PAIR ? 1 : NM, RW = PAIR ? 16 * NM : 16;
+                                         const float *s_d8, Prologue prologue, Out out) {
+    constexpr int NP = PAIR ? 1 : NM, RW = PAIR ? 16 * NM : 16, RG = RW * MX_WAVES;
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, q = lane >> 4;
-    const int tl = wid / S, j = wid - tl * S;
-    const int rt0 = r0 + RW * tl;
-    // steps of the wave: its blocks of one tile (S > 1), or its tiles' blocks (S = 1)
-    const int tiles = S > 1 ? 1 : (r1 - rt0 + RW * MX_WAVES - 1) / (RW * MX_WAVES);
-    const int steps = rt0 < r1 ? (S > 1 ? (j < nb ? (nb - j + S - 1) / S : 0) : tiles * nb) : 0;
+    const int rt0 = r0 + RW * wid;
+    const int tiles = rt0 < r1 ? (r1 - rt0 + RG - 1) / RG : 0;
     Planes P[NP];
 #pragma unroll
     for (int t = 0; t < NP; ++t) P[t] = make_planes(mv[t].planes, mv[t].units, mv[t].bytes);
-    const uint8_t *tp = bq + 64 * q;
+    const uint8_t *tp = bq + 16 * q;
+    auto tokens = [&](int b, uint4 (&tok)[4]) {
+        const uint4 *src = reinterpret_cast<const uint4 *>(tp + b * 256);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) tok[k] = src[4 * k];
+    };
+    auto scales = [&](int b) { return *reinterpret_cast<const float4 *>(s_d8 + 16 * b + 4 * q); };
+    MxChains<TY, NM> ch;
+    ch.clear();
     // The loads are unconditional: a step past the wave's last one reloads the
     // last (in bounds, never used), so the compiler's wait before a step's use
     // counts exactly the younger step's loads.
-    int ir = rt0 < r1 ? rt0 : r0, ib = S > 1 ? (j < nb ? j : nb - 1) : 0;   // next tile row and block to load
-    auto issue = [&](MxStep<TY, NM> &st) {
+    int ir = rt0 < r1 ? rt0 : r0, ib = 0;   // next tile row and block to load
+    int pr = rt0, pb = 0;                   // tile row and block of the step being computed
+    if constexpr (TILE) {
+        const int steps = tiles * nb;
+        struct Step {
+            MxW<TY> w[NM];
+            uint4 tok[4];
+        };
+        auto issue = [&](Step &st) {
 #pragma unroll
-        for (int t = 0; t < NM; ++t) {
-            const int r = PAIR ? ir + 16 * t : ir;
-            const uint32_t u = TILE ? (uint32_t)(r * nb + 16 * ib) : (uint32_t)((r + c) * nb + ib);
-            mx_load<TILE>(P[PAIR ? 0 : t], u, lane, st.w[t]);
-        }
-        const uint4 *src = reinterpret_cast<const uint4 *>(tp + ib * 256);
+            for (int t = 0; t < NM; ++t)
+                mx_load(P[PAIR ? 0 : t], (uint32_t)((PAIR ? ir + 16 * t : ir) * nb + 16 * ib), lane, st.w[t]);
+            tokens(ib, st.tok);
+            if (ib + 1 < nb)
+                ++ib;
+            else if (ir + RG < r1)
+                ir += RG, ib = 0;
+        };
+        auto process = [&](const Step &st) {
+            const float4 d8 = scales(pb);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) st.tok[k] = src[k];
-        if constexpr (S > 1) {
-            ib = ib + S < nb ? ib + S : ib;
-        } else if (++ib == nb) {
-            if (ir + RW * MX_WAVES < r1)
-                ir += RW * MX_WAVES, ib = 0;
-            else
-                ib = nb - 1;
-        }
-    };
-    float chain[NM][4];   // S == 1
-#pragma unroll
-    for (int t = 0; t < NM; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) chain[t][i] = 0.0f;
-    int pr = rt0, pb = S > 1 ? j : 0;   // tile row and block of the step being computed
-    auto process = [&](const MxStep<TY, NM> &st) {
-        float d8[4];
-        if constexpr (S == 1) {
-            const float4 v = *reinterpret_cast<const float4 *>(s_d8 + 16 * pb + 4 * q);
-            d8[0] = v.x, d8[1] = v.y, d8[2] = v.z, d8[3] = v.w;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) d8[i] = d8_of(4 * q + i)[pb];
-        }
-#pragma unroll
-        for (int t = 0; t < NM; ++t) {
-            int32_t bs[4];
-            mx_block<TILE>(st.w[t], st.tok, tab, lane, bs);
-            const float d = f16_to_f32(st.w[t].d);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float term = __fmul_rn(__fmul_rn(d, d8[i]), (float)bs[i]);
-                if constexpr (S == 1)
-                    chain[t][i] = __fadd_rn(chain[t][i], term);   // blocks in order
-                else
-                    terms[((tl * NM + t) * nb + pb) * 256 + 16 * (4 * q + i) + c] = term;
+            for (int t = 0; t < NM; ++t) ch.add(t, st.w[t], st.tok, d8, tab, lane);
+            if (++pb == nb) {
+                ch.finish(q, pr + c, out);
+                pr += RG, pb = 0;
             }
-        }
-        if constexpr (S > 1) {
-            pb += S;
-        } else if (++pb == nb) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float res[NM];
-#pragma unroll
-                for (int t = 0; t < NM; ++t) {
-                    res[t] = TY == T_IQ2_S ? __fmul_rn(0.125f, chain[t][i]) : chain[t][i];   // q8_k.rs:369
-                    chain[t][i] = 0.0f;
-                }
-                out(4 * q + i, pr + c, res);
-            }
-            pr += RW * MX_WAVES, pb = 0;
-        }
-    };
-    MxStep<TY, NM> sa, sb;
-    issue(sa);
-    prologue();
-    for (int s = 0; s < steps; s += 2) {
-        issue(sb);
-        process(sa);
-        if (s + 1 >= steps) break;
+        };
+        Step sa, sb;
         issue(sa);
-        process(sb);
-    }
-    if constexpr (S > 1) {
-        __syncthreads();
-        for (int p = threadIdx.x; p < (MX_WAVES / S) * 256; p += MX_THREADS) {
-            const int ptl = p >> 8, cc = (p >> 4) & 15, row = p & 15;
-            const float *src = terms + ptl * NM * nb * 256 + cc * 16 + row;
-            float res[NM];
+        prologue();
+        for (int s = 0; s < steps; s += 2) {
+            issue(sb);
+            process(sa);
+            if (s + 1 >= steps) break;
+            issue(sa);
+            process(sb);
+        }
+    } else {
+        static_assert(!PAIR || NM == 1, "row-major streams take one row tile per step");
+        constexpr int G = TY == T_IQ2_S ? 4 : 8, H = G / 4;   // blocks per group, register sets of four
+        const int groups = tiles * ((nb + G - 1) / G);
+        MxRaw<TY> raw[H][NM];
+        auto issue = [&](int h) {
+            const int b = G == 8 ? ib + 2 * q + (c >> 3) : ib + q, r = G == 8 ? 8 * h + (c & 7) : c;
 #pragma unroll
-            for (int t = 0; t < NM; ++t) {
-                float ch = 0.0f;
-                for (int b = 0; b < nb; ++b) ch = __fadd_rn(ch, src[(t * nb + b) * 256]);
-                res[t] = TY == T_IQ2_S ? __fmul_rn(0.125f, ch) : ch;  // q8_k.rs:369
+            for (int t = 0; t < NM; ++t) mx_load_raw(P[t], (uint32_t)((ir + r) * nb + (b < nb ? b : nb - 1)), raw[h][t]);
+        };
+#pragma unroll
+        for (int h = 0; h < H; ++h) issue(h);
+        prologue();
+        for (int s = 0; s < groups; ++s) {
+            const int b0 = pb, n = nb - b0 < G ? nb - b0 : G;
+            uint4 tok[2][4];
+            MxW<TY> row[2][NM];   // the rows' own bytes of the block
+            auto next = [&](int k) {
+                const int b = b0 + k < nb ? b0 + k : nb - 1;
+                tokens(b, tok[k & 1]);
+#pragma unroll
+                for (int t = 0; t < NM; ++t) mx_load_row(P[t], (uint32_t)((pr + c) * nb + b), row[k & 1][t]);
+            };
+            next(0);
+            MxW<TY> w[H][NM][4];
+            if constexpr (G == 8) {
+#pragma unroll
+                for (int k = 0; k < (int)(sizeof(raw[0][0].v) / 4); ++k)
+#pragma unroll
+                    for (int t = 0; t < NM; ++t) mx_rows8(raw[0][t].v[k], raw[H - 1][t].v[k]);
             }
-            out(cc, r0 + 16 * ptl + row, res);
+#pragma unroll
+            for (int h = 0; h < H; ++h)
+#pragma unroll
+                for (int t = 0; t < NM; ++t) mx_slices(raw[h][t], w[h][t]);
+            if (ib + G < nb)
+                ib += G;
+            else if (ir + RG < r1)
+                ir += RG, ib = 0;
+            if (G == 4) issue(0);
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                if (k < n) {
+                    next(k + 1);
+                    const float4 d8 = scales(b0 + k);
+#pragma unroll
+                    for (int t = 0; t < NM; ++t) {
+                        MxW<TY> &x = w[G == 8 ? k & 1 : 0][t][G == 8 ? k >> 1 : k];
+                        mx_set_row(x, row[k & 1][t]);
+                        ch.add(t, x, tok[k & 1], d8, tab, lane);
+                    }
+                }
+                if (G == 8 && k == 3) issue(0);   // half of the set registers are free again
+            }
+            if (G == 8) issue(H - 1);
+            pb += G;
+            if (pb >= nb) {
+                ch.finish(q, pr + c, out);
+                pr += RG, pb = 0;
+            }
         }
     }
 }
 
 // Tables and token scales of a matrix-core workgroup into LDS.
-template <int TY, int S, class D8>
+template <int TY, class D8>
 __device__ __forceinline__ void mx_prologue(uint8_t *tab, float *s_d8, int n, int nb, D8 d8_of) {
     mx_fill<TY>(tab);
-    if constexpr (S == 1)
-        for (int k = threadIdx.x; k < 16 * nb; k += MX_THREADS) {
-            const int i = k & 15;
-            s_d8[k] = i < n ? d8_of(i)[k >> 4] : 0.0f;
-        }
+    for (int k = threadIdx.x; k < 16 * nb; k += MX_THREADS) {
+        const int i = k & 15;
+        s_d8[k] = i < n ? d8_of(i)[k >> 4] : 0.0f;
+    }
     __syncthreads();
 }
 
+// The shared expert's K-quant rows in a stage launch (lbh_kt.h): workgroup wg of
+// kt_wgs(): 64 rows (one 16-row tile per wave) of matrix m against KT_NT token
+// tiles; the token groups of a row quad are neighbours, so its weights are
+// fetched once.
+constexpr int KT_NT = 1;
+__host__ __device__ inline int kt_groups(int n_tokens) { return ((n_tokens + 15) / 16 + KT_NT - 1) / KT_NT; }
+template <int TY>
+__device__ __forceinline__ void kt_workgroup(const uint8_t *w, int rows, int nb, const uint8_t *tok, int n_tokens, float *y,
+                                             int wg) {
+    const int ng = kt_groups(n_tokens), quad = wg / ng, g = wg - quad * ng;
+    const int rt = 4 * quad + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    kt_rows<TY, KT_NT>(w, kt_w_bytes(TY, rows, nb), rt, nb, tok, g * KT_NT, (n_tokens + 15) / 16,
+                       [&](int t, int r, float v) {
+                           if (t < n_tokens) y[(long long)t * rows + rt * 16 + r] = v;
+                       });
+}
+
 // Gate/up on the matrix cores (as k_mb_gate_up): workgroup (chunk, row tile).
-// TILE: the chunks whose expert has tile copies, else the others.
-template <int TY, bool SHARED, int S, bool TILE>
-__global__ void __launch_bounds__(MX_THREADS) k_mx_gate_up(BatchArgs a) {
-    extern __shared__ __align__(16) uint8_t smem[];
+// TILE: the chunks whose expert has tile copies, else the others.  NM: gate and
+// up in one workgroup (2) or in two (1: few chunks of row-major matrices).  KTY: the
+// first kt_wgs workgroups run the shared expert's gate and up (K-quant type
+// KTY), so that one launch holds all of the stage's work.
+template <int TY, bool SHARED, bool TILE, int NM, int KTY = 0>
+__global__ void __launch_bounds__(MX_THREADS) k_mx_gate_up(BatchArgs a, int kt_wgs) {
     __shared__ __align__(16) uint8_t tab[MxTab<TY>::BYTES];
-    __shared__ __align__(16) float s_d8[S == 1 ? MX_MAX_NB * 16 : 4];
+    __shared__ __align__(16) float s_d8[MX_MAX_NB * 16];
     if (a.plan[1]) return;
     const int nb = a.hidden / 256;
-    const int ffn = SHARED ? a.ffn_s : a.ffn_r, rt = S == 1 ? a.mx_rows_gu : 16 * MX_WAVES / S;
-    const int tiles = (ffn + rt - 1) / rt;
-    const int ci = blockIdx.x / tiles, tile = blockIdx.x - ci * tiles;
+    if constexpr (KTY != 0) {
+        if ((int)blockIdx.x < kt_wgs) {
+            const int half = kt_wgs / 2, up = (int)blockIdx.x >= half;
+            kt_workgroup<KTY>(a.kt_w[up], a.ffn_s, nb, a.kt_x, a.n_tokens, up ? a.u_s : a.g_s, (int)blockIdx.x - up * half);
+            return;
+        }
+    }
+    const int wg = (int)blockIdx.x - kt_wgs;
+    // NM = 1: gate and up of a row tile are neighbouring workgroups.
+    const int ffn = SHARED ? a.ffn_s : a.ffn_r, rt = a.mx_rows_gu;
+    const int tiles = (ffn + rt - 1) / rt * (3 - NM);
+    const int ci = wg / tiles, up = NM == 1 ? (wg - ci * tiles) & 1 : 0, tile = (wg - ci * tiles) / (3 - NM);
     const int r0 = tile * rt, r1 = r0 + rt < ffn ? r0 + rt : ffn;
     int p0, n;
     MatView mv[2];
@@ -1139,30 +1261,37 @@ __global__ void __launch_bounds__(MX_THREADS) k_mx_gate_up(BatchArgs a) {
     };
     auto d8_of = [&](int i) { return a.xd_mx + token(i) * nb; };
     float *g = SHARED ? a.g_s : a.g_r, *u = SHARED ? a.u_s : a.u_r;
-    mx_tiles<TY, 2, S, TILE, false>(
-        mv, r0, r1, nb, a.xq_mx + token(threadIdx.x & 15) * nb * 256, tab, s_d8, reinterpret_cast<float *>(smem),
-        [&]() { mx_prologue<TY, S>(tab, s_d8, n, nb, d8_of); }, d8_of,
+    if (up) g = u, mv[0] = mv[1];
+    mx_tiles<TY, NM, TILE, false>(
+        mv, r0, r1, nb, a.xq_mx + token(threadIdx.x & 15) * nb * 256, tab, s_d8,
+        [&]() { mx_prologue<TY>(tab, s_d8, n, nb, d8_of); },
         [&](int i, int r, const float *res) {
             if (i < n) {
                 const long long o = (long long)(p0 + i) * ffn + r;
                 g[o] = res[0];
-                u[o] = res[1];
+                if constexpr (NM == 2) u[o] = res[1];
             }
         });
 }
 
-// Down on the matrix cores (as k_mb_down); with S = 1 each wave takes two
+// Down on the matrix cores (as k_mb_down); over tile copies each wave takes two
 // adjacent 16-row tiles a step, which share the token operands.
-template <int TY, bool SHARED, int S, bool TILE>
-__global__ void __launch_bounds__(MX_THREADS) k_mx_down(BatchArgs a) {
-    extern __shared__ __align__(16) uint8_t smem[];
+template <int TY, bool SHARED, bool TILE, int KTY = 0>
+__global__ void __launch_bounds__(MX_THREADS) k_mx_down(BatchArgs a, int kt_wgs) {
     __shared__ __align__(16) uint8_t tab[MxTab<TY>::BYTES];
-    __shared__ __align__(16) float s_d8[S == 1 ? MX_MAX_NB * 16 : 4];
+    __shared__ __align__(16) float s_d8[MX_MAX_NB * 16];
     if (a.plan[1]) return;
+    if constexpr (KTY != 0) {
+        if ((int)blockIdx.x < kt_wgs) {
+            kt_workgroup<KTY>(a.kt_w[2], a.hidden, a.ffn_s / 256, a.kt_h, a.n_tokens, a.d_s, (int)blockIdx.x);
+            return;
+        }
+    }
+    const int wg = (int)blockIdx.x - kt_wgs;
     const int nb = (SHARED ? a.ffn_s : a.ffn_r) / 256;
-    const int rt = S == 1 ? a.mx_rows_d : 16 * MX_WAVES / S;
+    const int rt = a.mx_rows_d;
     const int tiles = (a.hidden + rt - 1) / rt;
-    const int ci = blockIdx.x / tiles, tile = blockIdx.x - ci * tiles;
+    const int ci = wg / tiles, tile = wg - ci * tiles;
     const int r0 = tile * rt, r1 = r0 + rt < a.hidden ? r0 + rt : a.hidden;
     int p0, n;
     MatView mv[1];
@@ -1181,16 +1310,25 @@ __global__ void __launch_bounds__(MX_THREADS) k_mx_down(BatchArgs a) {
     const int c = (int)(threadIdx.x & 15) < n ? (int)(threadIdx.x & 15) : n - 1;
     auto d8_of = [&](int i) { return hd + (long long)(p0 + (i < n ? i : n - 1)) * nb; };
     float *d = SHARED ? a.d_s : a.d_r;
-    constexpr int NM = S == 1 ? 2 : 1;
-    mx_tiles<TY, NM, S, TILE, true>(
-        mv, r0, r1, nb, hq + (long long)(p0 + c) * nb * 256, tab, s_d8, reinterpret_cast<float *>(smem),
-        [&]() { mx_prologue<TY, S>(tab, s_d8, n, nb, d8_of); }, d8_of,
+    constexpr int NM = TILE ? 2 : 1;
+    mx_tiles<TY, NM, TILE, true>(
+        mv, r0, r1, nb, hq + (long long)(p0 + c) * nb * 256, tab, s_d8,
+        [&]() { mx_prologue<TY>(tab, s_d8, n, nb, d8_of); },
         [&](int i, int r, const float *res) {
             if (i < n) {
 #pragma unroll
                 for (int t = 0; t < NM; ++t) d[(long long)(p0 + i) * a.hidden + r + 16 * t] = res[t];
             }
         });
+}
+
+// The shared expert's K-quant rows alone (a batch whose routed chunks all run
+// on the VALU).
+template <int TY>
+__global__ void __launch_bounds__(MX_THREADS) k_kt_rows(const uint8_t *w0, const uint8_t *w1, int rows, int nb,
+                                                        const uint8_t *tok, int n_tokens, float *y0, float *y1, int half) {
+    const int second = (int)blockIdx.x >= half;
+    kt_workgroup<TY>(second ? w1 : w0, rows, nb, tok, n_tokens, second ? y1 : y0, (int)blockIdx.x - second * half);
 }
 
 // Ordered combine of one token's routed outputs in its slot (ascending id)
@@ -1247,10 +1385,10 @@ static int stream_lds_of(int ty, int nm, int tc, int nb) {
 
 // LDS of the launches of one stream: the VALU kernel's, and the matrix-core
 // kernel's when it runs that type.
-static int stream_max(const BatchArgs &a, int ty, int nm, int nb, int split) {
+static int stream_max(const BatchArgs &a, int ty, int nm, int nb) {
     const int v = stream_lds_of(ty, nm, valu_cap(a, ty), nb);
     if (!a.mx || (ty != T_IQ2_S && ty != T_IQ3_S)) return v;
-    const int m = mx_lds_bytes(ty, nm, split < 1 ? 1 : split, nb);
+    const int m = mx_lds_bytes(ty);
     return v > m ? v : m;
 }
 
@@ -1263,10 +1401,10 @@ int batch_lds_bytes(const BatchArgs &a, int stage) {
         const int sort = (a.n_experts * W + 3 * a.n_experts + 2 * MB_THREADS + 4) * 4;
         return sort > MB_WAVES * 4 * 292 ? sort : MB_WAVES * 4 * 292;
     }
-    case 1: return stream_max(a, a.type_gate_r, 2, nbh, a.mx_split_gu);
-    case 2: return a.has_shared ? stream_max(a, a.shared.gate.type, 2, nbh, a.mx_split_gu) : 0;
-    case 3: return stream_max(a, a.type_down_r, 1, nbr, a.mx_split_d);
-    default: return a.has_shared ? stream_max(a, a.shared.down.type, 1, nbs, a.mx_split_d) : 0;
+    case 1: return stream_max(a, a.type_gate_r, 2, nbh);
+    case 2: return a.has_shared ? stream_max(a, a.shared.gate.type, 2, nbh) : 0;
+    case 3: return stream_max(a, a.type_down_r, 1, nbr);
+    default: return a.has_shared ? stream_max(a, a.shared.down.type, 1, nbs) : 0;
     }
 }
 
@@ -1325,57 +1463,75 @@ static hipError_t down_typed(const BatchArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int TY, bool SHARED, int S, bool TILE>
+// Workgroups of the shared expert's K-quant rows (kt_workgroup).
+static int kt_wgs(const BatchArgs &a, int rows) { return rows / 64 * kt_groups(a.n_tokens); }
+
+// KTY: the launch also holds the shared expert's K-quant gate and up / down.
+template <int TY, bool SHARED, bool TILE, int NM, int KTY = 0>
 static hipError_t mx_gate_up_launch(const BatchArgs &a, hipStream_t s) {
-    const int lds = mx_dyn_lds(2, S, a.hidden / 256), rows = S == 1 ? a.mx_rows_gu : 16 * MX_WAVES / S;
-    const hipError_t e = allow_lds(k_mx_gate_up<TY, SHARED, S, TILE>, lds);
-    if (e != hipSuccess) return e;
-    const int grid = (SHARED ? cdiv(a.n_tokens, a.tc) : a.max_chunks) * cdiv(SHARED ? a.ffn_s : a.ffn_r, rows);
-    hipLaunchKernelGGL((k_mx_gate_up<TY, SHARED, S, TILE>), dim3(grid), dim3(MX_THREADS), lds, s, a);
+    const int kt = KTY ? 2 * kt_wgs(a, a.ffn_s) : 0;
+    const int grid = (SHARED ? cdiv(a.n_tokens, a.tc) : a.max_chunks) * cdiv(SHARED ? a.ffn_s : a.ffn_r, a.mx_rows_gu) * (3 - NM);
+    hipLaunchKernelGGL((k_mx_gate_up<TY, SHARED, TILE, NM, KTY>), dim3(kt + grid), dim3(MX_THREADS), 0, s, a, kt);
     return hipGetLastError();
 }
 
-template <int TY, bool SHARED, int S, bool TILE>
+template <int TY, bool SHARED, bool TILE, int KTY = 0>
 static hipError_t mx_down_launch(const BatchArgs &a, hipStream_t s) {
-    const int nb = (SHARED ? a.ffn_s : a.ffn_r) / 256;
-    const int lds = mx_dyn_lds(1, S, nb), rows = S == 1 ? a.mx_rows_d : 16 * MX_WAVES / S;
-    const hipError_t e = allow_lds(k_mx_down<TY, SHARED, S, TILE>, lds);
-    if (e != hipSuccess) return e;
-    const int grid = (SHARED ? cdiv(a.n_tokens, a.tc) : a.max_chunks) * cdiv(a.hidden, rows);
-    hipLaunchKernelGGL((k_mx_down<TY, SHARED, S, TILE>), dim3(grid), dim3(MX_THREADS), lds, s, a);
+    const int kt = KTY ? kt_wgs(a, a.hidden) : 0;
+    const int grid = (SHARED ? cdiv(a.n_tokens, a.tc) : a.max_chunks) * cdiv(a.hidden, a.mx_rows_d);
+    hipLaunchKernelGGL((k_mx_down<TY, SHARED, TILE, KTY>), dim3(kt + grid), dim3(MX_THREADS), 0, s, a, kt);
     return hipGetLastError();
 }
 
 // One launch for the experts with tile copies, one for the others (a layer
-// with copies of some experts only needs both).
-template <int TY, bool SHARED, int S>
-static hipError_t mx_gate_up_split(const BatchArgs &a, hipStream_t s) {
-    hipError_t e = hipSuccess;
-    if (SHARED || a.mx_copies != 2) e = mx_gate_up_launch<TY, SHARED, S, false>(a, s);
-    if constexpr (!SHARED)
-        if (e == hipSuccess && a.mx_copies) e = mx_gate_up_launch<TY, SHARED, S, true>(a, s);
-    return e;
+// with copies of some experts only needs both); the shared expert's K-quant
+// rows go with the stage's first launch.
+template <int TY, bool SHARED>
+static hipError_t mx_gate_up_launches(const BatchArgs &a, hipStream_t s) {
+    if constexpr (SHARED) {
+        return mx_gate_up_launch<TY, true, false, 2>(a, s);
+    } else {
+        hipError_t e = hipSuccess;
+        bool kt = a.shared_kt;
+        if (a.mx_copies) {
+            e = kt ? mx_gate_up_launch<TY, false, true, 2, T_Q4_K>(a, s) : mx_gate_up_launch<TY, false, true, 2>(a, s);
+            kt = false;
+        }
+        if (e != hipSuccess || a.mx_copies == 2) return e;
+        // Row-major: with few workgroups gate and up apart fill the waves more
+        // evenly (step of 5 tokens of top-8: 112 against 120 us, 16 tokens 190
+        // against 196), with many the shared token loads count (64 tokens: 368
+        // against 356 us).
+        if ((long long)a.max_chunks * cdiv(a.ffn_r, a.mx_rows_gu) < 4096)
+            return kt ? mx_gate_up_launch<TY, false, false, 1, T_Q4_K>(a, s) : mx_gate_up_launch<TY, false, false, 1>(a, s);
+        return kt ? mx_gate_up_launch<TY, false, false, 2, T_Q4_K>(a, s) : mx_gate_up_launch<TY, false, false, 2>(a, s);
+    }
 }
 
-template <int TY, bool SHARED, int S>
-static hipError_t mx_down_split(const BatchArgs &a, hipStream_t s) {
-    hipError_t e = hipSuccess;
-    if (SHARED || a.mx_copies != 2) e = mx_down_launch<TY, SHARED, S, false>(a, s);
-    if constexpr (!SHARED)
-        if (e == hipSuccess && a.mx_copies) e = mx_down_launch<TY, SHARED, S, true>(a, s);
-    return e;
+template <int TY, bool SHARED>
+static hipError_t mx_down_launches(const BatchArgs &a, hipStream_t s) {
+    if constexpr (SHARED) {
+        return mx_down_launch<TY, true, false>(a, s);
+    } else {
+        hipError_t e = hipSuccess;
+        bool kt = a.shared_kt;
+        if (a.mx_copies) {
+            e = kt ? mx_down_launch<TY, false, true, T_Q5_K>(a, s) : mx_down_launch<TY, false, true>(a, s);
+            kt = false;
+        }
+        if (e == hipSuccess && a.mx_copies != 2)
+            e = kt ? mx_down_launch<TY, false, false, T_Q5_K>(a, s) : mx_down_launch<TY, false, false>(a, s);
+        return e;
+    }
 }
 
 // An IQ stream with the matrix cores on: the matrix-core launch when some
 // chunk can reach mx_min tokens, then the VALU launch when some chunk can stay
-// below it (each kernel returns early on the other's chunks).  mx_split_* is
-// the number of waves that share a 16-row tile (1, 2 or 4).
+// below it (each kernel returns early on the other's chunks).
 template <int TY, bool SHARED>
 static hipError_t mx_gate_up_typed(const BatchArgs &a, hipStream_t s_mx, hipStream_t s_valu) {
     if (a.mx_min <= a.tc) {
-        const hipError_t e = a.mx_split_gu == 4   ? mx_gate_up_split<TY, SHARED, 4>(a, s_mx)
-                             : a.mx_split_gu == 2 ? mx_gate_up_split<TY, SHARED, 2>(a, s_mx)
-                                                  : mx_gate_up_split<TY, SHARED, 1>(a, s_mx);
+        const hipError_t e = mx_gate_up_launches<TY, SHARED>(a, s_mx);
         if (e != hipSuccess) return e;
     }
     return a.mx_min > 1 ? gate_up_typed<TY, SHARED>(a, s_valu) : hipSuccess;
@@ -1384,9 +1540,7 @@ static hipError_t mx_gate_up_typed(const BatchArgs &a, hipStream_t s_mx, hipStre
 template <int TY, bool SHARED>
 static hipError_t mx_down_typed(const BatchArgs &a, hipStream_t s_mx, hipStream_t s_valu) {
     if (a.mx_min <= a.tc) {
-        const hipError_t e = a.mx_split_d == 4   ? mx_down_split<TY, SHARED, 4>(a, s_mx)
-                             : a.mx_split_d == 2 ? mx_down_split<TY, SHARED, 2>(a, s_mx)
-                                                 : mx_down_split<TY, SHARED, 1>(a, s_mx);
+        const hipError_t e = mx_down_launches<TY, SHARED>(a, s_mx);
         if (e != hipSuccess) return e;
     }
     return a.mx_min > 1 ? down_typed<TY, SHARED>(a, s_valu) : hipSuccess;
@@ -1440,7 +1594,10 @@ hipError_t launch_moe_batch(const BatchArgs &a, hipStream_t s, const BatchStream
     if ((e = hipGetLastError()) != hipSuccess) return e;
     // Stage 1 (gate/up) and stage 2 (down) each fork the side stream after the
     // main stream's last dependency and join it before the next dependent launch.
-    const bool two = streams && streams->side;
+    // With every chunk on the matrix cores a stage is one launch (two for an IQ
+    // shared expert or copies of some experts only) and stays on the main
+    // stream: a fork and join cost 10-20 us per stage.
+    const bool two = streams && streams->side && !(a.mx && a.mx_min <= 1);
     const hipStream_t s2 = two ? streams->side : s;
     auto fork = [&](int i) -> hipError_t {
         if (!two) return hipSuccess;
@@ -1452,45 +1609,35 @@ hipError_t launch_moe_batch(const BatchArgs &a, hipStream_t s, const BatchStream
         hipError_t r = hipEventRecord(streams->join[i], s2);
         return r == hipSuccess ? hipStreamWaitEvent(s, streams->join[i], 0) : r;
     };
+    // The shared expert's K-quant rows ride in the routed matrix-core launch;
+    // without one (every chunk on the VALU) they run in a launch of their own.
+    const bool mx_launch = a.mx && a.mx_min <= a.tc;
     if ((e = fork(0)) != hipSuccess) return e;
-    if (a.has_shared && a.shared_gemm) {
-        // shared gate/up on the matrix cores: they only need Q8_K(x)
-        GemmArgs gm{};
-        gm.b = a.bx;
-        gm.nb = nbh;
-        gm.n_tokens = a.n_tokens;
-        gm.shape = a.gemm_shape;
-        gm.n_mat = 2;
-        gm.mat[0] = a.sg;
-        gm.mat[1] = a.su;
-        if ((e = launch_prep_b(a.q8x, a.n_tokens, nbh, a.bx, s2)) != hipSuccess) return e;
-        if ((e = launch_kq_gemm(gm, s2)) != hipSuccess) return e;
-    } else if (a.has_shared && (e = gate_up_any<true>(tsg, a, s2, s2)) != hipSuccess) {
+    if (a.shared_kt && !mx_launch) {
+        const int n = kt_wgs(a, a.ffn_s);
+        hipLaunchKernelGGL(k_kt_rows<T_Q4_K>, dim3(2 * n), dim3(MX_THREADS), 0, s2, a.kt_w[0], a.kt_w[1], a.ffn_s, nbh,
+                           a.kt_x, a.n_tokens, a.g_s, a.u_s, n);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    } else if (a.has_shared && !a.shared_kt && (e = gate_up_any<true>(tsg, a, s2, s2)) != hipSuccess) {
         return e;
     }
     if ((e = gate_up_any<false>(a.type_gate_r, a, s2, s)) != hipSuccess) return e;
     if ((e = join(0)) != hipSuccess) return e;
 
     const bool rm = tsd == T_Q4_K || tsd == T_Q5_K;
-    const int mode = !a.has_shared ? 0 : a.shared_gemm ? 2 : rm ? 1 : 0;
+    const int mode = !a.has_shared ? 0 : a.shared_kt ? 2 : rm ? 1 : 0;
     const long long br = (long long)a.n_tokens * a.top_k * (a.ffn_r / 256);
     const long long bs = a.has_shared ? (long long)a.n_tokens * (a.ffn_s / 256) : 0;
     hipLaunchKernelGGL(k_mb_quant_h, dim3(cdiv(((br + 3) & ~3ll) + bs, 4 * MB_WAVES)), dim3(MB_THREADS), 0, s, a, mode);
     if ((e = hipGetLastError()) != hipSuccess) return e;
 
     if ((e = fork(1)) != hipSuccess) return e;
-    if (a.has_shared && a.shared_gemm) {
-        const int nbs = a.ffn_s / 256;
-        GemmArgs gm{};
-        gm.b = a.bh;
-        gm.nb = nbs;
-        gm.n_tokens = a.n_tokens;
-        gm.shape = a.gemm_shape;
-        gm.n_mat = 1;
-        gm.mat[0] = a.sd;
-        if ((e = launch_prep_b(a.q8h_s, a.n_tokens, nbs, a.bh, s2)) != hipSuccess) return e;
-        if ((e = launch_kq_gemm(gm, s2)) != hipSuccess) return e;
-    } else if (a.has_shared && (e = down_any<true>(tsd, a, s2, s2)) != hipSuccess) {
+    if (a.shared_kt && !mx_launch) {
+        const int n = kt_wgs(a, a.hidden);
+        hipLaunchKernelGGL(k_kt_rows<T_Q5_K>, dim3(n), dim3(MX_THREADS), 0, s2, a.kt_w[2], nullptr, a.hidden, a.ffn_s / 256,
+                           a.kt_h, a.n_tokens, a.d_s, nullptr, n);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    } else if (a.has_shared && !a.shared_kt && (e = down_any<true>(tsd, a, s2, s2)) != hipSuccess) {
         return e;
     }
     if ((e = down_any<false>(a.type_down_r, a, s2, s)) != hipSuccess) return e;
@@ -1500,6 +1647,22 @@ hipError_t launch_moe_batch(const BatchArgs &a, hipStream_t s, const BatchStream
     int g = cdiv(total, MB_THREADS);
     g = g > 4096 ? 4096 : g;
     hipLaunchKernelGGL(k_mb_combine, dim3(g), dim3(MB_THREADS), 0, s, a);
+    return hipGetLastError();
+}
+
+size_t kt_weight_bytes(int ty, int rows, int nb) { return kt_w_bytes(ty, rows, nb); }
+size_t kt_token_bytes(int n_tokens, int nb) { return kt_tok_bytes(n_tokens, nb); }
+
+hipError_t launch_kt_pack(const MatView &m, uint8_t *dst, hipStream_t s) {
+    if (m.rows % 16) return hipErrorInvalidValue;
+    int grid = cdiv(m.units * 4, 256);
+    grid = grid > 8192 ? 8192 : grid;
+    if (m.type == T_Q4_K)
+        hipLaunchKernelGGL(k_kt_pack<T_Q4_K>, dim3(grid), dim3(256), 0, s, m, dst);
+    else if (m.type == T_Q5_K)
+        hipLaunchKernelGGL(k_kt_pack<T_Q5_K>, dim3(grid), dim3(256), 0, s, m, dst);
+    else
+        return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

@@ -206,20 +206,21 @@ struct BatchArgs {
     int32_t rt_d_r, rt_d_s;     // VALU streams: down rows per workgroup (routed, shared)
     int32_t type_gate_r, type_down_r;
     // The shared expert's gate / up outputs (every stream type; SwiGLU is
-    // formed in the h quantization, as for the routed pairs); on the K-quant
-    // types its gate/up and down run on the matrix cores (-> d_s).
-    int32_t shared_gemm, gemm_shape;
-    MatGemm sg, su, sd;         // MFMA-ready copies of the shared gate / up / down
+    // formed in the h quantization, as for the routed pairs).  shared_kt: Q4_K
+    // gate and up and Q5_K down on the f16 matrix cores (lbh_kt.h), from tile
+    // copies of the three and operand tiles of x and of the shared h.
+    int32_t shared_kt;
+    int32_t valu;               // some routed chunk may run on the VALU streams (Q8_K rows needed)
     float *g_s, *u_s;           // [n_tokens][ffn_s]
-    uint8_t *bx, *bh;           // GEMM activation tiles of x and of the shared h
+    const uint8_t *kt_w[3];     // gate, up, down
+    uint8_t *kt_x, *kt_h;
     // mx = 1: chunks of at least mx_min tokens of the IQ2_S / IQ3_S streams run
-    // on the int8 matrix cores (mx_split_* waves share each 16-row tile; split 1:
-    // mx_rows_* rows per workgroup) and read the operand copies of the Q8_K rows
+    // on the int8 matrix cores (mx_rows_* rows per workgroup) and read the operand copies of the Q8_K rows
     // (quants at 256 bytes a block, scales apart) of x and of the routed and
     // shared h; the VALU streams take the smaller chunks and stage vc = min(tc,
     // mx_min - 1) tokens (tc when mx = 0).  mx_copies: tile copies of no routed
     // expert (0), some (1) or all (2).
-    int32_t mx, mx_min, mx_split_gu, mx_split_d, vc;
+    int32_t mx, mx_min, vc;
     int32_t mx_rows_gu, mx_rows_d, mx_copies;
     int32_t residual;           // y[t][r] += delta (as MoeArgs::residual)
     // The matrix-core streams' routed views [n_experts]: an expert's 16-row
@@ -244,6 +245,10 @@ struct RouteBatchArgs {
 size_t gemm_a_bytes(int rows, int nb);
 size_t gemm_b_bytes(int n_tokens, int nb);
 hipError_t launch_prep_a(const MatView &m, uint8_t *a, hipStream_t s);
+// Tile copy of a Q4_K / Q5_K matrix for the batched shared expert (lbh_kt.h; kt_w_bytes bytes).
+hipError_t launch_kt_pack(const MatView &m, uint8_t *dst, hipStream_t s);
+size_t kt_weight_bytes(int ty, int rows, int nb);
+size_t kt_token_bytes(int n_tokens, int nb);
 hipError_t launch_prep_b(const uint8_t *q8, int n_tokens, int nb, uint8_t *b, hipStream_t s);
 hipError_t launch_kq_gemm(const GemmArgs &g, hipStream_t s);
 

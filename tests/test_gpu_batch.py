@@ -243,3 +243,37 @@ def test_batch_config4_shapes_zipf_bit_exact(be, oracle):
         got = run_checked(be, layer, ids, coefs, xs)
         bad = [t for t in range(64) if not _same(got[t], want[t])]
         assert not bad, f"call {rep}: tokens {bad[:8]}"
+
+
+@pytest.mark.parametrize("hidden,ffn_s", [(256, 768), (768, 256), (1280, 512)])
+@pytest.mark.parametrize("engine", [None, 0])
+def test_shared_kquant_rows_at_the_edges(be, oracle, hidden, ffn_s, engine):
+    """The shared expert's Q4_K / Q5_K rows on the f16 matrix cores at 1, 2, 3
+    and 5 blocks a row and token counts about the 16-token tiles: scales,
+    minimums and quants at their extremes (63, 63, 15 / 31), of either sign of
+    d, and inputs that quantize to +-127 give the largest integer sums.  In the
+    routed experts' launch and (engine 0) in a launch of their own."""
+    def extreme(ty, rows, k):
+        b = synth.random_matrix(ty, rows, k, seed=rows + ty).reshape(-1, synth.BLOCK_BYTES[ty])
+        b[0::3, 4:], b[1::3, 4:] = 0xff, 0
+        b[0::2, 1] |= 0x80   # negative d
+        return b.reshape(rows, -1)
+
+    rng = np.random.default_rng(hidden + ffn_s)
+    tys, shp = (Q4_K, Q4_K, Q5_K), ((ffn_s, hidden), (ffn_s, hidden), (hidden, ffn_s))
+    ws = [extreme(t, r, k) for t, (r, k) in zip(tys, shp)]
+    layer = Layer(be, oracle, 2, hidden, 256, 256, (IQ2_S, IQ3_S, Q4_K, Q5_K), seed=191)
+    layer.orc_shared = oracle.make_expert(*(oracle.make_matrix(t, r, k, w) for t, (r, k), w in zip(tys, shp, ws)))
+    layer.moe = be.moe_create(layer._keep[0], tuple(be.upload(t, r, k, w) for t, (r, k), w in zip(tys, shp, ws)))
+    layer.moe.reserve_batch(33, 1)
+    if engine is not None:
+        layer.moe.set_batch_engine(engine)
+    for n in (1, 15, 16, 17, 33):
+        ids = (np.arange(n, dtype=np.uint32) % 2)[:, None]
+        coefs = rng.random((n, 1)).astype(np.float32)
+        xs = np.sign(rng.standard_normal((n, hidden))).astype(np.float32)
+        xs[1::2] *= rng.random((n // 2, hidden)).astype(np.float32)
+        want = oracle_batch(oracle, layer, ids, coefs, xs)
+        got = run_checked(be, layer, ids, coefs, xs)
+        bad = [t for t in range(n) if not np.array_equal(got[t], want[t], equal_nan=True)]
+        assert not bad, f"{n} tokens: {bad}"
