@@ -421,72 +421,93 @@ constexpr int mb_lpu() {
 
 // ------------------------------------------------------------------ kernels
 
-// Sort of the batch's pairs by expert (workgroup 0) and Q8_K of every token
-// (the other workgroups, four blocks per wave).
-__device__ __forceinline__ void quantize_rows_out(const float *x, long long nblocks, long long first, uint8_t *plain,
-                                                  uint8_t *rm, uint8_t *lds_wave, MxRows mx, uint8_t *kt, int nb) {
-    // Blocks [first, first + 4) (x points at block `first`) of rows of nb
-    // blocks into the wave's LDS, then out to global memory: (plain != NULL)
-    // the GGML bytes, (rm != NULL) the copy with residue-major qs, (mx.q !=
-    // NULL) the matrix-core operand copy, (kt != NULL) the f16 operand tiles of
-    // the K-quant rows (lbh_kt.h).
+// Q8_K of one block by one wave, lane l holding elements 4l .. 4l + 3 (v), in
+// the forms the consumers read: block `blk` of the GGML bytes (plain != NULL),
+// of the copy with residue-major qs (rm != NULL), of the matrix-core operand
+// copy (mx.q != NULL), and of the f16 operand tiles of the K-quant rows (kt !=
+// NULL, rows of nb blocks; lbh_kt.h).  lds: 292 bytes of the wave.
+//
+// These kernels are latency-bound: a block per wave with four elements a lane
+// and one coalesced dword a lane per copy took the 64-token (256-token) h
+// quantization from 13 (34) us, at four blocks per wave and 16 elements a lane
+// copied out of LDS, to 7 (16) us.
+__device__ __forceinline__ void quantize_block_out(const float4 v, long long blk, uint8_t *plain, uint8_t *rm, uint8_t *lds,
+                                                   MxRows mx, uint8_t *kt, int nb) {
     const int lane = threadIdx.x & 63;
-    const long long cnt = nblocks - first < 4 ? nblocks - first : 4;
-    quantize_blocks_wave(x, lds_wave, 0, cnt);
-    wave_sync();
+    const float e[4] = {v.x, v.y, v.z, v.w};
+    // the lane's largest |x| and the value at its first index, then the lowest
+    // lane holding the wave's (q8_k.rs:43-49: the first index on ties)
+    uint32_t am = __float_as_uint(fabsf(e[0]));
+    float mv = e[0];
+#pragma unroll
+    for (int i = 1; i < 4; ++i) {
+        const uint32_t b = __float_as_uint(fabsf(e[i]));
+        if (b > am) am = b, mv = e[i];
+    }
+    const uint32_t amax = wave_max_u32(am);
+    const int owner = (int)__builtin_ctzll(__ballot(am == amax));
+    const float maxv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mv), owner));
+    uint32_t q = 0;
+    int32_t sum = 0;
+    float d = 0.0f;
+    if (amax != 0) {
+        const float iscale = -127.0f / maxv;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            int32_t x = nearest_int(__fmul_rn(iscale, e[i]));
+            x = x < 127 ? x : 127;
+            q |= (uint32_t)(uint8_t)(int8_t)x << (8 * i);
+            sum += (int8_t)x;
+        }
+        d = 1.0f / iscale;
+    }
+    // bsums of 16 elements (four lanes), and the next group's
+    sum += (int32_t)dpp_row<0xB1>((uint32_t)sum);
+    sum += (int32_t)dpp_row<0x4E>((uint32_t)sum);
+    const int32_t after = __builtin_amdgcn_update_dpp(0, sum, 0x104, 0xf, 0xf, false);   // row_shl:4
+    const uint32_t pair = (uint32_t)(uint16_t)(int16_t)sum | ((uint32_t)(uint16_t)(int16_t)after << 16);
     if (mx.q) {
-        for (int k = lane; k < (int)cnt * 64; k += 64) {
-            const int blk = k >> 6, w = k & 63;
-            // w: destination dword, from source dword sw
-            const int p = (w >> 2) & 3, o = 4 * (w >> 4) + (w & 3);   // quarter p, its dword o
-            const int sw = mx.split ? 8 * (o >> 1) + 2 * p + (o & 1) : 16 * p + o;
-            reinterpret_cast<uint32_t *>(mx.q)[(first + blk) * 64 + w] =
-                *reinterpret_cast<const uint32_t *>(lds_wave + blk * 292 + 4 + 4 * sw);
-        }
-        if (lane < cnt) mx.d[first + lane] = *reinterpret_cast<const float *>(lds_wave + lane * 292);
+        // element dword `lane` as dword o of lane quarter p (MxRows)
+        const int p = mx.split ? (lane >> 1) & 3 : lane >> 4, o = mx.split ? 2 * (lane >> 3) + (lane & 1) : lane & 15;
+        reinterpret_cast<uint32_t *>(mx.q)[blk * 64 + 16 * (o >> 2) + 4 * p + (o & 3)] = q;
+        if (lane == 0) mx.d[blk] = d;
     }
-    if (kt) {
-        for (int k = lane; k < (int)cnt * KT_STORE_PIECES; k += 64) {
-            const int blk = k / KT_STORE_PIECES;
-            const long long g = first + blk, t = g / nb;
-            kt_store_piece(kt, t, (int)(g - t * nb), nb, lds_wave + blk * 292, k - blk * KT_STORE_PIECES);
-        }
-    }
-    if (!plain && !rm) {
-        wave_sync();
-        return;
-    }
-    const int dw = (int)cnt * 73;
-    for (int k = lane; k < dw; k += 64) {
-        const int blk = k / 73, w = k - blk * 73;
-        const uint8_t *sb = lds_wave + blk * 292;
-        const uint32_t v = *reinterpret_cast<const uint32_t *>(sb + 4 * w);
-        if (plain) *reinterpret_cast<uint32_t *>(plain + (first + blk) * 292 + 4 * w) = v;
-        if (rm) {
-            uint32_t r = v;
-            if (w >= 1 && w <= 64) {
-                const int q = w - 1, g = q >> 3, t = q & 7;
-                const uint8_t *src = sb + 4 + 32 * g + t;
-                r = (uint32_t)src[0] | ((uint32_t)src[8] << 8) | ((uint32_t)src[16] << 16) | ((uint32_t)src[24] << 24);
-            }
-            *reinterpret_cast<uint32_t *>(rm + (first + blk) * 292 + 4 * w) = r;
-        }
-    }
+    auto store = [&](uint8_t *b) {
+        uint32_t *o = reinterpret_cast<uint32_t *>(b);
+        if (lane == 0) o[0] = __float_as_uint(d);
+        o[1 + lane] = q;
+        if ((lane & 7) == 0) o[65 + (lane >> 3)] = pair;
+    };
+    if (plain) store(plain + blk * 292);
+    if (!kt && !rm) return;
+    store(lds);
     wave_sync();
+    if (kt && lane < KT_STORE_PIECES) {
+        const long long t = blk / nb;
+        kt_store_piece(kt, t, (int)(blk - t * nb), nb, lds, lane);
+    }
+    if (rm) {
+        uint32_t *o = reinterpret_cast<uint32_t *>(rm + blk * 292);
+        const uint8_t *src = lds + 4 + 32 * (lane >> 3) + (lane & 7);
+        o[1 + lane] = (uint32_t)src[0] | ((uint32_t)src[8] << 8) | ((uint32_t)src[16] << 16) | ((uint32_t)src[24] << 24);
+        if (lane == 0) o[0] = __float_as_uint(d);
+        if ((lane & 7) == 0) o[65 + (lane >> 3)] = pair;
+    }
 }
 
+// Sort of the batch's pairs by expert (workgroup 0) and Q8_K of every token
+// (the other workgroups, a block per wave).
 __global__ void __launch_bounds__(MB_THREADS) k_mb_prep(BatchArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x;
     if (blockIdx.x > 0) {
         const int nb = a.hidden / 256;
-        const long long nblocks = (long long)a.n_tokens * nb;
-        const long long first = ((long long)(blockIdx.x - 1) * MB_WAVES + (tid >> 6)) * 4;
+        const long long blk = (long long)(blockIdx.x - 1) * MB_WAVES + (tid >> 6);
+        if (blk >= (long long)a.n_tokens * nb) return;
         const bool rm = a.has_shared && !a.shared_kt && (a.shared.gate.type == T_Q4_K || a.shared.gate.type == T_Q5_K);
-        if (first < nblocks)
-            quantize_rows_out(a.x + first * 256, nblocks, first, a.valu ? a.q8x : nullptr, rm ? a.q8x_rm : nullptr,
-                              smem + (tid >> 6) * 4 * 292, MxRows{a.mx ? a.xq_mx : nullptr, a.xd_mx, false},
-                              a.shared_kt ? a.kt_x : nullptr, nb);
+        const float4 v = reinterpret_cast<const float4 *>(a.x + blk * 256)[tid & 63];
+        quantize_block_out(v, blk, a.valu ? a.q8x : nullptr, rm ? a.q8x_rm : nullptr, smem + (tid >> 6) * 304,
+                           MxRows{a.mx ? a.xq_mx : nullptr, a.xd_mx, false}, a.shared_kt ? a.kt_x : nullptr, nb);
         return;
     }
     const int NE = a.n_experts, T = a.n_tokens, K = a.top_k, TC = a.tc;
@@ -495,14 +516,22 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_prep(BatchArgs a) {
     int32_t *cnt = reinterpret_cast<int32_t *>(bm + NE * W);       // [NE]
     int32_t *off = cnt + NE;                                       // [NE] first sorted pair
     int32_t *coff = off + NE;                                      // [NE] first chunk
-    int32_t *part = coff + NE;                                     // [2][MB_THREADS] scan partials
-    int32_t *flags = part + 2 * MB_THREADS;
+    int32_t *part = coff + NE;                                     // [MB_WAVES] scan partials
+    int32_t *flags = part + MB_WAVES;
+    // the thread's pairs tid, tid + 256, ..: every load in flight at once
+    constexpr int PAIRS = BATCH_MAX_TOKENS * MOE_MAX_ROUTED / MB_THREADS;
+    uint32_t ids[PAIRS];
+#pragma unroll
+    for (int i = 0; i < PAIRS; ++i) ids[i] = i * MB_THREADS + tid < T * K ? a.ids[i * MB_THREADS + tid] : 0u;
     for (int i = tid; i < NE * W; i += MB_THREADS) bm[i] = 0;
     if (tid == 0) flags[0] = 0;
     __syncthreads();
-    for (int p = tid; p < T * K; p += MB_THREADS) {
+#pragma unroll
+    for (int i = 0; i < PAIRS; ++i) {
+        const int p = i * MB_THREADS + tid;
+        if (p >= T * K) break;
         const int t = p / K;
-        const uint32_t e = a.ids[p];
+        const uint32_t e = ids[i];
         if (e >= (uint32_t)NE) {
             atomicOr(&flags[0], 1);
             continue;
@@ -523,20 +552,24 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_prep(BatchArgs a) {
         sc += c;
         sk += (c + TC - 1) / TC;
     }
-    part[tid] = sc;
-    part[MB_THREADS + tid] = sk;
+    // Exclusive scan of (pairs, chunks), both at most 4096, as one word.
+    static_assert(BATCH_MAX_TOKENS * MOE_MAX_ROUTED < 0x8000, "two sums share a word");
+    uint32_t sum = (uint32_t)sc << 16 | (uint32_t)sk;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)sum, d, 64);
+        if ((tid & 63) >= d) sum += o;
+    }
+    if ((tid & 63) == 63) part[tid >> 6] = (int32_t)sum;
     __syncthreads();
-    // Inclusive scan of the partials (Hillis-Steele), then exclusive offsets.
-    for (int d = 1; d < MB_THREADS; d <<= 1) {
-        const int v0 = tid >= d ? part[tid - d] : 0;
-        const int v1 = tid >= d ? part[MB_THREADS + tid - d] : 0;
-        __syncthreads();
-        part[tid] += v0;
-        part[MB_THREADS + tid] += v1;
-        __syncthreads();
+    uint32_t before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < MB_WAVES; ++w) {
+        if (w < tid >> 6) before += (uint32_t)part[w];
+        total += (uint32_t)part[w];
     }
     {
-        int o = part[tid] - sc, ko = part[MB_THREADS + tid] - sk;
+        const uint32_t at = before + sum - ((uint32_t)sc << 16 | (uint32_t)sk);
+        int o = (int)(at >> 16), ko = (int)(at & 0xffffu);
         for (int e = e0; e < e1; ++e) {
             off[e] = o;
             coff[e] = ko;
@@ -547,9 +580,12 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_prep(BatchArgs a) {
     __syncthreads();
     const bool bad = flags[0] != 0;
     if (!bad) {
-        for (int p = tid; p < T * K; p += MB_THREADS) {
+#pragma unroll
+        for (int i = 0; i < PAIRS; ++i) {
+            const int p = i * MB_THREADS + tid;
+            if (p >= T * K) break;
             const int t = p / K;
-            const uint32_t e = a.ids[p];
+            const uint32_t e = ids[i];
             int rank = __popc(bm[e * W + (t >> 5)] & ((1u << (t & 31)) - 1u));
             for (int w = 0; w < (t >> 5); ++w) rank += __popc(bm[e * W + w]);
             const int pos = off[e] + rank;
@@ -567,7 +603,7 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_prep(BatchArgs a) {
         }
     }
     if (tid == 0) {
-        a.plan[0] = bad ? 0 : part[2 * MB_THREADS - 1];
+        a.plan[0] = bad ? 0 : (int32_t)(total & 0xffffu);
         a.plan[1] = flags[0];
     }
 }
@@ -652,39 +688,32 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_gate_up(BatchArgs a) {
 // bytes plus the matrix-core operand copy (IQ down); 1: residue-major qs only
 // (VALU K-quant down); 2: the f16 operand tiles (matrix-core K-quant down).
 __global__ void __launch_bounds__(MB_THREADS) k_mb_quant_h(BatchArgs a, int shared_mode) {
-    __shared__ __align__(16) uint8_t lds[MB_WAVES * 4 * 292];
-    __shared__ __align__(16) float hbuf[MB_WAVES][4 * 256];
-    if (a.plan[1]) return;
+    __shared__ __align__(16) uint8_t lds[MB_WAVES][304];
+    __shared__ uint64_t exp_tab[32];
+    if (threadIdx.x < 32) exp_tab[threadIdx.x] = c_expf_tab[threadIdx.x];
     const int nbr = a.ffn_r / 256, nbs = a.ffn_s / 256;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const long long br = (long long)a.n_tokens * a.top_k * nbr;
-    const long long brp = (br + 3) & ~3ll;   // chunks of four never straddle the two ranges
     const long long bs = a.has_shared ? (long long)a.n_tokens * nbs : 0;
-    const long long chunk = ((long long)blockIdx.x * MB_WAVES + wid) * 4;
-    uint8_t *lw = lds + wid * 4 * 292;
-    // Lane (block first + lane / 16, elements 16 (lane % 16) ..) forms the
-    // sixteen values it quantizes below.
-    auto swiglu_blocks = [&](const float *g, const float *u, long long first, long long nblocks) {
-        const long long blk = first + (lane >> 4);
-        if (blk < nblocks) {
-            const long long base = blk * 256 + 16 * (lane & 15);
-            float *hb = &hbuf[wid][(lane >> 4) * 256 + 16 * (lane & 15)];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) hb[i] = swiglu_ref(g[base + i], u[base + i]);
-        }
-        wave_sync();
-    };
-    if (chunk < br) {
-        swiglu_blocks(a.g_r, a.u_r, chunk, br);
-        quantize_rows_out(&hbuf[wid][0], br, chunk, a.valu ? a.q8h_r : nullptr, nullptr, lw,
-                          MxRows{a.mx ? a.hq_mx_r : nullptr, a.hd_mx_r, a.type_down_r == T_IQ3_S}, nullptr, nbr);
-    } else if (chunk >= brp && chunk - brp < bs) {
-        const long long f = chunk - brp;
-        swiglu_blocks(a.g_s, a.u_s, f, bs);
-        quantize_rows_out(&hbuf[wid][0], bs, f, shared_mode == 0 ? a.q8h_s : nullptr, shared_mode == 1 ? a.q8h_s : nullptr,
-                          lw, MxRows{a.mx && shared_mode == 0 ? a.hq_mx_s : nullptr, a.hd_mx_s, a.shared.down.type == T_IQ3_S},
-                          shared_mode == 2 ? a.kt_h : nullptr, nbs);
+    long long blk = (long long)blockIdx.x * MB_WAVES + wid;   // routed blocks, then the shared ones
+    const bool routed = blk < br, on = blk < br + bs;
+    if (!routed) blk -= br;
+    float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f), u = g;
+    if (on) {
+        g = reinterpret_cast<const float4 *>((routed ? a.g_r : a.g_s) + blk * 256)[lane];
+        u = reinterpret_cast<const float4 *>((routed ? a.u_r : a.u_s) + blk * 256)[lane];
     }
+    __syncthreads();
+    if (!on || a.plan[1]) return;
+    const float4 h = make_float4(swiglu_ref(g.x, u.x, exp_tab), swiglu_ref(g.y, u.y, exp_tab),
+                                 swiglu_ref(g.z, u.z, exp_tab), swiglu_ref(g.w, u.w, exp_tab));
+    if (routed)
+        quantize_block_out(h, blk, a.valu ? a.q8h_r : nullptr, nullptr, lds[wid],
+                           MxRows{a.mx ? a.hq_mx_r : nullptr, a.hd_mx_r, a.type_down_r == T_IQ3_S}, nullptr, nbr);
+    else
+        quantize_block_out(h, blk, shared_mode == 0 ? a.q8h_s : nullptr, shared_mode == 1 ? a.q8h_s : nullptr, lds[wid],
+                           MxRows{a.mx && shared_mode == 0 ? a.hq_mx_s : nullptr, a.hd_mx_s, a.shared.down.type == T_IQ3_S},
+                           shared_mode == 2 ? a.kt_h : nullptr, nbs);
 }
 
 // Down rows -> d, one launch per stream (as k_mb_gate_up; PART 1: every
@@ -1333,20 +1362,41 @@ __global__ void __launch_bounds__(MX_THREADS) k_kt_rows(const uint8_t *w0, const
 
 // Ordered combine of one token's routed outputs in its slot (ascending id)
 // order, then the shared expert at 1.0 (moe.rs:141-146).
+// Workgroup (1024 rows, token): the token's pairs are scalar reads, and the
+// rows of eight experts are in flight at once (64 / 256 tokens: 9.0 / 20 -> 5.0 /
+// 9.0 us against one row a thread with each expert's loads behind the last's).
 __global__ void __launch_bounds__(MB_THREADS) k_mb_combine(BatchArgs a) {
     if (a.plan[1]) return;
-    const long long total = (long long)a.n_tokens * a.hidden;
-    for (long long k = (long long)blockIdx.x * MB_THREADS + threadIdx.x; k < total;
-         k += (long long)gridDim.x * MB_THREADS) {
-        const int t = (int)(k / a.hidden), r = (int)(k - (long long)t * a.hidden);
-        float acc = 0.0f;
-        for (int s = 0; s < a.top_k; ++s) {
-            const int p = a.pair_of[t * a.top_k + s];
-            acc = __fadd_rn(acc, __fmul_rn(a.coefs[t * a.top_k + s], a.d_r[(long long)p * a.hidden + r]));
-        }
-        if (a.has_shared) acc = __fadd_rn(acc, __fmul_rn(1.0f, a.d_s[(long long)t * a.hidden + r]));
-        a.y[k] = a.residual ? __fadd_rn(a.y[k], acc) : acc;
+    const int t = blockIdx.y, r = (int)(blockIdx.x * MB_THREADS + threadIdx.x) * 4;
+    if (r >= a.hidden) return;
+    const long long at = (long long)t * a.hidden + r;
+    float4 sh = make_float4(0.0f, 0.0f, 0.0f, 0.0f), y = sh, acc = sh;
+    if (a.has_shared) sh = *reinterpret_cast<const float4 *>(a.d_s + at);
+    if (a.residual) y = *reinterpret_cast<const float4 *>(a.y + at);
+    for (int s0 = 0; s0 < a.top_k; s0 += 8) {
+        float4 d[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            if (s0 + s < a.top_k)
+                d[s] = *reinterpret_cast<const float4 *>(a.d_r + (long long)a.pair_of[t * a.top_k + s0 + s] * a.hidden + r);
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            if (s0 + s < a.top_k) {
+                const float c = a.coefs[t * a.top_k + s0 + s];
+                acc.x = __fadd_rn(acc.x, __fmul_rn(c, d[s].x));
+                acc.y = __fadd_rn(acc.y, __fmul_rn(c, d[s].y));
+                acc.z = __fadd_rn(acc.z, __fmul_rn(c, d[s].z));
+                acc.w = __fadd_rn(acc.w, __fmul_rn(c, d[s].w));
+            }
     }
+    if (a.has_shared) {
+        acc.x = __fadd_rn(acc.x, __fmul_rn(1.0f, sh.x));
+        acc.y = __fadd_rn(acc.y, __fmul_rn(1.0f, sh.y));
+        acc.z = __fadd_rn(acc.z, __fmul_rn(1.0f, sh.z));
+        acc.w = __fadd_rn(acc.w, __fmul_rn(1.0f, sh.w));
+    }
+    if (a.residual) acc = make_float4(__fadd_rn(y.x, acc.x), __fadd_rn(y.y, acc.y), __fadd_rn(y.z, acc.z), __fadd_rn(y.w, acc.w));
+    *reinterpret_cast<float4 *>(a.y + at) = acc;
 }
 
 // Top-k selection of every token of a batch from finished logits, one wave per token.
@@ -1398,8 +1448,8 @@ int batch_lds_bytes(const BatchArgs &a, int stage) {
     switch (stage) {
     case 0: {
         const int W = (a.n_tokens + 31) / 32;
-        const int sort = (a.n_experts * W + 3 * a.n_experts + 2 * MB_THREADS + 4) * 4;
-        return sort > MB_WAVES * 4 * 292 ? sort : MB_WAVES * 4 * 292;
+        const int sort = (a.n_experts * W + 3 * a.n_experts + MB_WAVES + 4) * 4;
+        return sort > MB_WAVES * 304 ? sort : MB_WAVES * 304;
     }
     case 1: return stream_max(a, a.type_gate_r, 2, nbh);
     case 2: return a.has_shared ? stream_max(a, a.shared.gate.type, 2, nbh) : 0;
@@ -1589,7 +1639,7 @@ hipError_t launch_moe_batch(const BatchArgs &a, hipStream_t s, const BatchStream
     const int nbh = a.hidden / 256;
     hipError_t e = allow_lds(k_mb_prep, lds[0]);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_mb_prep, dim3(1 + cdiv((long long)a.n_tokens * nbh, 4 * MB_WAVES)), dim3(MB_THREADS), lds[0],
+    hipLaunchKernelGGL(k_mb_prep, dim3(1 + cdiv((long long)a.n_tokens * nbh, MB_WAVES)), dim3(MB_THREADS), lds[0],
                        s, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     // Stage 1 (gate/up) and stage 2 (down) each fork the side stream after the
@@ -1628,7 +1678,7 @@ hipError_t launch_moe_batch(const BatchArgs &a, hipStream_t s, const BatchStream
     const int mode = !a.has_shared ? 0 : a.shared_kt ? 2 : rm ? 1 : 0;
     const long long br = (long long)a.n_tokens * a.top_k * (a.ffn_r / 256);
     const long long bs = a.has_shared ? (long long)a.n_tokens * (a.ffn_s / 256) : 0;
-    hipLaunchKernelGGL(k_mb_quant_h, dim3(cdiv(((br + 3) & ~3ll) + bs, 4 * MB_WAVES)), dim3(MB_THREADS), 0, s, a, mode);
+    hipLaunchKernelGGL(k_mb_quant_h, dim3(cdiv(br + bs, MB_WAVES)), dim3(MB_THREADS), 0, s, a, mode);
     if ((e = hipGetLastError()) != hipSuccess) return e;
 
     if ((e = fork(1)) != hipSuccess) return e;
@@ -1643,10 +1693,7 @@ hipError_t launch_moe_batch(const BatchArgs &a, hipStream_t s, const BatchStream
     if ((e = down_any<false>(a.type_down_r, a, s2, s)) != hipSuccess) return e;
     if ((e = join(1)) != hipSuccess) return e;
 
-    const long long total = (long long)a.n_tokens * a.hidden;
-    int g = cdiv(total, MB_THREADS);
-    g = g > 4096 ? 4096 : g;
-    hipLaunchKernelGGL(k_mb_combine, dim3(g), dim3(MB_THREADS), 0, s, a);
+    hipLaunchKernelGGL(k_mb_combine, dim3(cdiv(a.hidden, 4 * MB_THREADS), a.n_tokens), dim3(MB_THREADS), 0, s, a);
     return hipGetLastError();
 }
 

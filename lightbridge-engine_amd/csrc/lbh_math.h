@@ -35,7 +35,8 @@ namespace lbh {
 static __constant__ uint64_t c_expf_tab[32] = {LBH_EXPF_TABLE};
 static const uint64_t h_expf_tab[32] = {LBH_EXPF_TABLE};
 
-__host__ __device__ inline float expf_libm(float x) {
+// tab (device): the table, e.g. a copy in LDS.
+__host__ __device__ inline float expf_libm(float x, const uint64_t *tab = nullptr) {
     constexpr double N = 32.0;
     constexpr double INV_LN2_N = 0x1.71547652b82fep+0 * N;
     constexpr double SHIFT = 0x1.8p+52;
@@ -56,7 +57,7 @@ __host__ __device__ inline float expf_libm(float x) {
     kd -= SHIFT;
     const double r = fma(INV_LN2_N, xd, -kd);
 #ifdef __HIP_DEVICE_COMPILE__
-    const uint64_t t = c_expf_tab[ki % 32] + (ki << 47);
+    const uint64_t t = (tab ? tab[ki % 32] : c_expf_tab[ki % 32]) + (ki << 47);
 #else
     const uint64_t t = h_expf_tab[ki % 32] + (ki << 47);
 #endif
@@ -71,8 +72,8 @@ __host__ __device__ inline float expf_libm(float x) {
 
 // apply_swiglu's element (activation.rs:170-178): gate / (1 + exp(-gate)) * up,
 // each step separately rounded.
-__host__ __device__ inline float swiglu_ref(float gate, float up) {
-    const float e = expf_libm(-gate);
+__host__ __device__ inline float swiglu_ref(float gate, float up, const uint64_t *tab = nullptr) {
+    const float e = expf_libm(-gate, tab);
     const float act = gate / (1.0f + e);
     return act * up;
 }
