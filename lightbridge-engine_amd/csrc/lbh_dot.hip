@@ -138,64 +138,107 @@ struct DequantArgs {
     const DevStatus *status;   // skip every write when the input scan found a non-finite lane
 };
 
-// The 32 products w * x of group `sub` (32 consecutive elements) of unit u.
+// The bytes of group `sub` (32 consecutive elements) of unit u, loaded apart
+// from their use so that the next step's are in flight.
+template <int TY>
+struct DqRaw {   // K-quants
+    uint4 hdr, q[2], h[TY == T_Q5_K ? 2 : 1];
+};
+template <>
+struct DqRaw<T_IQ2_S> {
+    uint32_t d, qs, sg, qh, sc;
+};
+template <>
+struct DqRaw<T_IQ3_S> {
+    uint32_t d, sg, qh, ps;
+    uint2 qs;
+};
+template <int TY>
+__device__ __forceinline__ DqRaw<TY> dequant_load(const Planes &P, uint32_t u, int sub) {
+    DqRaw<TY> o;
+    if constexpr (TY == T_Q4_K || TY == T_Q5_K) {
+        constexpr int QS0 = TY == T_Q5_K ? 3 : 1;
+        const int g = sub >> 1;
+        o.hdr = bld128(P, u * 16, 0);
+        o.q[0] = bld128(P, u * 16 + (uint32_t)(2 * g) * P.U16, QS0 * P.U16);
+        o.q[1] = bld128(P, u * 16 + (uint32_t)(2 * g) * P.U16, (QS0 + 1) * P.U16);
+        if constexpr (TY == T_Q5_K) o.h[0] = bld128(P, u * 16, P.U16), o.h[1] = bld128(P, u * 16, 2 * P.U16);
+    } else if constexpr (TY == T_IQ2_S) {
+        // device encoding (lbh_layout.h): rotated qs bytes, the qh dword of
+        // groups 4 (sub / 4) .. + 3, bit-sliced sign dword
+        const uint32_t po = (uint32_t)(sub >> 2) * P.U16;
+        o.d = bld16(P, u * 2, 5 * P.U16);
+        o.qs = bld32(P, u * 16 + 4 * (sub & 3) + po, 0);
+        o.sg = bld32(P, u * 16 + 4 * (sub & 3) + po, 2 * P.U16);
+        o.qh = bld32(P, u * 16 + 4 * (sub >> 2), 4 * P.U16);
+        o.sc = bld8(P, u * 16 + 8 + sub, 4 * P.U16);
+    } else {
+        const uint32_t tail_base = 6 * P.U16;
+        o.d = bld16(P, u * 2, 6 * P.U16 + 12 * P.U);
+        o.qs = bld64(P, u * 16 + 8 * (sub & 1) + (uint32_t)(sub >> 1) * P.U16, 0);
+        o.sg = bld32(P, u * 16 + 4 * (sub & 3) + (uint32_t)(sub >> 2) * P.U16, 4 * P.U16);
+        o.qh = bld8(P, u * 12 + sub, tail_base);
+        o.ps = bld8(P, u * 12 + 8 + (sub >> 1), tail_base);
+    }
+    return o;
+}
+
+// The 32 products w * x of the group.
 // Decode formulas and their f32 operation order: k_quants.rs:242-300 (K-quants,
 // sub-block j = sub), iq2_s.rs:9-39 and iq3_s.rs:9-53 (group g = sub).
 template <int TY>
-__device__ __forceinline__ void dequant_group(const Planes &P, uint32_t u, int sub, const float *x, float *out) {
+__device__ __forceinline__ void dequant_group(const DqRaw<TY> &o, int sub, const void *grid_lds, const float *x, float *out) {
+    // w with its sign bit flipped where bit b of s is set: w * -1.0 exactly
+    auto flip = [](float w, uint32_t s, int b) {
+        return __uint_as_float(__float_as_uint(w) ^ ((s << (31 - b)) & 0x80000000u));
+    };
     if constexpr (TY == T_Q4_K || TY == T_Q5_K) {
-        constexpr int QS0 = TY == T_Q5_K ? 3 : 1;
-        const uint4 hdr = bld128(P, u * 16, 0);
-        const int g = sub >> 1, hi = sub & 1;
-        const uint4 q0 = bld128(P, u * 16, (QS0 + 2 * g) * P.U16), q1 = bld128(P, u * 16, (QS0 + 2 * g + 1) * P.U16);
-        const uint32_t q[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+        const uint4 hdr = o.hdr;
+        const int hi = sub & 1;
+        const uint32_t q[8] = {o.q[0].x, o.q[0].y, o.q[0].z, o.q[0].w, o.q[1].x, o.q[1].y, o.q[1].z, o.q[1].w};
         uint32_t h[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         if constexpr (TY == T_Q5_K) {
-            const uint4 h0 = bld128(P, u * 16, P.U16), h1 = bld128(P, u * 16, 2 * P.U16);
+            const uint4 h0 = o.h[0], h1 = o.h[1];
             h[0] = h0.x, h[1] = h0.y, h[2] = h0.z, h[3] = h0.w, h[4] = h1.x, h[5] = h1.y, h[6] = h1.z, h[7] = h1.w;
         }
         int32_t sc, mn;
         scale_min_of(hdr.y, hdr.z, hdr.w, sub, sc, mn);
         const float d1 = __fmul_rn(f16_to_f32(hdr.x & 0xffffu), (float)sc);
         const float m1 = __fmul_rn(f16_to_f32(hdr.x >> 16), (float)mn);
+        // element l of the group's 32 bytes sits in residue-major dword l % 8, byte l / 8
+        uint32_t v[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            v[t] = (q[t] >> (4 * hi)) & 0x0f0f0f0fu;
+            if constexpr (TY == T_Q5_K) v[t] |= ((h[t] >> sub) & 0x01010101u) << 4;
+        }
 #pragma unroll
         for (int l = 0; l < 32; ++l) {
-            // element l of the group's 32 bytes sits in residue-major dword l % 8, byte l / 8
-            uint32_t qv = (byte_of(q[l % 8], l / 8) >> (4 * hi)) & 15u;
-            if constexpr (TY == T_Q5_K) qv += ((byte_of(h[l % 8], l / 8) >> sub) & 1u) * 16u;
-            const float w = __fsub_rn(__fmul_rn(d1, (float)qv), m1);
+            const float w = __fsub_rn(__fmul_rn(d1, (float)byte_of(v[l % 8], l / 8)), m1);
             out[l] = __fmul_rn(w, x[l]);
         }
     } else if constexpr (TY == T_IQ2_S) {
-        const float d = f16_to_f32(bld16(P, u * 2, 5 * P.U16));
-        // device encoding (lbh_layout.h): rotated qs bytes, the qh dword of
-        // groups 4 (sub / 4) .. + 3, bit-sliced sign dword
-        const uint32_t qs = bld32(P, u * 16 + 4 * (sub & 3), (sub >> 2) * P.U16);
-        const uint32_t sg = bld32(P, u * 16 + 4 * (sub & 3), (2 + (sub >> 2)) * P.U16);
-        const uint32_t qh = bld32(P, u * 16 + 4 * (sub >> 2), 4 * P.U16);
-        const uint32_t sc = bld8(P, u * 16 + 8 + sub, 4 * P.U16);
+        const float d = f16_to_f32(o.d);
+        const uint32_t qs = o.qs, sg = o.sg, qh = o.qh, sc = o.sc;
         const float bs[2] = {__fmul_rn(__fmul_rn(d, __fadd_rn(0.5f, (float)(sc & 15u))), 0.25f),
                              __fmul_rn(__fmul_rn(d, __fadd_rn(0.5f, (float)(sc >> 4))), 0.25f)};
 #pragma unroll
         for (int lg = 0; lg < 4; ++lg) {
             const uint32_t h = (byte_of(qh, lg) >> (2 * (sub & 3))) & 3u;
             const uint32_t idx = iq2s_unrot_q(byte_of(qs, lg)) | (h << 8);
-            const uint64_t grid = c_iq2s_grid[idx];
+            const uint2 grid = static_cast<const uint2 *>(grid_lds)[idx];
 #pragma unroll
             for (int l = 0; l < 8; ++l) {
                 // weight 8 lg + l of the group: bit 2 lg + l / 4 of sign byte l % 4
-                const float sign = (byte_of(sg, l & 3) >> (2 * lg + (l >> 2))) & 1u ? -1.0f : 1.0f;
-                const float w = __fmul_rn(__fmul_rn(bs[lg >> 1], (float)((grid >> (8 * l)) & 0xffu)), sign);
+                const float w = flip(__fmul_rn(bs[lg >> 1], (float)byte_of(l < 4 ? grid.x : grid.y, l & 3)), sg,
+                                     8 * (l & 3) + 2 * lg + (l >> 2));
                 out[8 * lg + l] = __fmul_rn(w, x[8 * lg + l]);
             }
         }
     } else {  // IQ3_S
-        const uint32_t tail_base = 6 * P.U16;
-        const float d = f16_to_f32(bld16(P, u * 2, 6 * P.U16 + 12 * P.U));
-        const uint2 qs = bld64(P, u * 16 + 8 * (sub & 1), (sub >> 1) * P.U16);
-        const uint32_t sg = bld32(P, u * 16 + 4 * (sub & 3), (4 + (sub >> 2)) * P.U16);
-        const uint32_t qh = bld8(P, u * 12 + sub, tail_base);
-        const uint32_t ps = bld8(P, u * 12 + 8 + (sub >> 1), tail_base);
+        const float d = f16_to_f32(o.d);
+        const uint2 qs = o.qs;
+        const uint32_t sg = o.sg, qh = o.qh, ps = o.ps;
         const float sc = __fmul_rn(d, (float)(1u + 2u * ((ps >> (4 * (sub & 1))) & 15u)));
 #pragma unroll
         for (int lg = 0; lg < 4; ++lg) {
@@ -203,14 +246,11 @@ __device__ __forceinline__ void dequant_group(const Planes &P, uint32_t u, int s
             const int sh = 16 * (lg & 1);
             const uint32_t i1 = ((qq >> sh) & 0xffu) | ((qh << (8 - 2 * lg)) & 0x100u);
             const uint32_t i2 = ((qq >> (sh + 8)) & 0xffu) | ((qh << (7 - 2 * lg)) & 0x100u);
-            const uint32_t g1 = c_iq3s_grid[i1], g2 = c_iq3s_grid[i2];
-            const uint32_t s = byte_of(sg, lg);
+            const uint32_t g1 = static_cast<const uint32_t *>(grid_lds)[i1], g2 = static_cast<const uint32_t *>(grid_lds)[i2];
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
-                const float s1 = (s >> l) & 1u ? -1.0f : 1.0f;
-                const float s2 = (s >> (l + 4)) & 1u ? -1.0f : 1.0f;
-                const float w1 = __fmul_rn(__fmul_rn(sc, (float)byte_of(g1, l)), s1);
-                const float w2 = __fmul_rn(__fmul_rn(sc, (float)byte_of(g2, l)), s2);
+                const float w1 = flip(__fmul_rn(sc, (float)byte_of(g1, l)), sg, 8 * lg + l);
+                const float w2 = flip(__fmul_rn(sc, (float)byte_of(g2, l)), sg, 8 * lg + 4 + l);
                 out[8 * lg + l] = __fmul_rn(w1, x[8 * lg + l]);
                 out[8 * lg + 4 + l] = __fmul_rn(w2, x[8 * lg + 4 + l]);
             }
@@ -218,6 +258,10 @@ __device__ __forceinline__ void dequant_group(const Planes &P, uint32_t u, int s
     }
 }
 
+// One wave per workgroup adds the rows' products in order, three produce them a
+// block ahead.  What bounds it: the dependent f32 adds, 256 a block at 8 cycles
+// at best and 11.6 as measured (Q4_K 4096x4096: 36.2 -> 22.9 us with the next
+// block's bytes in flight, the codebooks in LDS and one wait per 64 adds).
 template <int TY>
 __global__ void __launch_bounds__(256) k_gemv_dequant(DequantArgs p) {
     __shared__ __align__(16) float s_prod[2][DQ_ROWS * DQ_STRIDE];
@@ -230,36 +274,73 @@ __global__ void __launch_bounds__(256) k_gemv_dequant(DequantArgs p) {
     const Planes P = make_planes(p.m.planes, p.m.units, p.m.bytes);
     const int tid = threadIdx.x;
     float sum = 0.0f;
-    // Step s: producers fill block s, the consumer adds block s - 1.
-    for (int s = 0; s <= nb; ++s) {
+    // Producer lane: group sub of row slot; rows past the matrix decode a real
+    // row (never stored).
+    const int slot = (tid - 64) >> 3, sub = tid & 7;
+    const int pr = r0 + slot < rows ? r0 + slot : rows - 1;
+    DqRaw<TY> ra, rb;
+    float4 xa[8], xb[8];
+    auto load = [&](int s, DqRaw<TY> &w, float4 (&x)[8]) {
+        w = dequant_load<TY>(P, (uint32_t)(pr * nb + s), sub);
+        const float4 *xs = reinterpret_cast<const float4 *>(p.x + (long long)s * 256 + 32 * sub);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = xs[i];
+    };
+    if (tid >= 64) load(0, ra, xa);
+    // the codebook to LDS: gathered from global memory its latency was the step's
+    __shared__ __align__(16) uint32_t s_grid[TY == T_IQ2_S ? 2048 : TY == T_IQ3_S ? 512 : 4];
+    if constexpr (TY == T_IQ2_S || TY == T_IQ3_S) {
+        const uint4 *src = reinterpret_cast<const uint4 *>(TY == T_IQ2_S ? (const void *)c_iq2s_grid : (const void *)c_iq3s_grid);
+        for (int i = tid; i < (int)(sizeof(s_grid) / 16); i += 256) reinterpret_cast<uint4 *>(s_grid)[i] = src[i];
+        __syncthreads();
+    }
+    // Step s: producers fill block s (block s + 1's loads in flight), the
+    // consumer adds block s - 1.
+    auto step = [&](int s, const DqRaw<TY> &raw, const float4 (&xv)[8], DqRaw<TY> &raw_next, float4 (&xv_next)[8]) {
         if (tid >= 64) {
             if (s < nb) {
-                const int t = tid - 64, slot = t >> 3, sub = t & 7;
-                int r = r0 + slot;
-                r = r < rows ? r : rows - 1;   // rows past the matrix decode a real row; never stored
-                float xv[32], out[32];
-                const float4 *xs = reinterpret_cast<const float4 *>(p.x + (long long)s * 256 + 32 * sub);
+                load(s + 1 < nb ? s + 1 : s, raw_next, xv_next);
+                float x[32], out[32];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float4 f = xs[i];
-                    xv[4 * i] = f.x, xv[4 * i + 1] = f.y, xv[4 * i + 2] = f.z, xv[4 * i + 3] = f.w;
-                }
-                dequant_group<TY>(P, (uint32_t)(r * nb + s), sub, xv, out);
+                for (int i = 0; i < 8; ++i) x[4 * i] = xv[i].x, x[4 * i + 1] = xv[i].y, x[4 * i + 2] = xv[i].z, x[4 * i + 3] = xv[i].w;
+                dequant_group<TY>(raw, sub, s_grid, x, out);
                 float4 *dst = reinterpret_cast<float4 *>(&s_prod[s & 1][slot * DQ_STRIDE + 32 * sub]);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) dst[i] = make_float4(out[4 * i], out[4 * i + 1], out[4 * i + 2], out[4 * i + 3]);
             }
         } else if (s > 0 && tid < DQ_ROWS) {
+            // The chain: batches of 64 products, one wait per batch, the next
+            // batch's reads issued ahead of this batch's adds (a read and a wait
+            // between every four adds ran at 13.4 cycles per add).
             const float4 *src = reinterpret_cast<const float4 *>(&s_prod[(s - 1) & 1][tid * DQ_STRIDE]);
-            for (int i = 0; i < 64; ++i) {
-                const float4 v = src[i];
-                sum = __fadd_rn(sum, v.x);
-                sum = __fadd_rn(sum, v.y);
-                sum = __fadd_rn(sum, v.z);
-                sum = __fadd_rn(sum, v.w);
+            float4 v[2][16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) v[0][i] = src[i];
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+                __builtin_amdgcn_sched_barrier(0);
+                if (b < 3) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) v[(b + 1) & 1][i] = src[16 * (b + 1) + i];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const float4 f = v[b & 1][i];
+                    sum = __fadd_rn(sum, f.x);
+                    sum = __fadd_rn(sum, f.y);
+                    sum = __fadd_rn(sum, f.z);
+                    sum = __fadd_rn(sum, f.w);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         __syncthreads();
+    };
+    for (int s = 0; s <= nb; s += 2) {
+        step(s, ra, xa, rb, xb);
+        if (s + 1 <= nb) step(s + 1, rb, xb, ra, xa);
     }
     const int r = r0 + tid;
     if (tid < DQ_ROWS && r < rows) {
