@@ -1,5 +1,5 @@
 // lbh_gemm.hip — Q4_K / Q5_K x Q8_K for a batch of tokens on the f16 matrix
-// cores (v_mfma_f32_32x32x16_f16), bit-identical to the reference's per-row
+// cores (v_mfma_f32_16x16x32_f16, 32x32x16), bit-identical to the reference's per-row
 // dot (dot_q4_or_q5_k, crates/bridge-quant-layout/src/q8_k.rs:247-327) for
 // every (row, token):
 //
@@ -16,17 +16,17 @@
 // (32 * 1953 * 128 < 2^23), so the f32 accumulation inside the instruction
 // is exact in any order and the result equals lane_sums[l] converted to f32
 // (which the reference's `as f32` also does exactly).  Each lane sum (the 32
-// elements of residue l) is two K = 16 instructions, the second accumulating
-// onto the first.  The minimum sum is a 17th instruction on the 6-bit mins
+// elements of residue l) is one K = 32 instruction on an operand pair, or two
+// K = 16 ones, the second accumulating onto the first.  The minimum sum is a
+// K = 16 instruction on the 6-bit mins
 // against the pair sums of bsums split as 128 * bh + bl: A holds
 // (128 mn_j, mn_j), B holds (bh_j, bl_j), |partial sums| < 8 * 63 * 8128.
 //
 // Layouts (built once per matrix by k_prep_a, per call by k_prep_b):
 //   A tile (32 rows, block b): 17 operands x 64 lanes x 16 B, operand o at
-//     position op_pos(o) (0-3, 16, 4-15: the order the three-pass schedule
-//     reads them in), then the 32 rows' d, -dmin, d, d as f32 (a pass of the
-//     three-pass schedule stages rows 0-1 or 2-3: chain 2's scale row 1 is
-//     then -dmin in pass 0 and d after it, at a fixed address).
+//     position op_pos(o) (0-3, 16, 4-15: a pass of the three-pass form reads
+//     consecutive ones), then the 32 rows' d, -dmin, d, d as f32 (the last two
+//     keep the tile a multiple of 512 B).
 //     Operand 2l + p, lane j: row j % 32, the 8 f16 of sub-blocks
 //     4p + 2 (j / 32) + e / 4, element 8 (e % 4) + l.
 //     Operand 16, lane j: sub-blocks 4 (j / 32) + e / 2, (128 mn, mn).
@@ -40,7 +40,6 @@
 namespace lbh {
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int OPS = 17;                          // 8 residues x 2 halves + the minimum
 constexpr int OP_BYTES = 1024;                   // 64 lanes x 8 f16
@@ -193,17 +192,93 @@ __global__ void __launch_bounds__(64) k_prep_b(const uint8_t *q8, int n_tokens, 
 
 // ------------------------------------------------------------------ GEMM
 //
-// Workgroup: 2 x 2 tiles of 32 rows x 32 tokens, two waves per tile: wave
-// half 0 runs residues 0-3 and the minimum, half 1 residues 4-7 (the eight
-// lane-sum chains are independent until the final sum), so a wave keeps 16
-// (row, token) pairs x 4 or 5 f32 chains in registers and two waves share
-// each SIMD.  Per block the workgroup stages its two A tiles and two B tiles
-// (70 KiB) in LDS, double-buffered.  Two ways to fill the buffers (`mode`):
-//   0  global -> registers -> LDS, two blocks ahead: block b + 2 is loaded
-//      into one register set while block b is computed, and the set loaded
-//      during block b - 1 is written to LDS after it (140 KiB in flight per
-//      CU; the loads are latency-bound, so depth is what buys bandwidth);
-//   1  direct buffer-to-LDS loads one block ahead (no staging registers).
+// Three forms, chosen by their counts of workgroups (launch_kq_gemm).  All run
+// the f32 chains on the VALU in the reference's block order, 8 instructions per
+// chain, 16 x 16 pairs and block, besides the scales.
+//
+//   k_kq_gemm_split  16 rows x 16 NT tokens per workgroup of three waves, each
+//     running three of the nine chains, both operands from L1 / L2: a short
+//     pass for launches of few pairs, bound by the operands' traffic from L2.
+//     77 tokens x 4096 rows x 4096 (Q4_K): 19 us with NT = 3, 21 with NT = 2
+//     (330 MB), 29 with the 2 x 2 form; 1024 rows: 16 us where that took 31.
+//   k_kq_gemm_2x2    64 rows x 64 tokens, both operands in LDS: 31-35 us for any
+//     count of workgroups up to the 256 CUs (LDS reads and staging latency).
+//   k_kq_gemm_lds    128 rows x 64 tokens, a wave 16 rows x 64 tokens in three
+//     passes over K of three chains each (64 accumulators: four waves fit a
+//     SIMD).  The row operands go straight from L2 to registers, one block
+//     ahead, each serving the wave's four token tiles; the token operands are
+//     staged in LDS two blocks at a time (direct buffer-to-LDS loads).  512
+//     tokens x 12288 rows x 4096 (Q5_K): 112 us, of which 68 are the issue of
+//     the VALU and matrix instructions, 58 the LDS reads and 16 the row
+//     operands' way past L2; with both operands in LDS and one 32 x 32 tile per
+//     wave, which reads LDS twice as much, 137.  All nine chains at once with 16
+//     x 64 pairs (two waves per SIMD, the tokens read once) took 136, four-wave
+//     workgroups of 64 rows 124, plain workgroup order 133, row operands and
+//     staging two blocks ahead 113.
+//
+// The split and LDS forms use v_mfma_f32_16x16x32_f16 with tokens as operand A
+// and rows as operand B: lane 16 q + c supplies token / row c and the 8
+// elements that tile lane (row c, half q & 1) holds in operand 2l + q / 2, so
+// one instruction gives a lane sum of 16 x 16 pairs, result i of the lane being
+// (token 4q + i, row c): the row's d is the lane's own and the four tokens' d8
+// one 16-byte read.
+
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+// Lane 16 q + c's place in a 32-row tile's operand pair 2l, 2l + 1 (rows 16 half
+// + c), in its minimum operand, and in its scale rows.
+__device__ __forceinline__ uint32_t op_lane(int lane, int half) {
+    const int q = lane >> 4, c = lane & 15;
+    return (uint32_t)((q >> 1) * OP_BYTES + (16 * half + c + 32 * (q & 1)) * 16);
+}
+__device__ __forceinline__ uint32_t min_lane(int lane, int half) {
+    const int q = lane >> 4, c = lane & 15;
+    return (uint32_t)(op_pos(16) * OP_BYTES + (16 * half + c + 32 * (q >> 1)) * 16 + 8 * (q & 1));
+}
+
+// The row operands of one wave: 16 rows of an A tile row, every block.
+struct RowSrc {
+    __amdgpu_buffer_rsrc_t r;
+    uint32_t op, mn, sc;   // lane offsets: operands, minimum operand, d / -dmin
+    __device__ __forceinline__ RowSrc(const uint8_t *a, int tile, int half, int nb, int lane) {
+        r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(a + (long long)tile * nb * A_TILE), (short)0, nb * A_TILE,
+                                              0x00020000);
+        op = op_lane(lane, half);
+        mn = min_lane(lane, half);
+        sc = (uint32_t)(OPS * OP_BYTES + (16 * half + (lane & 15)) * 4);
+    }
+    __device__ __forceinline__ v8h residue(int b, int l) const {
+        return __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(r, op, (uint32_t)(b * A_TILE + op_pos(2 * l) * OP_BYTES), 0));
+    }
+    __device__ __forceinline__ v4h minimum(int b) const {
+        return __builtin_bit_cast(v4h, __builtin_amdgcn_raw_buffer_load_b64(r, mn, (uint32_t)(b * A_TILE), 0));
+    }
+    __device__ __forceinline__ float d(int b) const {
+        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, sc, (uint32_t)(b * A_TILE), 0));
+    }
+    __device__ __forceinline__ float neg_dmin(int b) const {
+        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, sc, (uint32_t)(b * A_TILE + 128), 0));
+    }
+};
+
+// acc += (scale * d8) * sum for one chain of one token tile.
+__device__ __forceinline__ void fold4(float (&acc)[4], const float (&s)[4], const v4f &r) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn(s[i], r[i]));
+}
+
+// ---- 2 x 2 tiles in LDS
+//
+// Workgroup: 2 x 2 tiles of 32 rows x 32 tokens (v_mfma_f32_32x32x16_f16, two
+// per lane sum), two waves per tile: wave half 0 runs residues 0-3 and the
+// minimum, half 1 residues 4-7, so a wave keeps 16 (row, token) pairs x 4 or 5
+// f32 chains in registers and two waves share each SIMD.  Per block the
+// workgroup stages its two A tiles and two B tiles (70 KiB) in LDS,
+// double-buffered, through registers two blocks ahead: block b + 2 is loaded
+// into one register set while block b is computed, and the set loaded during
+// block b - 1 is written to LDS after it (140 KiB in flight per CU).
 constexpr int RG = 2, TG = 2;                 // row tiles, token tiles per workgroup
 constexpr int NW = 2 * RG * TG;               // waves
 constexpr int UNITS = (RG + TG) * PIECES;     // 1 KiB staging units per block
@@ -218,8 +293,6 @@ struct GemmLDS {
     uint8_t a[2][RG][LDS_TILE];
     uint8_t b[2][TG][LDS_TILE];
 };
-
-typedef __attribute__((address_space(3))) void lds_void;
 
 // Where staging unit k of wave `wid` lives: unit u = wid + NW k is piece
 // u % PIECES of tile u / PIECES (A tiles first).  Tiles past the matrix or
@@ -277,16 +350,6 @@ __device__ __forceinline__ void store_regs(GemmLDS &S, const uint4 (&R)[UPW], in
         reinterpret_cast<uint4 *>(unit_dst(S, x, buf))[lane] = R[k];
     }
 }
-__device__ __forceinline__ void stage_dma(const StageSrc &src, GemmLDS &S, int nb, int b, int buf, int wid, int lane) {
-#pragma unroll
-    for (int k = 0; k < UPW; ++k) {
-        const Unit x = unit_of(wid, k);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(x.is_a ? src.ra : src.rb, (lds_void *)unit_dst(S, x, buf), 16,
-                                                 lane * 16, unit_offset(src, x, nb, b), 0, 0);
-    }
-}
-__device__ __forceinline__ void wait_dma() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
 // Both MFMAs of residue l (operands 2l, 2l + 1), or the minimum (l = 8).
 __device__ __forceinline__ v16f residue_mfma(const v8h *Av, const v8h *Bv, int l) {
     const v16f zero = {};
@@ -357,7 +420,7 @@ __device__ __forceinline__ void fold_block(Chains<HV> &ch, const uint8_t *At, co
     }
 }
 
-template <int MODE, int HV>
+template <int HV>
 __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const MatGemm &M, GemmLDS &S, const StageSrc &src,
                                           int rg, int tg, int tw, int wid, int lane, int rt0, int tt0) {
     const int nb = g.nb;
@@ -368,40 +431,27 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const MatGemm &M, G
 #pragma unroll
         for (int r = 0; r < 4; ++r) ch.c[i][r] = 0.0f;
     }
-    if (MODE == 0) {
-        // Block j: loaded into R[j % 2] during block j - 2, written to LDS
-        // buffer j % 2 after block j - 1, computed as block j.  Every load
-        // is unconditional, so the compiler's wait before each LDS store
-        // leaves the younger set's loads in flight; loads past the last
-        // block are sent out of the descriptor's range (they return zeros
-        // without touching memory).
-        uint4 R0[UPW], R1[UPW];
-        stage_regs(src, R0, nb, 0, wid, lane);
-        stage_regs(src, R1, nb, 1, wid, lane);
-        store_regs(S, R0, 0, wid, lane);
+    // Block j: loaded into R[j % 2] during block j - 2, written to LDS
+    // buffer j % 2 after block j - 1, computed as block j.  Every load
+    // is unconditional, so the compiler's wait before each LDS store
+    // leaves the younger set's loads in flight; loads past the last
+    // block are sent out of the descriptor's range (they return zeros
+    // without touching memory).
+    uint4 R0[UPW], R1[UPW];
+    stage_regs(src, R0, nb, 0, wid, lane);
+    stage_regs(src, R1, nb, 1, wid, lane);
+    store_regs(S, R0, 0, wid, lane);
+    __syncthreads();
+    for (int b = 0; b < nb; b += 2) {
+        stage_regs(src, R0, nb, b + 2, wid, lane);
+        fold_block<HV>(ch, S.a[0][rg], S.b[0][tg], lane);
+        if (b + 1 < nb) store_regs(S, R1, 1, wid, lane);
         __syncthreads();
-        for (int b = 0; b < nb; b += 2) {
-            stage_regs(src, R0, nb, b + 2, wid, lane);
-            fold_block<HV>(ch, S.a[0][rg], S.b[0][tg], lane);
-            if (b + 1 < nb) store_regs(S, R1, 1, wid, lane);
-            __syncthreads();
-            if (b + 1 >= nb) break;
-            stage_regs(src, R1, nb, b + 3, wid, lane);
-            fold_block<HV>(ch, S.a[1][rg], S.b[1][tg], lane);
-            if (b + 2 < nb) store_regs(S, R0, 0, wid, lane);
-            __syncthreads();
-        }
-    } else {
-        stage_dma(src, S, nb, 0, 0, wid, lane);
-        wait_dma();
+        if (b + 1 >= nb) break;
+        stage_regs(src, R1, nb, b + 3, wid, lane);
+        fold_block<HV>(ch, S.a[1][rg], S.b[1][tg], lane);
+        if (b + 2 < nb) store_regs(S, R0, 0, wid, lane);
         __syncthreads();
-        for (int b = 0; b < nb; ++b) {
-            const int buf = b & 1;
-            if (b + 1 < nb) stage_dma(src, S, nb, b + 1, buf ^ 1, wid, lane);
-            fold_block<HV>(ch, S.a[buf][rg], S.b[buf][tg], lane);
-            wait_dma();
-            __syncthreads();
-        }
     }
 
     // result = minimum chain + sums[0] + ... + sums[7]: half 0 adds its four
@@ -433,8 +483,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const MatGemm &M, G
     }
 }
 
-template <int MODE>
-__global__ void __launch_bounds__(64 * NW) k_kq_gemm(GemmArgs g) {
+__global__ void __launch_bounds__(64 * NW) k_kq_gemm_2x2(GemmArgs g) {
     extern __shared__ __align__(16) uint8_t smem[];
     GemmLDS &S = *reinterpret_cast<GemmLDS *>(smem);
     const int lane = threadIdx.x & 63;
@@ -482,291 +531,312 @@ __global__ void __launch_bounds__(64 * NW) k_kq_gemm(GemmArgs g) {
                                                (src.last_b + 1) * g.nb * B_TILE, 0x00020000);
 
     if (hv == 0)
-        gemm_tile<MODE, 0>(g, M, S, src, rg, tg, tw, wid, lane, rt0, tt0);
+        gemm_tile<0>(g, M, S, src, rg, tg, tw, wid, lane, rt0, tt0);
     else
-        gemm_tile<MODE, 1>(g, M, S, src, rg, tg, tw, wid, lane, rt0, tt0);
+        gemm_tile<1>(g, M, S, src, rg, tg, tw, wid, lane, rt0, tt0);
 }
 
-// ------------------------------------------------------- three-pass GEMM
-//
-// The nine chains of a (row, token) pair are independent until the final sum
-// result = ((sum_min + s_0) + s_1) + ... + s_7, so they can run as three
-// passes over K in the reference's order, the running result kept in
-// registers between them:
-//   pass 0: lane chains 0, 1 and the minimum chain (tile positions 0-4)
-//   pass 1: lane chains 2, 3, 4 (positions 5-10)
-//   pass 2: lane chains 5, 6, 7 (positions 11-16)
-// A pass stages only its own operands (six slots: pass p's positions
-// 6p - (p > 0) + 0..5, pass 0's sixth slot zeros), plus the tile's scales,
-// so one workgroup covers RG x TG = 12 tiles of 32 x 32 with one wave per
-// tile and three chains per wave (3 waves per SIMD), and each staged tile
-// serves TG (A) or RG (B) tiles: about 60% of the 2 x 2 schedule's staged
-// bytes per output.  Chain c of a pass is the MFMA pair on slots 2c, 2c + 1;
-// pass 0's minimum chain pairs its operand with the zero slot (the second
-// instruction adds exact zeros).  A stage is (RG + TG) tiles x 7 KiB (six
-// operand slots, then the 1 KiB piece holding d/-dmin or d8), triple-buffered
-// in LDS by direct buffer-to-LDS loads two stages ahead.
-constexpr int P3_WAVES = 12;
-constexpr int P3_SLOTS = 7;                                   // 6 operands + the scale piece
-constexpr int P3_TILE = P3_SLOTS * OP_BYTES;
-constexpr int P3_MAX_TILES = 7;                               // RG + TG
-constexpr int P3_PAD = P3_MAX_TILES * P3_TILE;                // target of the padding loads
-constexpr int P3_BUF = P3_PAD + OP_BYTES;
-static_assert(op_pos(16) == 4 && op_pos(4) == 5, "pass windows: 0-4 (+ zeros), 5-10, 11-16");
+// ---- tokens in LDS
 
-// The three stage buffers are distinct LDS arrays, each addressed statically
-// (the stage loop is unrolled by three): the compiler's wait before an LDS
-// read then covers only the buffer-to-LDS loads into that array, not the
-// prefetches into the other two, which stay in flight.
-__shared__ __align__(16) uint8_t p3_lds0[P3_BUF];
-__shared__ __align__(16) uint8_t p3_lds1[P3_BUF];
-__shared__ __align__(16) uint8_t p3_lds2[P3_BUF];
+constexpr int GL_WAVES = 8, GL_NT = 4;
+constexpr int GL_PASS_OPS = 6;                       // operand positions of a pass (pass 0: five)
+constexpr int GL_TILE = GL_PASS_OPS * OP_BYTES;      // one 32-token tile's operands of a pass
+constexpr int GL_BLOCK = 2 * GL_TILE + 256;          // two tiles, then the 64 tokens' d8
+// Two distinct arrays: the compiler's wait before a read of one leaves the
+// loads into the other in flight.
+__shared__ __align__(16) uint8_t gl_lds0[2 * GL_BLOCK];
+__shared__ __align__(16) uint8_t gl_lds1[2 * GL_BLOCK];
+
+#define GL_FENCE __builtin_amdgcn_sched_barrier(0)
+
+typedef __attribute__((address_space(3))) void lds_void;
 
 template <int BUF>
-__device__ __forceinline__ uint8_t *p3_buffer() {
-    return BUF == 0 ? p3_lds0 : BUF == 1 ? p3_lds1 : p3_lds2;
+__device__ __forceinline__ uint8_t *gl_buffer() {
+    return BUF == 0 ? gl_lds0 : gl_lds1;
 }
 
-template <int RG_, int TG_>
-struct P3 {
-    static_assert(RG_ * TG_ == P3_WAVES, "one wave per tile");
-    static_assert(RG_ + TG_ <= P3_MAX_TILES, "stages fit the LDS buffers");
-    static constexpr int RG = RG_, TG = TG_;
-    static constexpr int UA = (RG * P3_SLOTS + P3_WAVES - 1) / P3_WAVES;   // A loads per wave per stage
-    static constexpr int UB = (TG * P3_SLOTS + P3_WAVES - 1) / P3_WAVES;   // B loads per wave per stage
-    static constexpr int UPW = UA + UB;
-};
-
-// This wave's share of a stage's loads, fixed for the whole K loop: load k of
-// the A side is unit u = wid + 12 k of the RG x 7 A units (slot u % 7 of A
-// tile u / 7), likewise for the TG x 7 B units; units past a side's count
-// are padding.  Per unit: its LDS offset in a stage buffer, the byte offset
-// in the side's descriptor of its piece in block 0 of pass 0 (the scale
-// piece: the same in every pass), and three masks: pad (0x80000000 for a
-// unit past the stage), zero (all ones for pass 0's sixth slot), win (all
-// ones unless the scale piece, which ignores the pass window).
-struct P3Unit {
-    int lds, off;
-    uint32_t pad, zero, win;
-};
-template <int SIDE_TILES, int TILE_BYTES>
-__device__ __forceinline__ P3Unit p3_unit(int u, int lds_tile0, int last, int nb) {
-    P3Unit x;
-    const int ti = u / P3_SLOTS, slot = u - ti * P3_SLOTS;
-    const bool in_stage = u < SIDE_TILES * P3_SLOTS;
-    x.pad = in_stage ? 0u : 0x80000000u;
-    x.zero = slot == 5 ? ~0u : 0u;
-    x.win = slot == 6 ? 0u : ~0u;
-    x.lds = in_stage ? (lds_tile0 + ti) * P3_TILE + slot * OP_BYTES : P3_PAD;
-    x.off = (ti < last ? ti : last) * nb * TILE_BYTES + (slot == 6 ? OPS : slot) * OP_BYTES;
-    return x;
-}
-
-// Issues this wave's loads of the stage at (poff, bA, bB) into buffer BUF:
-// poff = the pass's window start in bytes, bA / bB = the block's offset in a
-// tile row of the A / B side, dead = 0x80000000 for a stage past the end (all
-// its loads padding), z0 = 0x80000000 in pass 0 (its sixth slot is zeros),
-// soff = where the A scale piece starts (0 in pass 0, 256 after).
-// A padding load reads from beyond the descriptor range (zeros, no memory
-// traffic): units past the stage into the buffer's padding piece, pass 0's
-// sixth slot into that slot.  Every wave issues UPW loads per stage, with no
-// branch between them, so one wait count serves all and the compiler's own
-// waits before the LDS reads stay exact.
-template <class S, int BUF>
-__device__ __forceinline__ void p3_issue(const StageSrc &src, const P3Unit (&ua)[S::UA], const P3Unit (&ub)[S::UB],
-                                         int poff, int bA, int bB, uint32_t dead, uint32_t z0, uint32_t soff,
-                                         uint32_t lane16) {
-    uint8_t *buf = p3_buffer<BUF>();
+// Blocks b and b + 1 (clamped) of the token tiles, operand positions op0 .. op0
+// + 5: 24 pieces of 1 KiB, three per wave, and each block's d8 by one wave.
+template <int BUF>
+__device__ __forceinline__ void gl_stage(__amdgpu_buffer_rsrc_t rb, int last, int nb, int b, int op0, int wid, int lane) {
+    uint8_t *buf = gl_buffer<BUF>();
 #pragma unroll
-    for (int k = 0; k < S::UA + S::UB; ++k) {
-        const bool is_a = k < S::UA;
-        const P3Unit &x = is_a ? ua[k] : ub[k - S::UA];
-        const uint32_t vo = lane16 | (x.pad | dead | (z0 & x.zero));
-        uint32_t off = (uint32_t)(x.off + (is_a ? bA : bB)) + ((uint32_t)poff & x.win);
-        if (is_a) off += soff & ~x.win;   // A scale piece: rows 0-1 in pass 0, rows 2-3 after
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(is_a ? src.ra : src.rb, (lds_void *)(buf + x.lds), 16, vo, off, 0, 0);
+    for (int k = 0; k < 3; ++k) {
+        const int u = wid + GL_WAVES * k, blk = u / 12, t = (u / 6) & 1, piece = u % 6;
+        const int bb = b + blk < nb ? b + blk : nb - 1;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void *)(buf + blk * GL_BLOCK + t * GL_TILE + piece * OP_BYTES), 16, lane * 16,
+                                                 (uint32_t)(((t < last ? t : last) * nb + bb) * B_TILE + (op0 + piece) * OP_BYTES), 0, 0);
+    }
+    if (wid < 2) {
+        const int bb = b + wid < nb ? b + wid : nb - 1, t = lane >> 5;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void *)(buf + wid * GL_BLOCK + 2 * GL_TILE), 4,
+                                                 (t < last ? t : last) * nb * B_TILE + (lane & 31) * 4,
+                                                 (uint32_t)(bb * B_TILE + OPS * OP_BYTES), 0, 0);
     }
 }
 
-// One block of the wave's tile (At, Bt: its A and B tiles in the stage
-// buffer): chain c += (scale * d8) * integer sum, in the reference's order
-// (q8_k.rs:314-326), with scale = staged row 0 (d) for chains 0 and 1, and
-// for chain 2 row 1 in pass 0 (-dmin: the minimum chain) and d after it.
-// The operands of chain c + 1 are read from LDS while chain c's MFMAs run
-// and its fold issues.
-__device__ __forceinline__ void p3_block(float (&ch)[3][16], const uint8_t *At, const uint8_t *Bt, int lane,
-                                         bool first_pass) {
-    const int h = lane >> 5;
-    const v8h *Av = reinterpret_cast<const v8h *>(At) + lane;
-    const v8h *Bv = reinterpret_cast<const v8h *>(Bt) + lane;
-    const float d8 = reinterpret_cast<const float *>(Bt + 6 * OP_BYTES)[lane & 31];
-    const float4 *dv = reinterpret_cast<const float4 *>(At + 6 * OP_BYTES);
-    v8h a0 = Av[0], b0 = Bv[0], a1 = Av[64], b1 = Bv[64];
-    float sc[16];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const float4 d = dv[2 * q + h];
-        sc[4 * q] = __fmul_rn(d.x, d8);
-        sc[4 * q + 1] = __fmul_rn(d.y, d8);
-        sc[4 * q + 2] = __fmul_rn(d.z, d8);
-        sc[4 * q + 3] = __fmul_rn(d.w, d8);
+// Three chains of a pass and its running operands.  MIN (pass 0): the minimum
+// chain (slot 2) and lane chains 0, 1; otherwise three lane chains from l0.
+template <bool MIN>
+struct GlPass {
+    float c[3][GL_NT][4];
+    v8h a[3];
+    float d, ndm;
+
+    __device__ __forceinline__ void load(const RowSrc &A, int b, int l0, int k) {
+        if (MIN && k == 2) a[2] = __builtin_bit_cast(v8h, __builtin_shufflevector(A.minimum(b), A.minimum(b), 0, 1, 2, 3, 0, 1, 2, 3));
+        else a[k] = A.residue(b, l0 + k);
     }
+    __device__ __forceinline__ void load_scales(const RowSrc &A, int b) {
+        d = A.d(b);
+        if (MIN) ndm = A.neg_dmin(b);
+    }
+
+    __device__ __forceinline__ void block(const uint8_t *buf, const RowSrc &A, int bn, int l0, int lane) {
+        const int q = lane >> 4;
+        const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        // step 2 k + p: chain k, the token tiles of the 32-token tile p
+        v8h x[2][2];
+        auto tokens = [&](int st) {
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        const v16f zero = {};
-        asm volatile("" : "+v"(a0), "+v"(b0), "+v"(a1), "+v"(b1));
-        const v16f x = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b0, zero, 0, 0, 0);
-        const v16f cur = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b1, x, 0, 0, 0);
-        if (c < 2) {
-            a0 = Av[2 * (c + 1) * 64], b0 = Bv[2 * (c + 1) * 64];
-            a1 = Av[(2 * c + 3) * 64], b1 = Bv[(2 * c + 3) * 64];
-        }
-        __builtin_amdgcn_sched_barrier(0);   // the reads go out before this chain's fold
-        if (c < 2 || !first_pass) {
+            for (int n = 0; n < 2; ++n) {
+                const uint8_t *t = buf + (st & 1) * GL_TILE;
+                if (MIN && st >= 4) {
+                    const v4h h = *reinterpret_cast<const v4h *>(t + min_lane(lane, n));
+                    x[st & 1][n] = __builtin_shufflevector(h, h, 0, 1, 2, 3, 0, 1, 2, 3);
+                } else {
+                    x[st & 1][n] = *reinterpret_cast<const v8h *>(t + (st & ~1) * OP_BYTES + op_lane(lane, n));
+                }
+            }
+        };
+        float4 e[GL_NT];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) ch[c][i] = __fadd_rn(ch[c][i], __fmul_rn(sc[i], cur[i]));
-        } else {
+        for (int n = 0; n < GL_NT; ++n) e[n] = *reinterpret_cast<const float4 *>(buf + 2 * GL_TILE + (16 * n + 4 * q) * 4);
+        tokens(0);
+        GL_FENCE;
+        float s[GL_NT][4], m[MIN ? GL_NT : 1][4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float4 e = dv[8 + 2 * q + h];
-                const float ms[4] = {__fmul_rn(e.x, d8), __fmul_rn(e.y, d8), __fmul_rn(e.z, d8), __fmul_rn(e.w, d8)};
+        for (int n = 0; n < GL_NT; ++n) {
+            const float d8[4] = {e[n].x, e[n].y, e[n].z, e[n].w};
 #pragma unroll
-                for (int k = 0; k < 4; ++k) ch[2][4 * q + k] = __fadd_rn(ch[2][4 * q + k], __fmul_rn(ms[k], cur[4 * q + k]));
+            for (int i = 0; i < 4; ++i) {
+                s[n][i] = __fmul_rn(d, d8[i]);
+                if (MIN) m[n][i] = __fmul_rn(ndm, d8[i]);
             }
         }
-        asm volatile("" : "+v"(ch[c][0]), "+v"(ch[c][1]), "+v"(ch[c][2]), "+v"(ch[c][3]), "+v"(ch[c][4]),
-                     "+v"(ch[c][5]), "+v"(ch[c][6]), "+v"(ch[c][7]), "+v"(ch[c][8]), "+v"(ch[c][9]),
-                     "+v"(ch[c][10]), "+v"(ch[c][11]), "+v"(ch[c][12]), "+v"(ch[c][13]), "+v"(ch[c][14]),
-                     "+v"(ch[c][15]));
-    }
-}
-
-// Stage position: pass p, block b of the stage computed (cp, cb) and of the
-// stage issued two ahead (ip, ib), advanced without divisions; ipoff, ibA,
-// ibB the issued stage's pass window and block offsets.
-struct P3Pos {
-    int cp, cb, ip, ib, ipoff, ibA, ibB;
-};
-__device__ __forceinline__ void p3_next_issue(P3Pos &ps, int nb) {
-    ps.ibA += A_TILE, ps.ibB += B_TILE;
-    if (++ps.ib == nb) {
-        ps.ib = 0, ps.ibA = 0, ps.ibB = 0, ++ps.ip;
-        ps.ipoff = (6 * ps.ip - 1) * OP_BYTES;
-    }
-}
-// The issued stage's masks for p3_issue, made opaque to the compiler (an empty
-// asm statement) so it cannot specialise the loads on the pass.
-template <class S, int BUF>
-__device__ __forceinline__ void p3_issue_at(const StageSrc &src, const P3Unit (&ua)[S::UA],
-                                            const P3Unit (&ub)[S::UB], const P3Pos &ps, uint32_t lane16) {
-    uint32_t dead = (uint32_t)(2 - ps.ip) & 0x80000000u;   // ip == 3: past the end
-    uint32_t z0 = (uint32_t)(ps.ip - 1) & 0x80000000u;     // ip == 0
-    uint32_t soff = ~z0 >> 23 & 256u;                      // 0 in pass 0, 256 after
-    asm volatile("" : "+s"(dead), "+s"(z0), "+s"(soff));
-    p3_issue<S, BUF>(src, ua, ub, ps.ipoff, ps.ibA, ps.ibB, dead, z0, soff, lane16);
-}
-
-// Stage s of the K loop in buffer BUF = s % 3: wait for this wave's loads of
-// stage s (stage s + 1's stay in flight), barrier (every wave's loads of
-// stage s have landed and every wave has finished stage s - 1, whose buffer
-// is refilled next), issue stage s + 2 (padding past the end: the control
-// flow is the same in every stage, which keeps the compiler's own wait before
-// each LDS read down to the loads into that buffer), then the block's MFMAs
-// and folds for pass cp.  At a pass's last block the pass's chains go onto
-// the running result v in the reference's order (pass 0: minimum chain, then
-// lane chains 0, 1) and restart.
-template <class S, int BUF>
-__device__ __forceinline__ void p3_stage(float (&ch)[3][16], float (&v)[16], const StageSrc &src,
-                                         const P3Unit (&ua)[S::UA], const P3Unit (&ub)[S::UB], P3Pos &ps, int nb,
-                                         int lane, int rt, int tt) {
-    static_assert(S::UPW == 5, "the wait count below is one stage's loads");
-    asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    p3_issue_at<S, (BUF + 2) % 3>(src, ua, ub, ps, (uint32_t)lane * 16);
-    p3_next_issue(ps, nb);
-    // The lane index goes through an empty asm statement per stage, so the
-    // lane addresses into this buffer are formed here, not kept in registers
-    // across the loop for all three buffers.
-    int ln = lane;
-    asm volatile("" : "+v"(ln));
-    const uint8_t *buf = p3_buffer<BUF>();
-    const int p = ps.cp;
-    p3_block(ch, buf + rt * P3_TILE, buf + (S::RG + tt) * P3_TILE, ln, p == 0);
-    if (ps.cb == nb - 1) {
-        if (p == 0) {
+        load_scales(A, bn);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = __fadd_rn(__fadd_rn(ch[2][i], ch[0][i]), ch[1][i]);
-        } else {
+        for (int st = 0; st < 6; ++st) {
+            const int k = st >> 1, p = st & 1;
+            v4f r[2];
+            if (st < 5) tokens(st + 1);
+            GL_FENCE;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = __fadd_rn(__fadd_rn(__fadd_rn(v[i], ch[0][i]), ch[1][i]), ch[2][i]);
+            for (int n = 0; n < 2; ++n) {
+                if (MIN && k == 2)
+                    r[n] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_shufflevector(x[p][n], x[p][n], 0, 1, 2, 3),
+                                                                 __builtin_shufflevector(a[2], a[2], 0, 1, 2, 3), zero, 0, 0, 0);
+                else
+                    r[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[p][n], a[k], zero, 0, 0, 0);
+            }
+            if (p == 1) load(A, bn, l0, k);
+            GL_FENCE;
+#pragma unroll
+            for (int n = 0; n < 2; ++n) fold4(c[k][2 * p + n], MIN && k == 2 ? m[2 * p + n] : s[2 * p + n], r[n]);
         }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) ch[0][i] = ch[1][i] = ch[2][i] = 0.0f;
     }
-    if (++ps.cb == nb) ps.cb = 0, ++ps.cp;
+};
+
+// One pass over the blocks: v = ((v + c) + c') + c''.
+template <bool MIN>
+__device__ __forceinline__ void gl_pass(float (&v)[GL_NT][4], const RowSrc &A, __amdgpu_buffer_rsrc_t rb, int last, int nb, int l0,
+                                        int wid, int lane) {
+    const int op0 = MIN ? 0 : op_pos(4) + 2 * (l0 - 2);
+    GlPass<MIN> p;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int n = 0; n < GL_NT; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p.c[c][n][i] = 0.0f;
+    gl_stage<0>(rb, last, nb, 0, op0, wid, lane);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) p.load(A, 0, l0, k);
+    p.load_scales(A, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    for (int b = 0; b < nb; b += 4) {
+        // the next two blocks' tokens go to the other buffer meanwhile
+        gl_stage<1>(rb, last, nb, b + 2, op0, wid, lane);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            if (b + h < nb) p.block(gl_buffer<0>() + h * GL_BLOCK, A, b + h + 1 < nb ? b + h + 1 : nb - 1, l0, lane);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        gl_stage<0>(rb, last, nb, b + 4, op0, wid, lane);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            if (b + 2 + h < nb) p.block(gl_buffer<1>() + h * GL_BLOCK, A, b + h + 3 < nb ? b + h + 3 : nb - 1, l0, lane);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+#pragma unroll
+    for (int n = 0; n < GL_NT; ++n)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (MIN) v[n][i] = __fadd_rn(__fadd_rn(p.c[2][n][i], p.c[0][n][i]), p.c[1][n][i]);
+            else v[n][i] = __fadd_rn(__fadd_rn(__fadd_rn(v[n][i], p.c[0][n][i]), p.c[1][n][i]), p.c[2][n][i]);
+        }
 }
 
-template <int RG_, int TG_>
-__global__ void __launch_bounds__(64 * P3_WAVES) k_kq_gemm3(GemmArgs g) {
-    using S = P3<RG_, TG_>;
+__global__ void __launch_bounds__(64 * GL_WAVES, 4) k_kq_gemm_lds(GemmArgs g) {
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int rt = wid % S::RG, tt = wid / S::RG;
     const MatGemm &M = g.mat[blockIdx.y];
     const int nb = g.nb;
     const int n_rt = (M.rows + 31) / 32, n_tt = (g.n_tokens + 31) / 32;
-    const int row_wgs = (n_rt + S::RG - 1) / S::RG, tok_wgs = (n_tt + S::TG - 1) / S::TG;
-    // XCD-aware order: workgroups are dealt to the eight XCDs round robin;
-    // each XCD takes a contiguous run of row groups with all their token
-    // groups, so the token groups of a row group run together on one XCD and
-    // its A tiles are fetched into that XCD's L2 once.
+    const int row_wgs = (n_rt + 3) / 4, tok_wgs = (n_tt + 1) / 2;
+    // XCD-aware order: workgroups are dealt to the eight XCDs round robin; each
+    // XCD takes a contiguous run of row groups with all their token groups, so
+    // a row group's operands are fetched into one XCD's L2 once.
     const int nwg = row_wgs * tok_wgs;
     const int id = (int)blockIdx.x;
     if (id >= nwg) return;
     const int nfull = nwg & ~7;
     const int lin = id < nfull ? (id % 8) * (nfull / 8) + id / 8 : id;   // a bijection of [0, nwg)
-    const int wrt = lin / tok_wgs, wtt = lin - wrt * tok_wgs;
-    const int rt0 = wrt * S::RG, tt0 = wtt * S::TG;
-
-    // The descriptors span only the workgroup's valid tiles (the scale piece
-    // of the last one reads zeros past it, never memory past the allocation).
-    StageSrc src;
-    src.last_a = n_rt - 1 - rt0 < S::RG - 1 ? n_rt - 1 - rt0 : S::RG - 1;
-    src.last_b = n_tt - 1 - tt0 < S::TG - 1 ? n_tt - 1 - tt0 : S::TG - 1;
-    src.ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(M.a + (long long)rt0 * nb * A_TILE), (short)0,
-                                               (src.last_a + 1) * nb * A_TILE, 0x00020000);
-    src.rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(g.b + (long long)tt0 * nb * B_TILE), (short)0,
-                                               (src.last_b + 1) * nb * B_TILE, 0x00020000);
-
-    P3Unit ua[S::UA], ub[S::UB];
+    const int wrt = lin / tok_wgs, tt0 = (lin - wrt * tok_wgs) * 2;
+    const int rt = wrt * 4 + (wid >> 1), half = wid & 1;
+    const RowSrc A(M.a, rt < n_rt ? rt : n_rt - 1, half, nb, lane);   // rows past the matrix: never stored
+    const int last = n_tt - 1 - tt0 < 1 ? n_tt - 1 - tt0 : 1;
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(g.b + (long long)tt0 * nb * B_TILE), (short)0, (last + 1) * nb * B_TILE, 0x00020000);
+    float v[GL_NT][4];
+    gl_pass<true>(v, A, rb, last, nb, 0, wid, lane);
+    for (int l0 = 2; l0 < 8; l0 += 3) gl_pass<false>(v, A, rb, last, nb, l0, wid, lane);
+    const int row = rt * 32 + 16 * half + (lane & 15);
+    if (row >= M.rows) return;
 #pragma unroll
-    for (int k = 0; k < S::UA; ++k) ua[k] = p3_unit<S::RG, A_TILE>(wid + P3_WAVES * k, 0, src.last_a, nb);
+    for (int n = 0; n < GL_NT; ++n)
 #pragma unroll
-    for (int k = 0; k < S::UB; ++k) ub[k] = p3_unit<S::TG, B_TILE>(wid + P3_WAVES * k, S::RG, src.last_b, nb);
+        for (int i = 0; i < 4; ++i) {
+            const int t = tt0 * 32 + 16 * n + 4 * (lane >> 4) + i;
+            if (t < g.n_tokens) M.y[(long long)t * M.ldy + row] = v[n][i];
+        }
+}
 
-    const int total = 3 * nb;   // stages: (pass, block), a multiple of three
-    P3Pos ps{0, 0, 0, 0, 0, 0, 0};
-    p3_issue_at<S, 0>(src, ua, ub, ps, (uint32_t)lane * 16);
-    p3_next_issue(ps, nb);
-    p3_issue_at<S, 1>(src, ua, ub, ps, (uint32_t)lane * 16);
-    p3_next_issue(ps, nb);
-    float ch[3][16], v[16];
+// ---- chains split over three waves, tokens from L1 / L2
+
+constexpr int GS_WAVES = 3;
+
+// Wave W's chains: 0: the minimum and lane chains 0, 1; 1: 2, 3, 4; 2: 5, 6, 7
+// (slot k: residue first + k, slot 2 of wave 0 the minimum).
+template <int NT, int W>
+__device__ __forceinline__ void gs_chains(const RowSrc &A, const GemmArgs &g, int tt0, int lane, float (&acc)[3][NT][4]) {
+    constexpr int L0 = W == 0 ? 0 : 3 * W - 1, NL = W == 0 ? 2 : 3;
+    const int nb = g.nb, q = lane >> 4;
+    const int n16 = (g.n_tokens + 15) / 16;
+    const uint8_t *tp[NT];
+    int th[NT];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) ch[0][i] = ch[1][i] = ch[2][i] = v[i] = 0.0f;
-    for (int s = 0; s < total; s += 3) {
-        p3_stage<S, 0>(ch, v, src, ua, ub, ps, nb, lane, rt, tt);
-        p3_stage<S, 1>(ch, v, src, ua, ub, ps, nb, lane, rt, tt);
-        p3_stage<S, 2>(ch, v, src, ua, ub, ps, nb, lane, rt, tt);
+    for (int n = 0; n < NT; ++n) {
+        const int t = tt0 + n < n16 ? tt0 + n : n16 - 1;   // tiles past the batch: never stored
+        tp[n] = g.b + (long long)(t >> 1) * nb * B_TILE;
+        th[n] = t & 1;
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the padding loads land before the LDS is released
-
-    const int h = lane >> 5;
-    const int t = (tt0 + tt) * 32 + (lane & 31);
-    if (t >= g.n_tokens) return;
+    struct Step {
+        v8h a[NL], b[NL][NT];
+        v4h am, bm[NT];
+        float d, ndm;
+        float4 e[NT];
+    };
+    auto load = [&](int b, Step &x) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int row = (rt0 + rt) * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
-        if (row < M.rows) M.y[(long long)t * M.ldy + row] = v[i];
+        for (int l = 0; l < NL; ++l) {
+            x.a[l] = A.residue(b, L0 + l);
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                x.b[l][n] = *reinterpret_cast<const v8h *>(tp[n] + (long long)b * B_TILE + op_pos(2 * (L0 + l)) * OP_BYTES +
+                                                           op_lane(lane, th[n]));
+        }
+        x.d = A.d(b);
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+            x.e[n] = *reinterpret_cast<const float4 *>(tp[n] + (long long)b * B_TILE + OPS * OP_BYTES + (16 * th[n] + 4 * q) * 4);
+        if constexpr (W == 0) {
+            x.am = A.minimum(b), x.ndm = A.neg_dmin(b);
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                x.bm[n] = *reinterpret_cast<const v4h *>(tp[n] + (long long)b * B_TILE + min_lane(lane, th[n]));
+        }
+    };
+    auto compute = [&](const Step &x) {
+        const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const float d8[4] = {x.e[n].x, x.e[n].y, x.e[n].z, x.e[n].w};
+            float s[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] = __fmul_rn(x.d, d8[i]);
+#pragma unroll
+            for (int l = 0; l < NL; ++l)
+                fold4(acc[l][n], s, __builtin_amdgcn_mfma_f32_16x16x32_f16(x.b[l][n], x.a[l], zero, 0, 0, 0));
+            if constexpr (W == 0) {
+                float m[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) m[i] = __fmul_rn(x.ndm, d8[i]);
+                fold4(acc[2][n], m, __builtin_amdgcn_mfma_f32_16x16x16f16(x.bm[n], x.am, zero, 0, 0, 0));
+            }
+        }
+    };
+    Step sa, sb;
+    load(0, sa);
+    for (int b = 0; b < nb; b += 2) {
+        load(b + 1 < nb ? b + 1 : b, sb);
+        compute(sa);
+        if (b + 1 >= nb) break;
+        load(b + 2 < nb ? b + 2 : b + 1, sa);
+        compute(sb);
+    }
+}
+
+template <int NT>
+__global__ void __launch_bounds__(64 * GS_WAVES) k_kq_gemm_split(GemmArgs g) {
+    __shared__ __align__(16) float s_ch[9][NT][4][64];
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const MatGemm &M = g.mat[blockIdx.y];
+    const int n16 = (M.rows + 15) / 16, tg = ((g.n_tokens + 15) / 16 + NT - 1) / NT;
+    const int r16 = (int)blockIdx.x / tg, tt0 = ((int)blockIdx.x - r16 * tg) * NT;
+    if (r16 >= n16) return;
+    const RowSrc A(M.a, r16 >> 1, r16 & 1, g.nb, lane);
+    float acc[3][NT][4];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[c][n][i] = 0.0f;
+    if (wid == 0) gs_chains<NT, 0>(A, g, tt0, lane, acc);
+    else if (wid == 1) gs_chains<NT, 1>(A, g, tt0, lane, acc);
+    else gs_chains<NT, 2>(A, g, tt0, lane, acc);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int c = wid == 0 ? (k == 2 ? 8 : k) : 3 * wid - 1 + k;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s_ch[c][n][i][lane] = acc[k][n][i];
+    }
+    __syncthreads();
+    // result = minimum chain + lane chains 0..7 (q8_k.rs:320-326)
+    for (int o = threadIdx.x; o < NT * 256; o += 64 * GS_WAVES) {
+        const int n = o >> 8, i = (o >> 6) & 3, l = o & 63;
+        float v = s_ch[8][n][i][l];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) v = __fadd_rn(v, s_ch[c][n][i][l]);
+        const int t = 16 * (tt0 + n) + 4 * (l >> 4) + i, row = 16 * r16 + (l & 15);
+        if (t < g.n_tokens && row < M.rows) M.y[(long long)t * M.ldy + row] = v;
     }
 }
 
@@ -793,41 +863,65 @@ hipError_t launch_prep_b(const uint8_t *q8, int n_tokens, int nb, uint8_t *b, hi
     return hipGetLastError();
 }
 
-template <int MODE>
-static hipError_t gemm_mode(const GemmArgs &g, hipStream_t s) {
+template <int NT>
+static hipError_t gemm_split(const GemmArgs &g, int rows, hipStream_t s) {
+    const int grid = cdiv(rows, 16) * cdiv(cdiv(g.n_tokens, 16), NT);
+    hipLaunchKernelGGL((k_kq_gemm_split<NT>), dim3(grid, g.n_mat), dim3(64 * GS_WAVES), 0, s, g);
+    return hipGetLastError();
+}
+
+static hipError_t gemm_2x2(const GemmArgs &g, int rows, hipStream_t s) {
     const int lds = (int)sizeof(GemmLDS);
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_kq_gemm<MODE>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_kq_gemm_2x2), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return e;
-    int rows = 0;
-    for (int i = 0; i < g.n_mat; ++i) rows = g.mat[i].rows > rows ? g.mat[i].rows : rows;
     const int grid = cdiv(cdiv(rows, 32), RG) * cdiv(cdiv(g.n_tokens, 32), TG);
-    hipLaunchKernelGGL((k_kq_gemm<MODE>), dim3(grid, g.n_mat), dim3(64 * NW), lds, s, g);
+    hipLaunchKernelGGL(k_kq_gemm_2x2, dim3(grid, g.n_mat), dim3(64 * NW), lds, s, g);
     return hipGetLastError();
 }
 
-template <int RG_, int TG_>
-static hipError_t gemm_p3(const GemmArgs &g, hipStream_t s) {
-    using S = P3<RG_, TG_>;
-    int rows = 0;
-    for (int i = 0; i < g.n_mat; ++i) rows = g.mat[i].rows > rows ? g.mat[i].rows : rows;
-    const int grid = cdiv(cdiv(rows, 32), S::RG) * cdiv(cdiv(g.n_tokens, 32), S::TG);
-    hipLaunchKernelGGL((k_kq_gemm3<RG_, TG_>), dim3(grid, g.n_mat), dim3(64 * P3_WAVES), 0, s, g);
-    return hipGetLastError();
+// The forms' times on Q5_K rows of 4096 (1024 .. 16384 rows, 16 .. 512 tokens)
+// beyond about 7.6 us that all share, in ns; every form's time goes with K.
+//   split, NT = 1, 2, 3, 4: 19, 22, 30, 35 per workgroup from 256 on (4096 rows,
+//     48 / 64 / 96 / 128 tokens with the best NT: 18.9 / 19.6 / 22.2 / 25.2 us in
+//     all); with NT = 4 (190 VGPRs) workgroups come in rounds of 512 (512: 25.2
+//     us, 768: 38.8, 1024: 42).
+//   2 x 2: 24400 per round of 256 workgroups (192: 33 us, 384: 57).
+//   LDS: 33000 for the first 256 workgroups, 26000 for each 256 more (256: 41 us,
+//     384: 61, 768: 103).
+static long long split_ns(int rows, int n_tokens, int nt) {
+    static const int per[4] = {19, 22, 30, 35};
+    long long w = (long long)cdiv(rows, 16) * cdiv(cdiv(n_tokens, 16), nt);
+    if (nt == 4) w = 512LL * cdiv(w, 512);
+    return per[nt - 1] * (w > 256 ? w : 256);
 }
 
-// shape: 0 default (three passes from 97 tokens: four token tiles per
-// workgroup; the 2 x 2 schedule staged through registers below), 1 the 2 x 2
-// schedule with direct buffer-to-LDS staging, 2 the 2 x 2 schedule staged
-// through registers, 3 three passes.
+// shape: 0 default, 1 the split form, 2 the 2 x 2 form, 3 the LDS form.
 hipError_t launch_kq_gemm(const GemmArgs &g, hipStream_t s) {
     if (g.n_mat < 1 || g.n_mat > GEMM_MAX_MATS || g.n_tokens < 1 || g.nb < 1 || g.nb > 64) return hipErrorInvalidValue;
-    switch (g.shape) {
-    case 1: return gemm_mode<1>(g, s);
-    case 2: return gemm_mode<0>(g, s);
-    case 3: return gemm_p3<3, 4>(g, s);
-    default: return g.n_tokens > 96 ? gemm_p3<3, 4>(g, s) : gemm_mode<0>(g, s);
+    int rows = 0;
+    for (int i = 0; i < g.n_mat; ++i) rows = g.mat[i].rows > rows ? g.mat[i].rows : rows;
+    int nt = 1;
+    for (int n = 2; n <= 4; ++n)
+        if (split_ns(rows, g.n_tokens, n) < split_ns(rows, g.n_tokens, nt)) nt = n;
+    const long long lds_wgs = (long long)cdiv(rows, 128) * cdiv(g.n_tokens, 64);
+    int shape = g.shape;
+    if (shape == 0) {
+        const long long t1 = split_ns(rows, g.n_tokens, nt);
+        const long long t2 = 24400LL * cdiv((long long)cdiv(rows, 64) * cdiv(g.n_tokens, 64), 256);
+        const long long t3 = 7000 + 26000LL * cdiv(lds_wgs, 256);
+        shape = t1 <= t2 && t1 <= t3 ? 1 : t2 <= t3 ? 2 : 3;
     }
+    if (shape == 1) {
+        switch (nt) {
+        case 1: return gemm_split<1>(g, rows, s);
+        case 2: return gemm_split<2>(g, rows, s);
+        case 3: return gemm_split<3>(g, rows, s);
+        default: return gemm_split<4>(g, rows, s);
+        }
+    }
+    if (shape == 2) return gemm_2x2(g, rows, s);
+    hipLaunchKernelGGL(k_kq_gemm_lds, dim3((int)lds_wgs, g.n_mat), dim3(64 * GL_WAVES), 0, s, g);
+    return hipGetLastError();
 }
 
 }  // namespace lbh

@@ -17,7 +17,7 @@ struct lbh_ctx {
     lbh::DevStatus *status;        // device
     lbh::DevStatus *status_host;   // pinned mirror
     lbh::GemvTuning tuning;
-    int gemm_shape;           // K-quant GEMM staging (0: registers, two blocks ahead; 1: direct to LDS)
+    int gemm_shape;           // K-quant GEMM schedule (LBH_TUNE_GEMM_SHAPE; 0: by rows and tokens)
     uint8_t *scratch;         // this device's copy of the library's static scratch array (lbh_api.hip)
 };
 

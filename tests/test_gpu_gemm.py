@@ -138,3 +138,22 @@ def test_gemm_config5_full_shape_bit_exact(be, oracle):
     want = oracle_gemm(oracle, Q5_K, w, rows, k, q8)
     bad = np.argwhere(got.view(np.uint32) != want.view(np.uint32))
     assert bad.size == 0, f"{len(bad)} mismatches, first {bad[:4].tolist()}"
+
+
+@pytest.mark.parametrize("ty,rows,k,n", [(Q4_K, 1, 256, 1), (Q5_K, 17, 768, 16), (Q4_K, 47, 512, 17), (Q5_K, 33, 1280, 49),
+                                         (Q4_K, 129, 256, 65), (Q5_K, 160, 768, 97), (Q4_K, 255, 1280, 64),
+                                         (Q5_K, 4081, 256, 17), (Q4_K, 4081, 256, 33), (Q5_K, 4081, 256, 115)])
+def test_gemm_forms_at_the_edges(be, oracle, ty, rows, k, n):
+    # Row tiles of 16 and groups of 128, token tiles of 16 and groups of 64,
+    # odd and single block counts, one to four token tiles of the split form
+    # (4081 rows: two, three, four), in every form: each value bit for bit.
+    w = synth.random_matrix(ty, rows, k, seed=rows)
+    q8 = q8_rows(oracle, np.random.default_rng(rows).standard_normal((n, k)).astype(np.float32))
+    want = oracle_gemm(oracle, ty, w, rows, k, q8)
+    for shape in (0, 1, 2, 3):
+        be.set_tuning(be.TUNE_GEMM_SHAPE, shape)
+        try:
+            got = run_gemm(be, ty, w, rows, k, q8)
+        finally:
+            be.set_tuning(be.TUNE_GEMM_SHAPE, 0)
+        assert _same(got, want), shape
