@@ -120,28 +120,36 @@ __device__ __forceinline__ uint32_t iq2s_qh_dword(uint32_t o) {
     return r;
 }
 
+// A unit's d and its N dwords: halfword loads from an even address (every block
+// of a buffer that starts even), else byte loads.
+template <int N>
+__device__ __forceinline__ void unit_dwords(const uint8_t *g, uint32_t (&v)[N], uint32_t &d) {
+    if ((reinterpret_cast<uintptr_t>(g) & 1u) == 0) {
+        const uint16_t *h = reinterpret_cast<const uint16_t *>(g);
+        d = h[0];
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = (uint32_t)h[1 + 2 * i] | ((uint32_t)h[2 + 2 * i] << 16);
+    } else {
+        d = (uint32_t)g[0] | ((uint32_t)g[1] << 8);
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            v[i] = (uint32_t)g[2 + 4 * i] | ((uint32_t)g[3 + 4 * i] << 8) | ((uint32_t)g[4 + 4 * i] << 16) |
+                   ((uint32_t)g[5 + 4 * i] << 24);
+    }
+}
+
 // One unit's GGML bytes `g` to the device layout (IQ2_S through its bit
-// encoding, iq2s_encode), and back.
+// encoding, iq2s_encode), and back.  The types that experts stream in go by
+// dwords and whole chunks: byte stores held an IQ3_S matrix of 4096 x 1536 (2.7
+// MB) at 25.7 us per k_repack, now 4.6 (an expert's record takes 127 us on its
+// way from the host).
 template <int TY>
 __device__ __forceinline__ void unit_to_device(const uint8_t *g, uint8_t *dst, long long U, long long u) {
     constexpr int BB = layout_of(TY).block_bytes;
     if constexpr (TY == T_IQ2_S) {
-        // d, then 20 dwords (qs 0-7, signs 8-15, qh 16-17, scales 18-19):
-        // halfword loads from an even address (every block of a buffer that
-        // starts even), else byte loads
+        // d, then 20 dwords (qs 0-7, signs 8-15, qh 16-17, scales 18-19)
         uint32_t v[20], d;
-        if ((reinterpret_cast<uintptr_t>(g) & 1u) == 0) {
-            const uint16_t *h = reinterpret_cast<const uint16_t *>(g);
-            d = h[0];
-#pragma unroll
-            for (int i = 0; i < 20; ++i) v[i] = (uint32_t)h[1 + 2 * i] | ((uint32_t)h[2 + 2 * i] << 16);
-        } else {
-            d = (uint32_t)g[0] | ((uint32_t)g[1] << 8);
-#pragma unroll
-            for (int i = 0; i < 20; ++i)
-                v[i] = (uint32_t)g[2 + 4 * i] | ((uint32_t)g[3 + 4 * i] << 8) | ((uint32_t)g[4 + 4 * i] << 16) |
-                       ((uint32_t)g[5 + 4 * i] << 24);
-        }
+        unit_dwords(g, v, d);
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = ((v[i] & 0x1f1f1f1fu) << 3) | ((v[i] >> 5) & 0x07070707u);
 #pragma unroll
@@ -152,6 +160,20 @@ __device__ __forceinline__ void unit_to_device(const uint8_t *g, uint8_t *dst, l
 #pragma unroll
         for (int k = 0; k < 5; ++k) c[k * cs] = make_uint4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
         reinterpret_cast<uint16_t *>(dst + 5 * U * 16)[u] = (uint16_t)d;
+    } else if constexpr (TY == T_IQ3_S) {
+        // d, then 27 dwords (qs 0-15, qh 16-17, signs 18-25, scales 26), loaded
+        // as above.
+        uint32_t v[27], d;
+        unit_dwords(g, v, d);
+        uint4 *c = reinterpret_cast<uint4 *>(dst + u * 16);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            const int i = k < 4 ? 4 * k : 4 * k + 2;
+            c[k * U] = make_uint4(v[i], v[i + 1], v[i + 2], v[i + 3]);
+        }
+        uint32_t *t = reinterpret_cast<uint32_t *>(dst + 6 * U * 16) + 3 * u;
+        t[0] = v[16], t[1] = v[17], t[2] = v[26];
+        reinterpret_cast<uint16_t *>(dst + 6 * U * 16 + 12 * U)[u] = (uint16_t)d;
     } else {
         for (int p = 0; p < BB; ++p) dst[dev_offset(TY, U, u, p)] = g[p];
     }
