@@ -1233,7 +1233,9 @@ __device__ __forceinline__ void mx_prologue(uint8_t *tab, float *s_d8, int n, in
 // The shared expert's K-quant rows in a stage launch (lbh_kt.h): workgroup wg of
 // kt_wgs(): 64 rows (one 16-row tile per wave) of matrix m against KT_NT token
 // tiles; the token groups of a row quad are neighbours, so its weights are
-// fetched once.
+// fetched once.  One tile a wave: two hold registers that the routed streams of
+// the launch then lack (steps of 5 / 64 / 256 tokens: 103 / 246 / 502 us with
+// one, 114 / 260 / 518 with two).
 constexpr int KT_NT = 1;
 __host__ __device__ inline int kt_groups(int n_tokens) { return ((n_tokens + 15) / 16 + KT_NT - 1) / KT_NT; }
 template <int TY>

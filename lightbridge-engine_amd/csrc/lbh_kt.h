@@ -21,8 +21,7 @@
 // (d, dmin).  The tokens come as f16 operands (kt_store_block) from L1 / L2.
 //
 // What bounds it: VALU issue, 80 instructions per token tile (16 per f32 chain
-// step pair and the scales) and about 80 for the weights of a step, hence
-// several token tiles per wave where the batch has them.
+// step pair and the scales) and about 80 for the weights of a step.
 #pragma once
 #include "lbh_dev.h"
 
