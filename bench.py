@@ -58,7 +58,7 @@ COLD_COPIES = 8
 # Bytes per launch (read from beyond L2 + written) measured with rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE over `bench.py --pmc-workloads`, each scaled by the same counter's reading for a plain
 # copy of known size (profiles/pmc_hot_kernels_traffic_and_valu.md).
-MEASURED_TRAFFIC = {"gate": 2363569 + 6144, "down": 2987388 + 19648, "prefill": 193234918 + 25644960}
+MEASURED_TRAFFIC = {"gate": 2363569 + 6144, "down": 2987388 + 19648, "prefill": 207200000 + 25166000}
 
 
 def parse():
@@ -525,10 +525,9 @@ def bench_batch(args, be, timer, torch, np, synth, state):
            "distinct_experts_hit_per_step": hits,
            "algorithmic_bytes_per_step": int(bytes_step),
            "GB/s": round(bytes_step / us / 1e3, 1), "roofline_frac": round(bytes_step / us / 1e3 / HBM_PEAK_GBS, 4),
-           "note": "the 33.5 MB shared expert is read once per step (K-quant GEMM on the f16 matrix cores); routed "
-                   "experts once per chunk of up to 16 tokens, chunks of 4+ tokens on the f16 matrix cores (exact "
-                   "integer block sums), smaller ones on the VALU integer dots; us_per_step is timed with a second "
-                   "copy of every routed expert's matrices with the 16 rows of each block adjacent (read by the "
+           "note": "the 33.5 MB shared expert is read once per step (f16 matrix cores, in the routed launches); routed "
+                   "experts once per chunk of up to 16 tokens on the int8 matrix cores (exact integer block "
+                   "sums); us_per_step is timed with a second copy of every routed expert's matrices with the 16 rows of each block adjacent (read by the "
                    "matrix-core streams only; tile_copy_hbm_bytes of HBM), us_per_step_without_tile_copies on the "
                    "matrices as uploaded"}
     check = dict(ids=ids_h[0].copy(), coefs=coefs[0].cpu().numpy(), xs=xs[0].cpu().numpy(), ys=ys[0].cpu().numpy())
@@ -737,7 +736,7 @@ def bench_prefill(args, be, timer, torch, np, synth):
     tops = PF_OPS / us / 1e6
     footprint = ms[0].device_bytes
     res = {"workload": "configs[4]: prefill 512 tokens, Q8_K activations [512 x 4096] x Q5_K [12288 x 4096] -> f32 "
-                       "[512 x 12288], f16 MFMA (v_mfma_f32_32x32x16_f16) on integer operands: exact "
+                       "[512 x 12288], f16 MFMA (v_mfma_f32_16x16x32_f16) on integer operands: exact "
                        "per-(block, lane residue) sums",
            "us_per_step": round(us, 2), "calls_timed": reps * copies, "warmup_calls": 20 * copies,
            "per_replay_spread": spread, "dot_TOPS": round(tops, 2),
