@@ -883,7 +883,7 @@ namespace {
 // down rows per workgroup (1, 5, 16, 64 and 256 tokens; 128 and 256 gate/up rows
 // 3-25% slower, 128 and 512 down rows 0-4%).  The VALU streams alone do best with
 // chunks of 8.
-constexpr int MX_MIN_DEFAULT = 1;
+constexpr int MX_MIN_DEFAULT = 1;   // also the default of lbhip's MoeLayer.set_batch_engine
 void set_batch_defaults(lbh_moe *m, int mx_min) {
     m->mx_min = mx_min;
     m->mx_rows_gu = 64, m->mx_rows_d = 256;

@@ -528,10 +528,10 @@ class MoeLayer:
         if st:
             raise KernelError(LbhError(status=st))
 
-    def set_batch_engine(self, mx_min_tokens: int = 4, mx_rows_gate_up: int = 0, mx_rows_down: int = 0) -> None:
+    def set_batch_engine(self, mx_min_tokens: int = 1, mx_rows_gate_up: int = 0, mx_rows_down: int = 0) -> None:
         """Batched IQ chunks of at least mx_min_tokens tokens on the matrix cores, the
         rest on the VALU dot4 path (0: all on the VALU); resets the batch launch shapes
-        to their defaults."""
+        to their defaults.  Without arguments: the engine of a new layer."""
         st = lib().lbh_moe_set_batch_engine(self.handle, mx_min_tokens, mx_rows_gate_up, mx_rows_down)
         if st:
             raise KernelError(LbhError(status=st))

@@ -60,3 +60,15 @@ def test_noalloc_scratch_limit_is_the_documented_token_count():
     for k, n in ((4096, 928), (7168, 544)):
         assert hb.gemm_workspace_bytes(n, k) <= limit < hb.gemm_workspace_bytes(n + 1, k)
         assert f"{n} tokens at k = {k}" in text
+
+
+def test_default_batch_engine_is_the_library_s():
+    """MoeLayer.set_batch_engine() without arguments sets the engine of a new
+    layer: the matrix-core threshold that the header and the library state."""
+    import inspect
+    import lbhip
+    got = inspect.signature(lbhip.MoeLayer.set_batch_engine).parameters["mx_min_tokens"].default
+    header = (ROOT / "include" / "lightbridge_hip.h").read_text()
+    source = (ROOT / "lightbridge-engine_amd" / "csrc" / "lbh_api.hip").read_text()
+    assert got == int(re.search(r"\(1\.\.16; (\d+) until this is called\)", header).group(1))
+    assert got == int(re.search(r"MX_MIN_DEFAULT = (\d+);", source).group(1))
