@@ -1367,6 +1367,8 @@ __global__ void __launch_bounds__(MX_THREADS) k_kt_rows(const uint8_t *w0, const
 // Workgroup (1024 rows, token): the token's pairs are scalar reads, and the
 // rows of eight experts are in flight at once (64 / 256 tokens: 9.0 / 20 -> 5.0 /
 // 9.0 us against one row a thread with each expert's loads behind the last's).
+// y is the caller's: floats, at any multiple of four bytes.
+typedef float y_f4 __attribute__((ext_vector_type(4), aligned(4)));
 __global__ void __launch_bounds__(MB_THREADS) k_mb_combine(BatchArgs a) {
     if (a.plan[1]) return;
     const int t = blockIdx.y, r = (int)(blockIdx.x * MB_THREADS + threadIdx.x) * 4;
@@ -1374,7 +1376,10 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_combine(BatchArgs a) {
     const long long at = (long long)t * a.hidden + r;
     float4 sh = make_float4(0.0f, 0.0f, 0.0f, 0.0f), y = sh, acc = sh;
     if (a.has_shared) sh = *reinterpret_cast<const float4 *>(a.d_s + at);
-    if (a.residual) y = *reinterpret_cast<const float4 *>(a.y + at);
+    if (a.residual) {
+        const y_f4 v = *reinterpret_cast<const y_f4 *>(a.y + at);
+        y = make_float4(v.x, v.y, v.z, v.w);
+    }
     for (int s0 = 0; s0 < a.top_k; s0 += 8) {
         float4 d[8];
 #pragma unroll
@@ -1398,7 +1403,7 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_combine(BatchArgs a) {
         acc.w = __fadd_rn(acc.w, __fmul_rn(1.0f, sh.w));
     }
     if (a.residual) acc = make_float4(__fadd_rn(y.x, acc.x), __fadd_rn(y.y, acc.y), __fadd_rn(y.z, acc.z), __fadd_rn(y.w, acc.w));
-    *reinterpret_cast<float4 *>(a.y + at) = acc;
+    *reinterpret_cast<y_f4 *>(a.y + at) = y_f4{acc.x, acc.y, acc.z, acc.w};
 }
 
 // Top-k selection of every token of a batch from finished logits, one wave per token.

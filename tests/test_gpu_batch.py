@@ -218,6 +218,30 @@ def test_batch_capacity_is_enforced(be, oracle, small):
     assert e.value.variant == "ScratchTooSmall"
 
 
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_batch_output_at_any_float_address(be, oracle, small, offset):
+    """y and hidden are the caller's floats: views that start 4, 8 or 12 bytes
+    off a 16-byte boundary, with the floats around them left alone."""
+    _, ids, coefs = zipf_routing(oracle, 9, 12, 4, seed=19)
+    xs = np.random.default_rng(20).standard_normal((9, 512)).astype(np.float32)
+    want = oracle_batch(oracle, small, ids, coefs, xs)
+    start = np.random.default_rng(21).standard_normal(9 * 512 + 4).astype(np.float32)
+    ids_d, coefs_d = dev(ids.view(np.int32)), dev(coefs)
+    for residual in (False, True):
+        buf = dev(start)
+        y = buf[offset:offset + 9 * 512].view(9, 512)
+        assert y.data_ptr() % 16 == 4 * offset
+        (be.moe_forward_batch_residual if residual else be.moe_forward_batch)(small.moe, ids_d, coefs_d, dev(xs), y)
+        got = host(buf)
+        assert _same(got[:offset], start[:offset]) and _same(got[offset + 9 * 512:], start[offset + 9 * 512:])
+        for t in range(9):
+            w = want[t]
+            if residual:
+                w = start[offset + 512 * t:offset + 512 * (t + 1)].copy()
+                oracle.residual_add_in_place(w, want[t])
+            assert _same(got[offset + 512 * t:offset + 512 * (t + 1)], w), f"token {t}, residual {residual}"
+
+
 def test_batch_async_invalid_device_ids_leave_the_output_unchanged(be, oracle, small):
     ids = torch.tensor([[0, 3], [2, 12]], dtype=torch.int32, device="cuda")     # 12 >= n_experts
     coefs = torch.full((2, 2), 0.5, dtype=torch.float32, device="cuda")
