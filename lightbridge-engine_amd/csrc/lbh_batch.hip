@@ -808,7 +808,7 @@ constexpr int MX_MAX_NB = 64;
 
 // IQ2_S scaled weights by scale nibble n: bytes 0-2 of {lo+, lo-, hi+, hi-} are
 // the split +-m (1 + 2n) = 256 hi + lo (lo signed) of m = 8, 25, 43.
-struct MxProducts {
+struct alignas(16) MxProducts {
     uint32_t v[16][4];
     constexpr MxProducts() : v{} {
         const int mag[3] = {8, 25, 43};
@@ -839,6 +839,7 @@ __device__ __forceinline__ void mx_fill(uint8_t *tab) {
     uint4 *o = reinterpret_cast<uint4 *>(tab);
 #pragma unroll
     for (int i = 0; i < MxTab<TY>::GRID / 16 / MX_THREADS; ++i) o[threadIdx.x + i * MX_THREADS] = g[threadIdx.x + i * MX_THREADS];
+    static_assert(alignof(MxProducts) % 16 == 0, "read as uint4");
     if (TY == T_IQ2_S && threadIdx.x < 16)
         o[MxTab<TY>::GRID / 16 + threadIdx.x] = reinterpret_cast<const uint4 *>(&c_mx_products.v[0][0])[threadIdx.x];
 }

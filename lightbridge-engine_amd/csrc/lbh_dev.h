@@ -421,8 +421,9 @@ __device__ __forceinline__ void load_act_res(const uint8_t *blk, const uint8_t *
 
 // Each translation unit holds its own copy (no relocatable device code).
 #include "lbh_iq_grids.inc"
-static __constant__ uint64_t c_iq2s_grid[1024] = {LBH_IQ2S_GRID_VALUES};
-static __constant__ uint32_t c_iq3s_grid[512] = {LBH_IQ3S_GRID_VALUES};
+// Tables that kernels copy in 16-byte pieces are aligned so.
+static __constant__ __align__(16) uint64_t c_iq2s_grid[1024] = {LBH_IQ2S_GRID_VALUES};
+static __constant__ __align__(16) uint32_t c_iq3s_grid[512] = {LBH_IQ3S_GRID_VALUES};
 
 // IQ3S: 512 (magnitude, negation) pairs of 8 bytes at iq3_pair_offset, then
 // the 256 sign-byte entries (iq3_sign_entry) at IQ3_SIGN_OFF.  The pair order
@@ -561,7 +562,7 @@ __device__ __forceinline__ uint32_t iq3_signed(uint2 pr, uint32_t sel) { return 
 
 // The LDS images of both tables (GridLDS layout), built at compile time from
 // the codebooks: a workgroup's fill is a plain copy with 16-byte loads.
-struct GridImages {
+struct alignas(16) GridImages {
     uint32_t iq2s[2 * 1024];
     uint32_t iq3s[2 * (512 + 256)];
     constexpr GridImages() : iq2s{}, iq3s{} {
@@ -590,7 +591,7 @@ struct GridImages {
 static __constant__ GridImages c_grid_images = GridImages();
 
 // The signed IQ3S table image (iq3_signed_offset layout).
-struct Iq3SignedImage {
+struct alignas(16) Iq3SignedImage {
     uint32_t w[8192];
     constexpr Iq3SignedImage() : w{} {
         const uint32_t g3[512] = {LBH_IQ3S_GRID_VALUES};
@@ -609,6 +610,7 @@ static __constant__ Iq3SignedImage c_iq3s_signed = Iq3SignedImage();
 
 template <int TY>
 __device__ __forceinline__ const uint4 *grid_image() {
+    static_assert(alignof(GridImages) % 16 == 0 && alignof(Iq3SignedImage) % 16 == 0, "read as uint4");
     if constexpr (TY == T_IQ3S_SGN) return reinterpret_cast<const uint4 *>(c_iq3s_signed.w);
     return reinterpret_cast<const uint4 *>(TY == T_IQ2_S ? c_grid_images.iq2s : c_grid_images.iq3s);
 }

@@ -290,6 +290,7 @@ __global__ void __launch_bounds__(256) k_gemv_dequant(DequantArgs p) {
     // the codebook to LDS: gathered from global memory its latency was the step's
     __shared__ __align__(16) uint32_t s_grid[TY == T_IQ2_S ? 2048 : TY == T_IQ3_S ? 512 : 4];
     if constexpr (TY == T_IQ2_S || TY == T_IQ3_S) {
+        static_assert(__alignof__(c_iq2s_grid) % 16 == 0 && __alignof__(c_iq3s_grid) % 16 == 0, "read as uint4");
         const uint4 *src = reinterpret_cast<const uint4 *>(TY == T_IQ2_S ? (const void *)c_iq2s_grid : (const void *)c_iq3s_grid);
         for (int i = tid; i < (int)(sizeof(s_grid) / 16); i += 256) reinterpret_cast<uint4 *>(s_grid)[i] = src[i];
         __syncthreads();
