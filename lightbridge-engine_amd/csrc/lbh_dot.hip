@@ -262,8 +262,11 @@ __device__ __forceinline__ void dequant_group(const DqRaw<TY> &o, int sub, const
 // block ahead.  What bounds it: the dependent f32 adds, 256 a block at 8 cycles
 // at best and 11.6 as measured (Q4_K 4096x4096: 36.2 -> 22.9 us with the next
 // block's bytes in flight, the codebooks in LDS and one wait per 64 adds).
-template <int TY>
-__global__ void __launch_bounds__(256) k_gemv_dequant(DequantArgs p) {
+// THREE (launch_gemv_dequant): three workgroups per CU instead of two, with half
+// the products ahead of the adds (152 registers for 214) and the codebook left in
+// global memory (50 KB of LDS for 58).
+template <int TY, bool THREE = false>
+__global__ void __launch_bounds__(256, THREE ? 3 : 2) k_gemv_dequant(DequantArgs p) {
     __shared__ __align__(16) float s_prod[2][DQ_ROWS * DQ_STRIDE];
     // A non-finite input or (accumulating) destination: the reference rejects
     // the call before it writes (gemv.rs:126-127, :195-211).
@@ -288,8 +291,11 @@ __global__ void __launch_bounds__(256) k_gemv_dequant(DequantArgs p) {
     };
     if (tid >= 64) load(0, ra, xa);
     // the codebook to LDS: gathered from global memory its latency was the step's
-    __shared__ __align__(16) uint32_t s_grid[TY == T_IQ2_S ? 2048 : TY == T_IQ3_S ? 512 : 4];
-    if constexpr (TY == T_IQ2_S || TY == T_IQ3_S) {
+    __shared__ __align__(16) uint32_t s_grid[THREE ? 4 : TY == T_IQ2_S ? 2048 : TY == T_IQ3_S ? 512 : 4];
+    const void *grid = s_grid;
+    if constexpr (THREE) {
+        grid = TY == T_IQ2_S ? (const void *)c_iq2s_grid : (const void *)c_iq3s_grid;
+    } else if constexpr (TY == T_IQ2_S || TY == T_IQ3_S) {
         static_assert(__alignof__(c_iq2s_grid) % 16 == 0 && __alignof__(c_iq3s_grid) % 16 == 0, "read as uint4");
         const uint4 *src = reinterpret_cast<const uint4 *>(TY == T_IQ2_S ? (const void *)c_iq2s_grid : (const void *)c_iq3s_grid);
         for (int i = tid; i < (int)(sizeof(s_grid) / 16); i += 256) reinterpret_cast<uint4 *>(s_grid)[i] = src[i];
@@ -304,30 +310,31 @@ __global__ void __launch_bounds__(256) k_gemv_dequant(DequantArgs p) {
                 float x[32], out[32];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) x[4 * i] = xv[i].x, x[4 * i + 1] = xv[i].y, x[4 * i + 2] = xv[i].z, x[4 * i + 3] = xv[i].w;
-                dequant_group<TY>(raw, sub, s_grid, x, out);
+                dequant_group<TY>(raw, sub, grid, x, out);
                 float4 *dst = reinterpret_cast<float4 *>(&s_prod[s & 1][slot * DQ_STRIDE + 32 * sub]);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) dst[i] = make_float4(out[4 * i], out[4 * i + 1], out[4 * i + 2], out[4 * i + 3]);
             }
         } else if (s > 0 && tid < DQ_ROWS) {
-            // The chain: batches of 64 products, one wait per batch, the next
+            // The chain: batches of 64 (THREE: 32) products, one wait per batch, the next
             // batch's reads issued ahead of this batch's adds (a read and a wait
             // between every four adds ran at 13.4 cycles per add).
             const float4 *src = reinterpret_cast<const float4 *>(&s_prod[(s - 1) & 1][tid * DQ_STRIDE]);
-            float4 v[2][16];
+            constexpr int N = THREE ? 8 : 16;
+            float4 v[2][N];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[0][i] = src[i];
+            for (int i = 0; i < N; ++i) v[0][i] = src[i];
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
+            for (int b = 0; b < 64 / N; ++b) {
                 __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
                 __builtin_amdgcn_sched_barrier(0);
-                if (b < 3) {
+                if (b < 64 / N - 1) {
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) v[(b + 1) & 1][i] = src[16 * (b + 1) + i];
+                    for (int i = 0; i < N; ++i) v[(b + 1) & 1][i] = src[N * (b + 1) + i];
                 }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
+                for (int i = 0; i < N; ++i) {
                     const float4 f = v[b & 1][i];
                     sum = __fadd_rn(sum, f.x);
                     sum = __fadd_rn(sum, f.y);
@@ -385,9 +392,26 @@ hipError_t launch_gemv_dequant(const MatView &m, const float *x, float *y, float
     if (m.rows < 1 || m.nb < 1) return hipErrorInvalidValue;
     DequantArgs a{m, x, y, coef, accumulate, st};
     const int grid = (m.rows + DQ_ROWS - 1) / DQ_ROWS;
+    // Codebook rows of few blocks: what a workgroup starts with (first bytes,
+    // codebook) is not spread over many steps, so past two workgroups on each of
+    // the 256 CUs a third one there counts for more than a faster step.  16384
+    // rows x 256, two / three per CU: IQ2_S 9.6 / 8.0 us, IQ3_S 8.6 / 7.9; 65536
+    // rows x 1024: 56.0 / 54.7 and 56.0 / 55.7; x 1536 IQ3_S 77.5 / 80.3; 4096
+    // rows x 1024: 8.6 / 10.3 and 8.7 / 9.7.
+    const bool three = m.nb <= 4 && grid > 512;
     switch (m.type) {
-    case T_IQ2_S: hipLaunchKernelGGL(k_gemv_dequant<T_IQ2_S>, dim3(grid), dim3(256), 0, s, a); break;
-    case T_IQ3_S: hipLaunchKernelGGL(k_gemv_dequant<T_IQ3_S>, dim3(grid), dim3(256), 0, s, a); break;
+    case T_IQ2_S:
+        if (three)
+            hipLaunchKernelGGL((k_gemv_dequant<T_IQ2_S, true>), dim3(grid), dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL(k_gemv_dequant<T_IQ2_S>, dim3(grid), dim3(256), 0, s, a);
+        break;
+    case T_IQ3_S:
+        if (three)
+            hipLaunchKernelGGL((k_gemv_dequant<T_IQ3_S, true>), dim3(grid), dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL(k_gemv_dequant<T_IQ3_S>, dim3(grid), dim3(256), 0, s, a);
+        break;
     case T_Q4_K: hipLaunchKernelGGL(k_gemv_dequant<T_Q4_K>, dim3(grid), dim3(256), 0, s, a); break;
     case T_Q5_K: hipLaunchKernelGGL(k_gemv_dequant<T_Q5_K>, dim3(grid), dim3(256), 0, s, a); break;
     default: return hipErrorInvalidValue;

@@ -258,7 +258,10 @@ def _dequant_want(oracle, ty, rows, k, w, x):
 
 
 @pytest.mark.parametrize("ty,rows,k", [(Q4_K, 4096, 4096), (IQ2_S, 1536, 4096), (IQ3_S, 4096, 1536),
-                                       (Q5_K, 301, 2048), (IQ2_S, 25, 256), (Q4_K, 49, 16384)])
+                                       (Q5_K, 301, 2048), (IQ2_S, 25, 256), (Q4_K, 49, 16384),
+                                       # about 512 workgroups of 24 rows and 4 blocks: the three-per-CU form's edges
+                                       (IQ2_S, 12288, 256), (IQ2_S, 12289, 256), (IQ2_S, 12311, 1024), (IQ3_S, 12289, 512),
+                                       (IQ3_S, 12312, 768), (IQ3_S, 12313, 1280)])
 def test_dequant_f32_bit_exact(be, oracle, ty, rows, k):
     w = synth.random_matrix(ty, rows, k, 61 + ty + rows)
     x = synth.random_activations(k, 62 + k)
