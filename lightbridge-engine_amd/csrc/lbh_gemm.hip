@@ -879,20 +879,36 @@ static hipError_t gemm_2x2(const GemmArgs &g, int rows, hipStream_t s) {
     return hipGetLastError();
 }
 
-// The forms' times on Q5_K rows of 4096 (1024 .. 16384 rows, 16 .. 512 tokens)
-// beyond about 7.6 us that all share, in ns; every form's time goes with K.
+// The forms' times on rows of 4096 beyond about 7.6 us that all share, in ns; they
+// go with K (256 .. 16384 measured).  Row operands in the 256 MB cache between L2
+// and HBM, as in a call repeated on one matrix (1024 .. 16384 rows, 16 .. 512
+// tokens):
 //   split, NT = 1, 2, 3, 4: 19, 22, 30, 35 per workgroup from 256 on (4096 rows,
 //     48 / 64 / 96 / 128 tokens with the best NT: 18.9 / 19.6 / 22.2 / 25.2 us in
 //     all); with NT = 4 (190 VGPRs) workgroups come in rounds of 512 (512: 25.2
 //     us, 768: 38.8, 1024: 42).
-//   2 x 2: 24400 per round of 256 workgroups (192: 33 us, 384: 57).
+//   2 x 2: 24400 per round of 256 workgroups, one per CU (192: 33 us, 384: 57).
 //   LDS: 33000 for the first 256 workgroups, 26000 for each 256 more (256: 41 us,
 //     384: 61, 768: 103).
-static long long split_ns(int rows, int n_tokens, int nt) {
-    static const int per[4] = {19, 22, 30, 35};
+// Beyond that cache the split form, whose waves load their own operands, loses
+// most: 24, 35, 43, 52 per workgroup, 2 x 2 28700 per round, LDS 48000 and 28000
+// for each 256 more (48 tokens, 12288 rows of 16384, 440 MB: 141 / 122 / 183 us;
+// 32 tokens, 16384 rows of 12288: 111 / 96 / 143; 48 tokens, 65536 rows of 4096:
+// 178 / 141 / 115).  The line: of matrices read from HBM one after the other, 147
+// MB (4096 rows of 16384) still has the cached times' order at every token count
+// and 110 MB (12288 of 4096) misses by 8% at 33 to 48 tokens only, 220 MB (12288
+// of 8192) by 12% there.
+struct FormTimes {
+    int split[4], round_2x2, lds0, lds;
+};
+static constexpr FormTimes KQ_CACHED = {{19, 22, 30, 35}, 24400, 7000, 26000};
+static constexpr FormTimes KQ_BEYOND = {{24, 35, 43, 52}, 28700, 20000, 28000};
+static constexpr size_t KQ_CACHED_BYTES = 192u << 20;
+
+static long long split_ns(const FormTimes &f, int rows, int n_tokens, int nt) {
     long long w = (long long)cdiv(rows, 16) * cdiv(cdiv(n_tokens, 16), nt);
     if (nt == 4) w = 512LL * cdiv(w, 512);
-    return per[nt - 1] * (w > 256 ? w : 256);
+    return f.split[nt - 1] * (w > 256 ? w : 256);
 }
 
 // shape: 0 default, 1 the split form, 2 the 2 x 2 form, 3 the LDS form.
@@ -900,15 +916,16 @@ hipError_t launch_kq_gemm(const GemmArgs &g, hipStream_t s) {
     if (g.n_mat < 1 || g.n_mat > GEMM_MAX_MATS || g.n_tokens < 1 || g.nb < 1 || g.nb > 64) return hipErrorInvalidValue;
     int rows = 0;
     for (int i = 0; i < g.n_mat; ++i) rows = g.mat[i].rows > rows ? g.mat[i].rows : rows;
+    const FormTimes &f = gemm_a_bytes(rows, g.nb) > KQ_CACHED_BYTES ? KQ_BEYOND : KQ_CACHED;
     int nt = 1;
     for (int n = 2; n <= 4; ++n)
-        if (split_ns(rows, g.n_tokens, n) < split_ns(rows, g.n_tokens, nt)) nt = n;
+        if (split_ns(f, rows, g.n_tokens, n) < split_ns(f, rows, g.n_tokens, nt)) nt = n;
     const long long lds_wgs = (long long)cdiv(rows, 128) * cdiv(g.n_tokens, 64);
     int shape = g.shape;
     if (shape == 0) {
-        const long long t1 = split_ns(rows, g.n_tokens, nt);
-        const long long t2 = 24400LL * cdiv((long long)cdiv(rows, 64) * cdiv(g.n_tokens, 64), 256);
-        const long long t3 = 7000 + 26000LL * cdiv(lds_wgs, 256);
+        const long long t1 = split_ns(f, rows, g.n_tokens, nt);
+        const long long t2 = (long long)f.round_2x2 * cdiv((long long)cdiv(rows, 64) * cdiv(g.n_tokens, 64), 256);
+        const long long t3 = f.lds0 + (long long)f.lds * cdiv(lds_wgs, 256);
         shape = t1 <= t2 && t1 <= t3 ? 1 : t2 <= t3 ? 2 : 3;
     }
     if (shape == 1) {

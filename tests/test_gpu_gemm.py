@@ -157,3 +157,24 @@ def test_gemm_forms_at_the_edges(be, oracle, ty, rows, k, n):
         finally:
             be.set_tuning(be.TUNE_GEMM_SHAPE, 0)
         assert _same(got, want), shape
+
+
+@pytest.mark.parametrize("rows", [5600, 5601])
+def test_gemm_rule_beyond_the_cache(be, oracle, rows):
+    # 5600 rows of 16384 are the last whose row operands count as held by the
+    # cache beyond L2 (175 tiles of 1.15 MB against 192 MiB); from 5601 the other
+    # times choose the form.  Every form's bits on three tokens are the oracle's.
+    k, n = 16384, 65
+    w = synth.random_matrix(Q4_K, rows, k, seed=3)
+    q8 = q8_rows(oracle, np.random.default_rng(4).standard_normal((n, k)).astype(np.float32))
+    at = [0, 33, 64]
+    want = oracle_gemm(oracle, Q4_K, w, rows, k, q8[at])
+    first = None
+    for shape in (0, 1, 2, 3):
+        be.set_tuning(be.TUNE_GEMM_SHAPE, shape)
+        try:
+            got = run_gemm(be, Q4_K, w, rows, k, q8)
+        finally:
+            be.set_tuning(be.TUNE_GEMM_SHAPE, 0)
+        first = got if first is None else first
+        assert _same(got[at], want) and _same(got, first), shape
