@@ -213,61 +213,6 @@ __global__ void k_repack_range(const uint8_t *__restrict__ src, uint8_t *__restr
         unit_to_device<TY>(src + i * BB, dst, U, u0 + i);
 }
 
-// A tile copy: the same bits with the units in 16-row tile order and, inside a
-// tile (16 rows of one block), the chunk bytes of the batched matrix-core
-// streams' 64 lanes side by side, lane 16 q + c holding what it reads of row c:
-//   IQ2_S  first 64 U bytes: 16 per lane, the qs and the sign dwords of groups
-//          2q, 2q + 1; next 16 U: 4 per lane, byte j the groups' qh fields of
-//          lookup j (low nibble) and the scale nibble of half group j; d plane.
-//   IQ3_S  first 64 U bytes: 16 per lane, dword k byte i the qs byte of lookup
-//          2q + k % 2 of the i-th of groups 0, 1, 4, 5 (k < 2) or 2, 3, 6, 7;
-//          next 32 U: 8 per lane, dword j byte i the sign byte q of the i-th of
-//          the same groups; tail and d planes in unit order.
-// One thread per lane slice; rows % 16 == 0.
-template <int TY>
-__global__ void k_units_to_tiles(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, long long rows, int nb) {
-    constexpr TypeLayout L = layout_of(TY);
-    const long long U = rows * nb, base = L.nchunk * U * 16;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < 4 * U; i += (long long)gridDim.x * blockDim.x) {
-        const long long tile = i >> 6;
-        const int lane = (int)(i & 63), q = lane >> 4, c = lane & 15;
-        const long long b = tile % nb, u = ((tile / nb) * 16 + c) * nb + b, ut = tile * 16 + c;
-        auto chunk = [&](int k) { return src + ((long long)k * U + u) * 16; };
-        if constexpr (TY == T_IQ2_S) {
-            const uint2 qs = ld_u64(chunk(q >> 1) + 8 * (q & 1)), sg = ld_u64(chunk(2 + (q >> 1)) + 8 * (q & 1));
-            reinterpret_cast<uint4 *>(dst)[i] = make_uint4(qs.x, qs.y, sg.x, sg.y);
-            const uint32_t sc = ld_u16(chunk(4) + 8 + 2 * q);
-            uint32_t e = (ld_u32(chunk(4) + 4 * (q >> 1)) >> (4 * (q & 1))) & 0x0f0f0f0fu;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) e |= ((sc >> (4 * j)) & 15u) << (8 * j + 4);
-            reinterpret_cast<uint32_t *>(dst + 64 * U)[i] = e;
-        } else {
-            uint32_t w[4] = {0, 0, 0, 0}, s[2] = {0, 0};
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int g = 4 * (k >> 1) + 2 * j + (k & 1);
-                    const uint8_t *qs = chunk(g >> 1) + 8 * (g & 1) + 2 * q;
-                    w[2 * j] |= (uint32_t)qs[0] << (8 * k);
-                    w[2 * j + 1] |= (uint32_t)qs[1] << (8 * k);
-                    s[j] |= (uint32_t)chunk(4 + (g >> 2))[4 * (g & 3) + q] << (8 * k);
-                }
-            reinterpret_cast<uint4 *>(dst)[i] = make_uint4(w[0], w[1], w[2], w[3]);
-            reinterpret_cast<uint2 *>(dst + 64 * U)[i] = make_uint2(s[0], s[1]);
-        }
-        if (q == 0) {
-#pragma unroll
-            for (int t = 0; t < L.tail / 4; ++t)
-                reinterpret_cast<uint32_t *>(dst + base)[ut * (L.tail / 4) + t] =
-                    reinterpret_cast<const uint32_t *>(src + base)[u * (L.tail / 4) + t];
-            reinterpret_cast<uint16_t *>(dst + base + L.tail * U)[ut] =
-                reinterpret_cast<const uint16_t *>(src + base + L.tail * U)[u];
-        }
-    }
-}
-
-// First non-finite f16 d / dmin in unit order (validate_scales, k_quants.rs:178-208).
 template <int TY>
 __global__ void k_validate_scales(const uint8_t *__restrict__ ggml, long long U, unsigned long long *first) {
     constexpr int BB = layout_of(TY).block_bytes;
@@ -413,22 +358,6 @@ hipError_t launch_repack_range(int ty, const uint8_t *src, uint8_t *dst, long lo
     case T_IQ3_S: hipLaunchKernelGGL(k_repack_range<T_IQ3_S>, dim3(grid), dim3(256), 0, s, src, dst, U, u0, n); break;
     case T_Q4_K: hipLaunchKernelGGL(k_repack_range<T_Q4_K>, dim3(grid), dim3(256), 0, s, src, dst, U, u0, n); break;
     case T_Q5_K: hipLaunchKernelGGL(k_repack_range<T_Q5_K>, dim3(grid), dim3(256), 0, s, src, dst, U, u0, n); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_units_to_tiles(const MatView &m, uint8_t *dst, hipStream_t s) {
-    if (m.rows % 16 != 0) return hipErrorInvalidValue;
-    int grid = cdiv(4 * m.units, 256);
-    grid = grid > 8192 ? 8192 : grid;
-    switch (m.type) {
-    case T_IQ2_S:
-        hipLaunchKernelGGL(k_units_to_tiles<T_IQ2_S>, dim3(grid), dim3(256), 0, s, m.planes, dst, (long long)m.rows, m.nb);
-        break;
-    case T_IQ3_S:
-        hipLaunchKernelGGL(k_units_to_tiles<T_IQ3_S>, dim3(grid), dim3(256), 0, s, m.planes, dst, (long long)m.rows, m.nb);
-        break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
