@@ -318,7 +318,9 @@ lbh_status lbh_gemm_q8_k_noalloc(lbh_ctx *ctx, const lbh_matrix *m, const uint8_
  * always-on shared expert, plus the scratch of one call (allocated once here, as the
  * reference's SwiGluScratch is: no allocation per call).  Supported type sets: routed
  * gate/up IQ2_S; routed down IQ3_S or IQ2_S; shared gate/up Q4_K or IQ2_S; shared down
- * Q5_K, IQ3_S or IQ2_S.  At most 16 routed experts per token. */
+ * Q5_K, IQ3_S or IQ2_S.  At most 16 routed experts per token.  A layer may be up to
+ * 16384 wide; the single-token calls take hidden and widths up to 8192 (a Q5_K
+ * shared width up to 4096) and fail with LBH_HIP_ERROR beyond, nothing launched. */
 
 /* [sync] */
 lbh_status lbh_moe_create(lbh_ctx *ctx, const lbh_matrix *const *gate, const lbh_matrix *const *up,

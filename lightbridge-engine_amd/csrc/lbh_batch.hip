@@ -1482,7 +1482,7 @@ __global__ void __launch_bounds__(64) k_route_batch(RouteBatchArgs a) {
 
 static inline int cdiv(long long a, long long b) { return (int)((a + b - 1) / b); }
 
-// LDS bytes of a stream launch of type ty (nm matrices, nb blocks per row).
+// LDS bytes of a VALU stream launch of type ty (nm matrices, nb blocks per row).
 static int stream_lds_of(int ty, int nm, int tc, int nb) {
     switch (ty) {
     case T_IQ2_S: return nm == 2 ? stream_lds<T_IQ2_S, 2>(tc, nb, 2) : stream_lds<T_IQ2_S, 1>(tc, nb, 2);
@@ -1493,18 +1493,23 @@ static int stream_lds_of(int ty, int nm, int tc, int nb) {
     }
 }
 
-// LDS of the launches of one stream: the VALU kernel's, and the matrix-core
-// kernel's when it runs that type.
+// LDS of the launches of one stream: the VALU kernel's where some chunk can run
+// there (past any limit where a row's units do not fit a wave, which leaves no row
+// step), and the matrix-core kernel's when it runs that type.
 static int stream_max(const BatchArgs &a, int ty, int nm, int nb) {
-    const int v = stream_lds_of(ty, nm, valu_cap(a, ty), nb);
-    if (!a.mx || (ty != T_IQ2_S && ty != T_IQ3_S)) return v;
-    const int m = mx_lds_bytes(ty);
+    const bool mx = a.mx && (ty == T_IQ2_S || ty == T_IQ3_S);
+    const int m = mx ? mx_lds_bytes(ty) : 0;
+    if (mx && a.mx_min <= 1) return m;
+    const int v = rows_per_step(2, nb) < 1 ? 1 << 30 : stream_lds_of(ty, nm, valu_cap(a, ty), nb);
     return v > m ? v : m;
 }
 
 // stage 0: sort + quantize; 1/2: routed / shared gate-up; 3/4: routed / shared down.
 int batch_lds_bytes(const BatchArgs &a, int stage) {
     const int nbh = a.hidden / 256, nbr = a.ffn_r / 256, nbs = a.ffn_s / 256;
+    // Q4_K / Q5_K shared rows run on the matrix cores (lbh_kt.h) and keep the limit
+    // of the VALU kernel's staging alone.
+    const bool kt = a.has_shared && a.shared.gate.type == T_Q4_K && a.shared.down.type == T_Q5_K;
     switch (stage) {
     case 0: {
         const int W = (a.n_tokens + 31) / 32;
@@ -1512,9 +1517,9 @@ int batch_lds_bytes(const BatchArgs &a, int stage) {
         return sort > MB_WAVES * 304 ? sort : MB_WAVES * 304;
     }
     case 1: return stream_max(a, a.type_gate_r, 2, nbh);
-    case 2: return a.has_shared ? stream_max(a, a.shared.gate.type, 2, nbh) : 0;
+    case 2: return kt ? stream_lds_of(T_Q4_K, 2, a.tc, nbh) : a.has_shared ? stream_max(a, a.shared.gate.type, 2, nbh) : 0;
     case 3: return stream_max(a, a.type_down_r, 1, nbr);
-    default: return a.has_shared ? stream_max(a, a.shared.down.type, 1, nbs) : 0;
+    default: return kt ? stream_lds_of(T_Q5_K, 1, a.tc, nbs) : a.has_shared ? stream_max(a, a.shared.down.type, 1, nbs) : 0;
     }
 }
 

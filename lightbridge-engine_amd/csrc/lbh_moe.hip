@@ -579,6 +579,14 @@ constexpr int moe_lpu() {
     return TY == T_Q5_K ? 4 : 2;
 }
 
+// A stream's row of nb blocks takes its lanes per block of one wave (LaneMap): past
+// 64 lanes there is no row step, and the item counts would divide by zero.
+static bool rows_fit(const MoeArgs &a) {
+    auto fits = [](int ty, int k) { return k / 256 * (ty == T_Q5_K ? moe_lpu<T_Q5_K>() : moe_lpu<T_Q4_K>()) <= 64; };
+    return fits(a.type_gate_r, a.hidden) && fits(a.type_down_r, a.ffn_r) &&
+           (!a.has_shared || (fits(a.shared.gate.type, a.hidden) && fits(a.shared.down.type, a.ffn_s)));
+}
+
 template <int TYR, int TYS>
 static hipError_t gate_up_typed(const MoeArgs &a, hipStream_t s) {
     const int nb = a.hidden / 256;
@@ -668,6 +676,7 @@ int moe_gate_up_resident_per_cu(int type_gate_r, int type_gate_s, int hidden) {
 }
 
 hipError_t launch_moe_router_shared(const MoeArgs &a, hipStream_t s) {
+    if (!rows_fit(a)) return hipErrorInvalidValue;
     const int nb = a.hidden / 256;
     const int rw = (a.router.n_experts + RT_EXPERTS - 1) / RT_EXPERTS;
     const int ts = a.shared.gate.type;
@@ -685,6 +694,7 @@ hipError_t launch_moe_router_shared(const MoeArgs &a, hipStream_t s) {
 }
 
 hipError_t launch_moe_gate_up(const MoeArgs &a, hipStream_t s) {
+    if (!rows_fit(a)) return hipErrorInvalidValue;
     const int tyr = a.type_gate_r;
     const int ts = a.has_shared ? a.shared.gate.type : tyr;
     if (tyr == T_IQ2_S && ts == T_Q4_K) return gate_up_typed<T_IQ2_S, T_Q4_K>(a, s);
@@ -693,6 +703,7 @@ hipError_t launch_moe_gate_up(const MoeArgs &a, hipStream_t s) {
 }
 
 hipError_t launch_moe_down(const MoeArgs &a, hipStream_t s) {
+    if (!rows_fit(a)) return hipErrorInvalidValue;
     const int tyr = a.type_down_r;
     const int ts = a.has_shared ? a.shared.down.type : tyr;
     if (tyr == T_IQ3_S && ts == T_Q5_K) return down_typed<T_IQ3_S, T_Q5_K>(a, s);

@@ -301,3 +301,35 @@ def test_shared_kquant_rows_at_the_edges(be, oracle, hidden, ffn_s, engine):
         got = run_checked(be, layer, ids, coefs, xs)
         bad = [t for t in range(n) if not np.array_equal(got[t], want[t], equal_nan=True)]
         assert not bad, f"{n} tokens: {bad}"
+
+
+@pytest.mark.parametrize("hidden,ffn_r,ffn_s,types,valu", [
+    (8448, 256, 256, (IQ2_S, IQ3_S, IQ2_S, IQ3_S), True),    # gate/up rows of 33 blocks
+    (512, 256, 4352, (IQ2_S, IQ3_S, Q4_K, Q5_K), False)])    # Q5_K down rows of 17 blocks, four lanes each
+def test_rows_longer_than_a_wave(be, oracle, hidden, ffn_r, ffn_s, types, valu):
+    """A row whose units do not fit the 64 lanes of a wave has no row step in the
+    single-token streams and the batch's VALU streams: those calls are refused
+    before anything is launched or written, and the matrix-core batch, which
+    takes such rows, gives the oracle's bits."""
+    import lbhip
+    layer = Layer(be, oracle, 2, hidden, ffn_r, ffn_s, types, seed=211)
+    ids, coefs = np.array([[0, 1]] * 3, np.uint32), np.full((3, 2), 0.5, np.float32)
+    xs = np.random.default_rng(22).standard_normal((3, hidden)).astype(np.float32)
+    y = dev(np.full(hidden, 7.0, np.float32))
+    for call in (be.moe_forward, be.moe_routed_by_id_into):
+        with pytest.raises(lbhip.KernelError):
+            call(layer.moe, ids[0], coefs[0], dev(xs[0]), y)
+    assert np.all(host(y) == 7.0)
+    layer.moe.reserve_batch(3, 2)
+    want = oracle_batch(oracle, layer, ids, coefs, xs)
+    got = run_checked(be, layer, ids, coefs, xs)
+    assert all(_same(got[t], want[t]) for t in range(3))
+    for engine in (2, 0):
+        if valu:
+            with pytest.raises(lbhip.KernelError) as e:
+                layer.moe.set_batch_engine(engine)
+            assert e.value.variant == "UnsupportedShape"
+        else:
+            layer.moe.set_batch_engine(engine)
+        got = run_checked(be, layer, ids, coefs, xs)
+        assert all(_same(got[t], want[t]) for t in range(3)), engine
