@@ -1414,15 +1414,6 @@ void lbh_debug_expf_host(const float *in, float *out, size_t n, int32_t swiglu, 
 
 namespace {
 
-MatGemm gemm_view(const lbh_matrix *m, float *y, int ldy) {
-    MatGemm g;
-    g.a = m->gemm_a;
-    g.y = y;
-    g.rows = (int32_t)m->rows;
-    g.ldy = ldy;
-    return g;
-}
-
 hipError_t prepare_gemm(lbh_matrix *m, hipStream_t s) {
     if (m->gemm_a) return hipSuccess;
     const int rows = (int)m->rows, nb = (int)m->nb;
@@ -1470,12 +1461,13 @@ lbh_status gemm_q8_k_into(lbh_ctx *ctx, const lbh_matrix *m, const uint8_t *q8, 
     const int nb = (int)m->nb;
     DeviceGuard g(ctx->device);
     GemmArgs a{};
+    a.a = m->gemm_a;
     a.b = bt;
+    a.y = y;
+    a.rows = (int32_t)m->rows;
     a.nb = nb;
     a.n_tokens = (int32_t)n_tokens;
-    a.n_mat = 1;
     a.shape = ctx->gemm_shape;
-    a.mat[0] = gemm_view(m, y, (int)m->rows);
     if (launch_prep_b(q8, (int)n_tokens, nb, bt, ctx->stream) != hipSuccess)
         return LBH_HIP_ERROR;
     return launch_kq_gemm(a, ctx->stream) == hipSuccess ? LBH_OK : LBH_HIP_ERROR;
@@ -1575,8 +1567,6 @@ BatchArgs batch_args(const lbh_moe *m, const uint32_t *ids, const float *coefs, 
     a.valu = !a.mx || a.mx_min > 1;
     return a;
 }
-
-bool is_kquant(int ty) { return ty == LBH_Q4_K || ty == LBH_Q5_K; }
 
 BatchStreams batch_streams(const lbh_moe *m) {
     BatchStreams b{};

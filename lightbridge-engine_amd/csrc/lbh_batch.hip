@@ -1284,22 +1284,20 @@ __device__ __forceinline__ void mx_prologue(uint8_t *tab, float *s_d8, int n, in
 }
 
 // The shared expert's K-quant rows in a stage launch (lbh_kt.h): workgroup wg of
-// kt_wgs(): 64 rows (one 16-row tile per wave) of matrix m against KT_NT token
-// tiles; the token groups of a row quad are neighbours, so its weights are
-// fetched once.  One tile a wave: two hold registers that the routed streams of
-// the launch then lack (steps of 5 / 64 / 256 tokens: 103 / 246 / 502 us with
-// one, 114 / 260 / 518 with two).
-constexpr int KT_NT = 1;
-__host__ __device__ inline int kt_groups(int n_tokens) { return ((n_tokens + 15) / 16 + KT_NT - 1) / KT_NT; }
+// kt_wgs(): 64 rows (one 16-row tile per wave) of matrix m against one token tile;
+// the token tiles of a row quad are neighbours, so its weights are fetched once.
+// Two tiles a wave hold registers that the routed streams of the launch then lack
+// (steps of 5 / 64 / 256 tokens: 103 / 246 / 502 us with one, 114 / 260 / 518 with
+// two).
 template <int TY>
 __device__ __forceinline__ void kt_workgroup(const uint8_t *w, int rows, int nb, const uint8_t *tok, int n_tokens, float *y,
                                              int wg) {
-    const int ng = kt_groups(n_tokens), quad = wg / ng, g = wg - quad * ng;
+    const int n_tt = (n_tokens + 15) / 16, quad = wg / n_tt, tt = wg - quad * n_tt;
     const int rt = 4 * quad + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    kt_rows<TY, KT_NT>(w, kt_w_bytes(TY, rows, nb), rt, nb, tok, g * KT_NT, (n_tokens + 15) / 16,
-                       [&](int t, int r, float v) {
-                           if (t < n_tokens) y[(long long)t * rows + rt * 16 + r] = v;
-                       });
+    kt_rows<TY>(w, kt_w_bytes(TY, rows, nb), rt, nb, tok + (size_t)tt * nb * KT_TOK_TILE, [&](int i, int r, float v) {
+        const int t = 16 * tt + i;
+        if (t < n_tokens) y[(long long)t * rows + rt * 16 + r] = v;
+    });
 }
 
 // Gate/up on the matrix cores (as k_mb_gate_up): workgroup (chunk, row tile).
@@ -1579,7 +1577,7 @@ static hipError_t down_typed(const BatchArgs &a, hipStream_t s) {
 }
 
 // Workgroups of the shared expert's K-quant rows (kt_workgroup).
-static int kt_wgs(const BatchArgs &a, int rows) { return rows / 64 * kt_groups(a.n_tokens); }
+static int kt_wgs(const BatchArgs &a, int rows) { return rows / 64 * cdiv(a.n_tokens, 16); }
 
 // KTY: the launch also holds the shared expert's K-quant gate and up / down.
 template <int TY, bool SHARED, bool TILE, int NM, int KTY = 0>

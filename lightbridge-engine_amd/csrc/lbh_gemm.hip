@@ -421,7 +421,7 @@ __device__ __forceinline__ void fold_block(Chains<HV> &ch, const uint8_t *At, co
 }
 
 template <int HV>
-__device__ __forceinline__ void gemm_tile(const GemmArgs &g, const MatGemm &M, GemmLDS &S, const StageSrc &src,
+__device__ __forceinline__ void gemm_tile(const GemmArgs &g, GemmLDS &S, const StageSrc &src,
                                           int rg, int tg, int tw, int wid, int lane, int rt0, int tt0) {
     const int nb = g.nb;
     Chains<HV> ch;
@@ -478,7 +478,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const MatGemm &M, G
             float v = xch[i * 64 + lane];
 #pragma unroll
             for (int r = 0; r < 4; ++r) v = __fadd_rn(v, ch.c[i][r]);
-            if (row < M.rows) M.y[(long long)t * M.ldy + row] = v;
+            if (row < g.rows) g.y[(long long)t * g.rows + row] = v;
         }
     }
 }
@@ -491,8 +491,7 @@ __global__ void __launch_bounds__(64 * NW) k_kq_gemm_2x2(GemmArgs g) {
     // waves w and w + RG * TG (the two halves of one tile) land on the same SIMD
     const int tw = wid % (RG * TG), hv = wid / (RG * TG);
     const int rg = tw % RG, tg = tw / RG;
-    const MatGemm &M = g.mat[blockIdx.y];   // which matrix of the launch
-    const int n_rt = (M.rows + 31) / 32, n_tt = (g.n_tokens + 31) / 32;
+    const int n_rt = (g.rows + 31) / 32, n_tt = (g.n_tokens + 31) / 32;
     const int row_wgs = (n_rt + RG - 1) / RG, tok_wgs = (n_tt + TG - 1) / TG;
     // XCD-aware order: workgroups are dealt to the eight XCDs round robin;
     // consecutive workgroups of one XCD share a row tile, so each A tile is
@@ -525,15 +524,15 @@ __global__ void __launch_bounds__(64 * NW) k_kq_gemm_2x2(GemmArgs g) {
     StageSrc src;
     src.last_a = n_rt - 1 - rt0 < RG - 1 ? n_rt - 1 - rt0 : RG - 1;
     src.last_b = n_tt - 1 - tt0 < TG - 1 ? n_tt - 1 - tt0 : TG - 1;
-    src.ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(M.a + (long long)rt0 * g.nb * A_TILE), (short)0,
+    src.ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(g.a + (long long)rt0 * g.nb * A_TILE), (short)0,
                                                (src.last_a + 1) * g.nb * A_TILE, 0x00020000);
     src.rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(g.b + (long long)tt0 * g.nb * B_TILE), (short)0,
                                                (src.last_b + 1) * g.nb * B_TILE, 0x00020000);
 
     if (hv == 0)
-        gemm_tile<0>(g, M, S, src, rg, tg, tw, wid, lane, rt0, tt0);
+        gemm_tile<0>(g, S, src, rg, tg, tw, wid, lane, rt0, tt0);
     else
-        gemm_tile<1>(g, M, S, src, rg, tg, tw, wid, lane, rt0, tt0);
+        gemm_tile<1>(g, S, src, rg, tg, tw, wid, lane, rt0, tt0);
 }
 
 // ---- tokens in LDS
@@ -693,9 +692,8 @@ __device__ __forceinline__ void gl_pass(float (&v)[GL_NT][4], const RowSrc &A, _
 __global__ void __launch_bounds__(64 * GL_WAVES, 4) k_kq_gemm_lds(GemmArgs g) {
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const MatGemm &M = g.mat[blockIdx.y];
     const int nb = g.nb;
-    const int n_rt = (M.rows + 31) / 32, n_tt = (g.n_tokens + 31) / 32;
+    const int n_rt = (g.rows + 31) / 32, n_tt = (g.n_tokens + 31) / 32;
     const int row_wgs = (n_rt + 3) / 4, tok_wgs = (n_tt + 1) / 2;
     // XCD-aware order: workgroups are dealt to the eight XCDs round robin; each
     // XCD takes a contiguous run of row groups with all their token groups, so
@@ -707,7 +705,7 @@ __global__ void __launch_bounds__(64 * GL_WAVES, 4) k_kq_gemm_lds(GemmArgs g) {
     const int lin = id < nfull ? (id % 8) * (nfull / 8) + id / 8 : id;   // a bijection of [0, nwg)
     const int wrt = lin / tok_wgs, tt0 = (lin - wrt * tok_wgs) * 2;
     const int rt = wrt * 4 + (wid >> 1), half = wid & 1;
-    const RowSrc A(M.a, rt < n_rt ? rt : n_rt - 1, half, nb, lane);   // rows past the matrix: never stored
+    const RowSrc A(g.a, rt < n_rt ? rt : n_rt - 1, half, nb, lane);   // rows past the matrix: never stored
     const int last = n_tt - 1 - tt0 < 1 ? n_tt - 1 - tt0 : 1;
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t *>(g.b + (long long)tt0 * nb * B_TILE), (short)0, (last + 1) * nb * B_TILE, 0x00020000);
@@ -715,13 +713,13 @@ __global__ void __launch_bounds__(64 * GL_WAVES, 4) k_kq_gemm_lds(GemmArgs g) {
     gl_pass<true>(v, A, rb, last, nb, 0, wid, lane);
     for (int l0 = 2; l0 < 8; l0 += 3) gl_pass<false>(v, A, rb, last, nb, l0, wid, lane);
     const int row = rt * 32 + 16 * half + (lane & 15);
-    if (row >= M.rows) return;
+    if (row >= g.rows) return;
 #pragma unroll
     for (int n = 0; n < GL_NT; ++n)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int t = tt0 * 32 + 16 * n + 4 * (lane >> 4) + i;
-            if (t < g.n_tokens) M.y[(long long)t * M.ldy + row] = v[n][i];
+            if (t < g.n_tokens) g.y[(long long)t * g.rows + row] = v[n][i];
         }
 }
 
@@ -805,11 +803,10 @@ __global__ void __launch_bounds__(64 * GS_WAVES) k_kq_gemm_split(GemmArgs g) {
     __shared__ __align__(16) float s_ch[9][NT][4][64];
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const MatGemm &M = g.mat[blockIdx.y];
-    const int n16 = (M.rows + 15) / 16, tg = ((g.n_tokens + 15) / 16 + NT - 1) / NT;
+    const int n16 = (g.rows + 15) / 16, tg = ((g.n_tokens + 15) / 16 + NT - 1) / NT;
     const int r16 = (int)blockIdx.x / tg, tt0 = ((int)blockIdx.x - r16 * tg) * NT;
     if (r16 >= n16) return;
-    const RowSrc A(M.a, r16 >> 1, r16 & 1, g.nb, lane);
+    const RowSrc A(g.a, r16 >> 1, r16 & 1, g.nb, lane);
     float acc[3][NT][4];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
@@ -836,7 +833,7 @@ __global__ void __launch_bounds__(64 * GS_WAVES) k_kq_gemm_split(GemmArgs g) {
 #pragma unroll
         for (int c = 0; c < 8; ++c) v = __fadd_rn(v, s_ch[c][n][i][l]);
         const int t = 16 * (tt0 + n) + 4 * (l >> 4) + i, row = 16 * r16 + (l & 15);
-        if (t < g.n_tokens && row < M.rows) M.y[(long long)t * M.ldy + row] = v;
+        if (t < g.n_tokens && row < g.rows) g.y[(long long)t * g.rows + row] = v;
     }
 }
 
@@ -864,18 +861,18 @@ hipError_t launch_prep_b(const uint8_t *q8, int n_tokens, int nb, uint8_t *b, hi
 }
 
 template <int NT>
-static hipError_t gemm_split(const GemmArgs &g, int rows, hipStream_t s) {
-    const int grid = cdiv(rows, 16) * cdiv(cdiv(g.n_tokens, 16), NT);
-    hipLaunchKernelGGL((k_kq_gemm_split<NT>), dim3(grid, g.n_mat), dim3(64 * GS_WAVES), 0, s, g);
+static hipError_t gemm_split(const GemmArgs &g, hipStream_t s) {
+    const int grid = cdiv(g.rows, 16) * cdiv(cdiv(g.n_tokens, 16), NT);
+    hipLaunchKernelGGL((k_kq_gemm_split<NT>), dim3(grid), dim3(64 * GS_WAVES), 0, s, g);
     return hipGetLastError();
 }
 
-static hipError_t gemm_2x2(const GemmArgs &g, int rows, hipStream_t s) {
+static hipError_t gemm_2x2(const GemmArgs &g, hipStream_t s) {
     const int lds = (int)sizeof(GemmLDS);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_kq_gemm_2x2), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return e;
-    const int grid = cdiv(cdiv(rows, 32), RG) * cdiv(cdiv(g.n_tokens, 32), TG);
-    hipLaunchKernelGGL(k_kq_gemm_2x2, dim3(grid, g.n_mat), dim3(64 * NW), lds, s, g);
+    const int grid = cdiv(cdiv(g.rows, 32), RG) * cdiv(cdiv(g.n_tokens, 32), TG);
+    hipLaunchKernelGGL(k_kq_gemm_2x2, dim3(grid), dim3(64 * NW), lds, s, g);
     return hipGetLastError();
 }
 
@@ -913,9 +910,8 @@ static long long split_ns(const FormTimes &f, int rows, int n_tokens, int nt) {
 
 // shape: 0 default, 1 the split form, 2 the 2 x 2 form, 3 the LDS form.
 hipError_t launch_kq_gemm(const GemmArgs &g, hipStream_t s) {
-    if (g.n_mat < 1 || g.n_mat > GEMM_MAX_MATS || g.n_tokens < 1 || g.nb < 1 || g.nb > 64) return hipErrorInvalidValue;
-    int rows = 0;
-    for (int i = 0; i < g.n_mat; ++i) rows = g.mat[i].rows > rows ? g.mat[i].rows : rows;
+    if (g.n_tokens < 1 || g.nb < 1 || g.nb > 64) return hipErrorInvalidValue;
+    const int rows = g.rows;
     const FormTimes &f = gemm_a_bytes(rows, g.nb) > KQ_CACHED_BYTES ? KQ_BEYOND : KQ_CACHED;
     int nt = 1;
     for (int n = 2; n <= 4; ++n)
@@ -930,14 +926,14 @@ hipError_t launch_kq_gemm(const GemmArgs &g, hipStream_t s) {
     }
     if (shape == 1) {
         switch (nt) {
-        case 1: return gemm_split<1>(g, rows, s);
-        case 2: return gemm_split<2>(g, rows, s);
-        case 3: return gemm_split<3>(g, rows, s);
-        default: return gemm_split<4>(g, rows, s);
+        case 1: return gemm_split<1>(g, s);
+        case 2: return gemm_split<2>(g, s);
+        case 3: return gemm_split<3>(g, s);
+        default: return gemm_split<4>(g, s);
         }
     }
-    if (shape == 2) return gemm_2x2(g, rows, s);
-    hipLaunchKernelGGL(k_kq_gemm_lds, dim3((int)lds_wgs, g.n_mat), dim3(64 * GL_WAVES), 0, s, g);
+    if (shape == 2) return gemm_2x2(g, s);
+    hipLaunchKernelGGL(k_kq_gemm_lds, dim3((int)lds_wgs), dim3(64 * GL_WAVES), 0, s, g);
     return hipGetLastError();
 }
 

@@ -154,20 +154,11 @@ struct MoeArgs {
 
 // ------------------------------------------------ K-quant GEMM on f16 MFMA
 
-constexpr int GEMM_MAX_MATS = 3;
-
-// One matrix of a GEMM launch: its MFMA-ready copy and output.
-struct MatGemm {
-    const uint8_t *a;      // [ceil(rows / 32)][nb] A tiles (operands, then (d, dmin) per row)
-    float *y;              // y[t * ldy + r]
-    int32_t rows;
-    int32_t ldy;
-};
-
 struct GemmArgs {
-    MatGemm mat[GEMM_MAX_MATS];   // matrices sharing K and the activations
-    const uint8_t *b;             // [ceil(n_tokens / 32)][nb] B tiles (operands, then d8 per token)
-    int32_t n_mat, nb, n_tokens, shape;
+    const uint8_t *a;      // [ceil(rows / 32)][nb] A tiles (operands, then (d, dmin) per row)
+    const uint8_t *b;      // [ceil(n_tokens / 32)][nb] B tiles (operands, then d8 per token)
+    float *y;              // y[t * rows + r]
+    int32_t rows, nb, n_tokens, shape;
 };
 
 // ------------------------------------------------------ batched MoE decode

@@ -1,5 +1,5 @@
-// lbh_kt.h — Q4_K / Q5_K rows against up to a few 16-token tiles on the f16
-// matrix cores, one wave per 16 rows, bit-identical to the reference's per-row
+// lbh_kt.h — Q4_K / Q5_K rows against 16-token tiles on the f16 matrix cores, one
+// wave per 16 rows and tile, bit-identical to the reference's per-row
 // dot (dot_q4_or_q5_k, crates/bridge-quant-layout/src/q8_k.rs:247-327).
 //
 // Per block the eight lane sums (residues mod 8) are one
@@ -18,7 +18,7 @@
 // its sub-blocks), Q5_K 64 bytes a lane (the quants as bytes: rebuilding the
 // fifth bit from its plane cost as many instructions as the products), then
 // the f16 scales and minimums of the lane's sub-blocks (8 bytes) and the rows'
-// (d, dmin).  The tokens come as f16 operands (kt_store_block) from L1 / L2.
+// (d, dmin).  The tokens come as f16 operands (kt_store_piece) from L1 / L2.
 //
 // What bounds it: VALU issue, 80 instructions per token tile (16 per f32 chain
 // step pair and the scales) and about 80 for the weights of a step.
@@ -117,44 +117,32 @@ __device__ __forceinline__ kt_h4 kt_mins(const KtW<TY> &w) {
     return __builtin_bit_cast(kt_h4, o);
 }
 
-// Row tile rt (16 rows) of a tile copy (K = 256 nb) against token tiles tt0 ..
-// tt0 + NT - 1 of tok (clamped to the last of n_tt): out(token, row in the
-// tile, value) for every token of the NT tiles.  The weights of the next block
-// and the token operands of the next RING residues are in flight while a
-// residue is computed.
-template <int TY, int NT, class Out>
-__device__ __forceinline__ void kt_rows(const uint8_t *w, size_t w_bytes, int rt, int nb, const uint8_t *tok, int tt0,
-                                        int n_tt, Out out) {
+// Row tile rt (16 rows) of a tile copy (K = 256 nb) against the 16-token tile at tok:
+// out(token in the tile, row in the tile, value).  The weights of the next block
+// and the token operands of the next RING residues are in flight while a residue
+// is computed.
+template <int TY, class Out>
+__device__ __forceinline__ void kt_rows(const uint8_t *w, size_t w_bytes, int rt, int nb, const uint8_t *tok, Out out) {
     constexpr int RING = 4;
     const int lane = threadIdx.x & 63, q = lane >> 4;
     Planes P;
     P.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(w), (short)0, (int)(uint32_t)w_bytes, 0x00020000);
-    const uint8_t *tp[NT];
-#pragma unroll
-    for (int n = 0; n < NT; ++n) tp[n] = tok + (size_t)(tt0 + n < n_tt ? tt0 + n : n_tt - 1) * nb * KT_TOK_TILE;
     KtW<TY> wa, wb;
-    kt_h8 ring[RING][NT];
-    kt_h4 mn[NT];
-    float4 d8[NT];
-    float acc[9][NT][4];
+    kt_h8 ring[RING];
+    kt_h4 mn;
+    float4 d8;
+    float acc[9][4];
 #pragma unroll
     for (int c = 0; c < 9; ++c)
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[c][n][i] = 0.0f;
+        for (int i = 0; i < 4; ++i) acc[c][i] = 0.0f;
     auto fetch = [&](int t, int b) {   // residue t (static) of block b
-#pragma unroll
-        for (int n = 0; n < NT; ++n)
-            ring[t % RING][n] = *reinterpret_cast<const kt_h8 *>(tp[n] + (size_t)b * KT_TOK_TILE + 1024 * t + 16 * lane);
+        ring[t % RING] = *reinterpret_cast<const kt_h8 *>(tok + (size_t)b * KT_TOK_TILE + 1024 * t + 16 * lane);
     };
     auto fetch_rest = [&](int b) {
-#pragma unroll
-        for (int n = 0; n < NT; ++n) {
-            const uint8_t *p = tp[n] + (size_t)b * KT_TOK_TILE;
-            mn[n] = *reinterpret_cast<const kt_h4 *>(p + KT_MIN + 8 * lane);
-            d8[n] = *reinterpret_cast<const float4 *>(p + KT_D8 + 16 * q);
-        }
+        const uint8_t *p = tok + (size_t)b * KT_TOK_TILE;
+        mn = *reinterpret_cast<const kt_h4 *>(p + KT_MIN + 8 * lane);
+        d8 = *reinterpret_cast<const float4 *>(p + KT_D8 + 16 * q);
     };
     const kt_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     auto block = [&](int b, const KtW<TY> &cur, KtW<TY> &next) {
@@ -162,31 +150,23 @@ __device__ __forceinline__ void kt_rows(const uint8_t *w, size_t w_bytes, int rt
         kt_load<TY>(P, (uint32_t)(rt * nb + bn), lane, next);
         const KtScales k = kt_scales<TY>(cur);
         const float d = f16_to_f32(cur.dd & 0xffffu), dmin = f16_to_f32(cur.dd >> 16);
-        float s[NT][4];
-        const kt_h4 wm = kt_mins<TY>(cur);
+        float s[4];
+        const kt_f4 m = __builtin_amdgcn_mfma_f32_16x16x16f16(mn, kt_mins<TY>(cur), zero, 0, 0, 0);
+        const float e[4] = {d8.x, d8.y, d8.z, d8.w};
 #pragma unroll
-        for (int n = 0; n < NT; ++n) {
-            const float e[4] = {d8[n].x, d8[n].y, d8[n].z, d8[n].w};
-            const kt_f4 m = __builtin_amdgcn_mfma_f32_16x16x16f16(mn[n], wm, zero, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                s[n][i] = __fmul_rn(d, e[i]);
-                acc[8][n][i] = __fsub_rn(acc[8][n][i], __fmul_rn(__fmul_rn(dmin, e[i]), m[i]));
-            }
+        for (int i = 0; i < 4; ++i) {
+            s[i] = __fmul_rn(d, e[i]);
+            acc[8][i] = __fsub_rn(acc[8][i], __fmul_rn(__fmul_rn(dmin, e[i]), m[i]));
         }
         fetch_rest(bn);
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const kt_h8 wt = kt_weights<TY>(cur, k, t);
-            kt_f4 r[NT];
-#pragma unroll
-            for (int n = 0; n < NT; ++n) r[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ring[t % RING][n], wt, zero, 0, 0, 0);
+            const kt_f4 r = __builtin_amdgcn_mfma_f32_16x16x32_f16(ring[t % RING], wt, zero, 0, 0, 0);
             if (t + RING < 8) fetch(t + RING, b);
             else fetch(t + RING - 8, bn);
 #pragma unroll
-            for (int n = 0; n < NT; ++n)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[t][n][i] = __fadd_rn(acc[t][n][i], __fmul_rn(s[n][i], r[n][i]));
+            for (int i = 0; i < 4; ++i) acc[t][i] = __fadd_rn(acc[t][i], __fmul_rn(s[i], r[i]));
         }
     };
     kt_load<TY>(P, (uint32_t)(rt * nb), lane, wa);
@@ -199,14 +179,12 @@ __device__ __forceinline__ void kt_rows(const uint8_t *w, size_t w_bytes, int rt
         block(b + 1, wb, wa);
     }
 #pragma unroll
-    for (int n = 0; n < NT; ++n)
+    for (int i = 0; i < 4; ++i) {
+        float v = acc[8][i];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float v = acc[8][n][i];
-#pragma unroll
-            for (int t = 0; t < 8; ++t) v = __fadd_rn(v, acc[t][n][i]);   // q8_k.rs:323-325
-            out(16 * (tt0 + n) + 4 * q + i, lane & 15, v);
-        }
+        for (int t = 0; t < 8; ++t) v = __fadd_rn(v, acc[t][i]);   // q8_k.rs:323-325
+        out(4 * q + i, lane & 15, v);
+    }
 }
 
 // The token operand pieces of one quantized block (292 Q8_K bytes at blk, LDS)
