@@ -98,23 +98,27 @@ def test_batch_single_token_single_expert(be, oracle, small):
     assert _same(run_checked(be, small, ids, coefs, xs)[0], want[0])
 
 
+@pytest.mark.parametrize("engine", [0, 4, 1])
 @pytest.mark.parametrize("tiles", [(1, 7, 5, 9, 3), (3, 64, 256, 20, 512), (16, 128, 128, 320, 128), (5, 2, 1, 1, 2)])
-def test_batch_launch_shapes_give_the_same_bits(be, oracle, small, tiles):
+def test_batch_launch_shapes_give_the_same_bits(be, oracle, small, tiles, engine):
+    """Tokens per chunk and the VALU streams' rows per workgroup, with every
+    chunk (0), those below four tokens (4) or none (1) on the VALU."""
     _, ids, coefs = zipf_routing(oracle, 21, 12, 4, seed=sum(tiles))
     xs = np.random.default_rng(10).standard_normal((21, 512)).astype(np.float32)
     want = oracle_batch(oracle, small, ids, coefs, xs)
+    small.moe.set_batch_engine(engine)
     small.moe.set_batch_tiles(*tiles)
     try:
         got = run_checked(be, small, ids, coefs, xs)
     finally:
-        small.moe.set_batch_tiles()
+        small.moe.set_batch_engine()
     assert all(_same(got[t], want[t]) for t in range(21))
 
 
 @pytest.mark.parametrize("engine", [(0, 0, 0), (1, 0, 0), (6, 0, 0), (3, 32, 64), (1, 64, 16), (16, 16, 32)])
 def test_batch_engines_bit_exact(be, oracle, small, engine):
-    """The IQ streams on the VALU integer dots (0), all chunks on the f16 matrix
-    cores (1), the per-chunk split at several thresholds and row tiles, with hot
+    """The IQ streams on the VALU integer dots (0), all chunks on the int8 matrix
+    cores (1), the chunks divided at several thresholds and row tiles, with hot
     experts past one 16-token chunk and single-token experts."""
     _, ids, coefs = zipf_routing(oracle, 40, 12, 4, seed=15)
     xs = np.random.default_rng(16).standard_normal((40, 512)).astype(np.float32)
@@ -136,11 +140,15 @@ def test_batch_engine_rejects_bad_settings(small, bad):
     small.moe.set_batch_engine()
 
 
+@pytest.mark.parametrize("ffn_s", [256, 2304, 4352])
 @pytest.mark.parametrize("types", [(IQ2_S, IQ3_S, IQ2_S, IQ3_S), (IQ2_S, IQ2_S, IQ2_S, IQ2_S),
-                                   (IQ2_S, IQ2_S, IQ2_S, IQ3_S)])
-def test_batch_type_sets(be, oracle, types):
-    """Hy3's own shared expert is IQ2_S/IQ3_S (profile.rs, schema.rs)."""
-    layer = Layer(be, oracle, 6, 1024, 512, 256, types, seed=61)
+                                   (IQ2_S, IQ2_S, IQ2_S, IQ3_S), (IQ2_S, IQ3_S, Q4_K, IQ3_S),
+                                   (IQ2_S, IQ3_S, IQ2_S, Q5_K)])
+def test_batch_type_sets(be, oracle, types, ffn_s):
+    """Hy3's own shared expert is IQ2_S/IQ3_S (profile.rs, schema.rs); Q4_K gate
+    and up or a Q5_K down alone stay on the VALU.  Shared down rows of one block,
+    and of 9 and 17 (two and three groups of eight of the row-major IQ3_S rows)."""
+    layer = Layer(be, oracle, 6, 1024, 512, ffn_s, types, seed=61)
     layer.moe.reserve_batch(16, 3)
     _, ids, coefs = zipf_routing(oracle, 11, 6, 3, seed=12)
     xs = np.random.default_rng(13).standard_normal((11, 1024)).astype(np.float32)
@@ -299,7 +307,8 @@ def test_shared_kquant_rows_at_the_edges(be, oracle, hidden, ffn_s, engine):
         xs[1::2] *= rng.random((n // 2, hidden)).astype(np.float32)
         want = oracle_batch(oracle, layer, ids, coefs, xs)
         got = run_checked(be, layer, ids, coefs, xs)
-        bad = [t for t in range(n) if not np.array_equal(got[t], want[t], equal_nan=True)]
+        assert np.isfinite(want).all()
+        bad = [t for t in range(n) if not _same(got[t], want[t])]
         assert not bad, f"{n} tokens: {bad}"
 
 

@@ -49,9 +49,8 @@ def batch_case(oracle, layer, n_tokens, n_experts, top_k, seed):
 
 @pytest.mark.parametrize("engine", [(1, 0, 0), (4, 0, 0), (3, 64, 64), (3, 32, 64), (1, 64, 16), (16, 16, 32)])
 def test_tile_copies_of_every_expert_bit_exact(be, oracle, small, engine):
-    """Every chunk size on the matrix cores (1), the split defaults (4), the
-    defaults with copies (3, one wave per tile) and other row tiles (waves per
-    16-row tile 1, 2, 4)."""
+    """Every chunk size on the matrix cores (1), smaller chunks on the VALU, which
+    reads the uploaded matrices (3, 4, 16), and other rows per workgroup."""
     ids, coefs, xs, want = batch_case(oracle, small, 40, 12, 4, seed=21)
     small.moe.make_batch_tile_copies()
     assert small.moe.batch_tile_copy_bytes == copy_bytes(small, range(12))
@@ -181,14 +180,17 @@ def test_tile_copies_async_device_routed_and_residual(be, oracle, small):
         small.moe.make_batch_tile_copies([])
 
 
-@pytest.mark.parametrize("hidden,ffn,down", [(256, 768, IQ3_S), (768, 256, IQ3_S), (1280, 256, IQ2_S), (512, 1280, IQ3_S)])
+@pytest.mark.parametrize("hidden,ffn,down", [(256, 768, IQ3_S), (768, 256, IQ3_S), (1280, 256, IQ2_S), (512, 1280, IQ3_S),
+                                             (512, 2048, IQ3_S), (768, 2304, IQ3_S), (256, 4352, IQ3_S), (512, 2304, IQ2_S)])
 @pytest.mark.parametrize("copied", [None, [0, 2], "all"])
 def test_int8_streams_at_the_edges(be, oracle, hidden, ffn, down, copied):
-    """The int8 matrix-core streams at block counts below, at and off the wave
-    split (1, 2, 3, 5 blocks a row), chunks of 1, 2 or 3, 15 and 16 tokens, weights
-    whose codes, signs and scales are all 0, all ones or random, and inputs
+    """The int8 matrix-core streams at 1, 2, 3, 5, 8, 9 and 17 blocks a row (the
+    row-major rows go in groups of four blocks, IQ3_S eight: none, one and several
+    whole ones, with and without a rest), chunks of 1, 2 or 3, 15 and 16 tokens,
+    weights whose codes, signs and scales are all 0, all ones or random, and inputs
     that quantize to +-127: the largest integer sums, over the matrices as
-    uploaded, with copies of some experts and of all, at every wave split."""
+    uploaded, with copies of some experts and of all, at the default rows per
+    workgroup (several tiles a wave) and at fewer."""
     def edge(e, *mats):
         for m in mats:
             b = m.reshape(-1, 110 if m is mats[2] and down == IQ3_S else 82)
@@ -208,7 +210,7 @@ def test_int8_streams_at_the_edges(be, oracle, hidden, ffn, down, copied):
     xs = np.sign(rng.standard_normal((n, hidden))).astype(np.float32)
     xs[1::2] *= rng.random((8, hidden)).astype(np.float32)
     want = oracle_batch(oracle, layer, ids, coefs, xs)
-    for engine in ((1, 64, 64), (1, 32, 32), (1, 16, 16), (2, 64, 16)):
+    for engine in ((1, 0, 0), (1, 64, 64), (1, 32, 32), (1, 16, 16), (2, 64, 16)):
         moe.set_batch_engine(*engine)
         got = run_checked(be, layer, ids, coefs, xs)
         bad = [t for t in range(n) if not _same(got[t], want[t])]

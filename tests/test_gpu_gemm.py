@@ -5,8 +5,8 @@ Every output y[t, r] must equal the reference's per-row dot
 token t's Q8_K row, bit for bit: random blocks, negative d/dmin, the integer
 extremes (scale 63, mins 63, 5-bit quants 31, activations at +-127), ragged row
 and token counts (row and token tiles not multiples of a workgroup's), every
-schedule (2 x 2 tiles staged through registers or buffer-to-LDS loads; 3 x 4
-tiles in three passes), and the BASELINE configs[4] shape
+form (chains split over waves, 2 x 2 tiles in LDS, tokens in LDS and three
+passes) and the rule that picks one, and the BASELINE configs[4] shape
 (Q5_K 12288 x 4096, 512 tokens) in full.
 """
 import numpy as np
@@ -71,7 +71,7 @@ def test_gemm_random_bit_exact(be, oracle, ty, rows, k, n):
 
 
 @pytest.mark.parametrize("ty", [Q4_K, Q5_K])
-@pytest.mark.parametrize("shape", [0, 3])
+@pytest.mark.parametrize("shape", [0, 1, 2, 3])
 def test_gemm_integer_extremes(be, oracle, ty, shape):
     rows, k, n = 48, 512, 40
     bb = synth.BLOCK_BYTES[ty]
