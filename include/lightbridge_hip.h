@@ -320,7 +320,8 @@ lbh_status lbh_gemm_q8_k_noalloc(lbh_ctx *ctx, const lbh_matrix *m, const uint8_
  * gate/up IQ2_S; routed down IQ3_S or IQ2_S; shared gate/up Q4_K or IQ2_S; shared down
  * Q5_K, IQ3_S or IQ2_S.  At most 16 routed experts per token.  A layer may be up to
  * 16384 wide; the single-token calls take hidden and widths up to 8192 (a Q5_K
- * shared width up to 4096) and fail with LBH_HIP_ERROR beyond, nothing launched. */
+ * shared width up to 4096) and fail with LBH_HIP_ERROR beyond, their output left
+ * alone. */
 
 /* [sync] */
 lbh_status lbh_moe_create(lbh_ctx *ctx, const lbh_matrix *const *gate, const lbh_matrix *const *up,
@@ -341,7 +342,7 @@ lbh_status lbh_moe_set_tiles(lbh_moe *moe, int32_t wg_routed, int32_t wg_shared,
  * lbh_moe_block_forward), forked from and joined back to the context's stream;
  * 0 (default) runs the routed and shared experts in the same two launches on
  * the context's stream, which measured faster on MI355X (38.7 vs 50.9 us per
- * token at the configs[2] shapes in HIP-graph replay).  Same bits either way.
+ * token of the layer of 192 experts in HIP-graph replay).  Same bits either way.
  * The layer's second stream and shared-output buffer are per layer: forwards
  * on one layer must be ordered (one caller stream). */
 lbh_status lbh_moe_set_streams(lbh_moe *moe, int32_t two_streams);
@@ -398,8 +399,12 @@ lbh_status lbh_moe_set_batch_tiles(lbh_moe *moe, int32_t tokens_per_chunk, int32
  * whose batch is a loop over tokens).  Chunks of at least mx_min_tokens tokens
  * (1..16; 1 until this is called) run on the int8 matrix cores, one 16-row x
  * 16-token product per block, with mx_rows_gate_up / mx_rows_down rows per
- * workgroup (16, 32 or 64; 0: the defaults 64 and 256); smaller chunks run on
- * the VALU integer dots; mx_min_tokens = 0 keeps every chunk on the VALU.
+ * workgroup (16, 32 or 64; 0: the defaults 64 and 256).  Each of a workgroup's
+ * four waves takes 16-row tiles of its own, down over tile copies 32 rows, so that
+ * fewer than 64 (128) rows leave waves idle, and 16 down rows run as 32.  Smaller
+ * chunks run on the VALU integer dots; mx_min_tokens = 0 keeps every chunk there.
+ * Engines that need the VALU streams fail with LBH_UNSUPPORTED_SHAPE on layers
+ * they cannot take (rows of more than 8192, or too many tokens for the LDS).
  * Every choice gives the same bits.  Resets the tokens per chunk (16 with the
  * matrix cores, 8 without) and the VALU row tiles to their defaults. */
 lbh_status lbh_moe_set_batch_engine(lbh_moe *moe, int32_t mx_min_tokens, int32_t mx_rows_gate_up,

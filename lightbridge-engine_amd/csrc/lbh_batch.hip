@@ -797,8 +797,8 @@ __global__ void __launch_bounds__(MB_THREADS) k_mb_down(BatchArgs a) {
 // weights) the same tile took about twice the VALU work: f16 signs and scales
 // for the weights, f16 conversions of the quants.  Measured on 192 experts of
 // hidden 4096, width 1536, top-8 Zipf(1.1), tile copies, kernel times:
-//   64 tokens   gate/up 159 -> 88 us, down 91 -> 61 us (step 417 -> 354 us)
-//   256 tokens  gate/up 375 -> 222 us, down 242 -> 143 us (step 832 -> 611 us)
+//   64 tokens   gate/up 159 -> 88 us, down 91 -> 61 us (step 417 -> 355 us)
+//   256 tokens  gate/up 375 -> 222 us, down 242 -> 143 us (step 832 -> 626 us)
 
 typedef int mx_i4 __attribute__((ext_vector_type(4)));
 
@@ -1533,9 +1533,9 @@ static hipError_t gate_up_typed(const BatchArgs &a, hipStream_t s) {
     const int lds = stream_lds<TY, 2>(valu_cap(a, TY), a.hidden / 256, 2) - al16(GridLDS<TY>::BYTES);
     const int grid = SHARED ? cdiv(a.n_tokens, a.tc) * cdiv(a.ffn_s, a.rt_gu_s) : a.max_chunks * cdiv(a.ffn_r, a.rt_gu_r);
     // Routed IQ chunks left to the VALU beside the matrix cores: one-token
-    // chunks in their own launch, then the rest (measured on MI355X at the
-    // configs[3] shapes: 378.7 -> 369.8 us per step; the fused rows for
-    // two-token chunks too measured slower, 405 us).
+    // chunks in their own launch, then the rest (64 tokens, chunks below four on
+    // the VALU beside the f16 form of the matrix-core streams: 378.7 -> 369.8 us
+    // per step; the fused rows for two-token chunks too measured slower, 405 us).
     if constexpr (!SHARED && (TY == T_IQ2_S || TY == T_IQ3_S)) {
         if (a.mx) {
             hipError_t e = allow_lds(k_mb_gate_up<TY, SHARED, 1>, lds);
@@ -1558,10 +1558,9 @@ static hipError_t down_typed(const BatchArgs &a, hipStream_t s) {
     const int lds = stream_lds<TY, 1>(valu_cap(a, TY), (SHARED ? a.ffn_s : a.ffn_r) / 256, 2) - al16(GridLDS<TY>::BYTES);
     const int grid = SHARED ? cdiv(a.n_tokens, a.tc) * cdiv(a.hidden, a.rt_d_s) : a.max_chunks * cdiv(a.hidden, a.rt_d_r);
     // Routed IQ downs beside the matrix cores taking every chunk of 2+ tokens:
-    // the VALU chunks all hold one token and run the fused rows (measured on
-    // MI355X at the configs[3] shapes: 365.5 -> 359-362 us per step; with
-    // 2-token chunks also left to the VALU, a second launch for them made the
-    // split slower, 382 against 370 us).
+    // the VALU chunks all hold one token and run the fused rows (64 tokens, as
+    // above: 365.5 -> 359-362 us per step; with 2-token chunks also left to the
+    // VALU, a second launch for them made the split slower, 382 against 370 us).
     if constexpr (!SHARED && (TY == T_IQ2_S || TY == T_IQ3_S)) {
         if (a.mx && a.mx_min <= 2) {
             const hipError_t e = allow_lds(k_mb_down<TY, SHARED, 1>, lds);

@@ -5,7 +5,7 @@ crates/bridge-kernels-reference/src/moe.rs:64-147, called per token by
 crates/bridge-runtime/src/hy3_scalar.rs:504-650).  Every token of a batch must
 come out bit-identical to the CPU oracle's moe_routed_by_id on that token
 alone, whatever the grouping: hot experts split over several chunks, ragged
-row tiles, one token, the BASELINE configs[3] shape with Zipf-skewed routing.
+row tiles, one token, the full layer's shape with Zipf-skewed routing.
 """
 import numpy as np
 import pytest
@@ -33,7 +33,7 @@ def _same(a, b):
 
 
 def zipf_routing(oracle, n_tokens, n_experts, top_k, seed, s=1.1):
-    """Per-token softmax top-k of seeded Zipf-skewed logits (the configs[3] routing)."""
+    """Per-token softmax top-k of seeded Zipf-skewed logits (a batch whose hot experts repeat)."""
     logits = synth.zipf_routes(n_tokens, n_experts, top_k, s, seed)
     ids = np.zeros((n_tokens, top_k), np.uint32)
     coefs = np.zeros((n_tokens, top_k), np.float32)
@@ -263,7 +263,7 @@ def test_batch_async_invalid_device_ids_leave_the_output_unchanged(be, oracle, s
 
 
 def test_batch_config4_shapes_zipf_bit_exact(be, oracle):
-    """BASELINE configs[3]: 64 tokens, hidden 4096, routed IQ2_S/IQ3_S ffn 1536,
+    """64 tokens, hidden 4096, routed IQ2_S/IQ3_S ffn 1536,
     Q4_K/Q5_K shared ffn 4096, top-8 of Zipf(1.1) logits (over 32 experts here so
     the oracle finishes in seconds; hot experts span several chunks)."""
     layer = Layer(be, oracle, 32, 4096, 1536, 4096, (IQ2_S, IQ3_S, Q4_K, Q5_K), seed=71)

@@ -121,7 +121,7 @@ def test_tile_copies_with_an_iq_shared_expert(be, oracle, types):
 
 
 def test_tile_copies_config3_shapes_zipf_bit_exact(be, oracle):
-    """BASELINE configs[3] shapes (hidden 4096, routed IQ2_S/IQ3_S ffn 1536,
+    """A step of the full layer (hidden 4096, routed IQ2_S/IQ3_S ffn 1536,
     Q4_K/Q5_K shared ffn 4096, 64 tokens of Zipf(1.1) top-8) over 32 experts,
     every expert copied, the default engine, two calls."""
     layer = Layer(be, oracle, 32, 4096, 1536, 4096, (IQ2_S, IQ3_S, Q4_K, Q5_K), seed=171)

@@ -10,7 +10,7 @@
   caller-supplied Q8_K (NonFiniteQ8Scale before any write).
 * lbh_gemv_dequant_* is ReferenceExecutionMode::DequantF32
   (crates/bridge-kernels-reference/src/gemv.rs:305-328): bit-exact against the
-  oracle's dot_dequant_row at the configs[0] shape, ragged shapes and an
+  oracle's dot_dequant_row at 4096 x 4096, ragged shapes and an
   order-sensitive row whose sequential sum is hand-computed.
 * The checked matvec's mixed-error precedence (destination before dimensions,
   input before scratch size) matches the reference order.

@@ -6,7 +6,7 @@ token t's Q8_K row, bit for bit: random blocks, negative d/dmin, the integer
 extremes (scale 63, mins 63, 5-bit quants 31, activations at +-127), ragged row
 and token counts (row and token tiles not multiples of a workgroup's), every
 form (chains split over waves, 2 x 2 tiles in LDS, tokens in LDS and three
-passes) and the rule that picks one, and the BASELINE configs[4] shape
+passes) and the rule that picks one, and the full prefill shape
 (Q5_K 12288 x 4096, 512 tokens) in full.
 """
 import numpy as np
@@ -130,7 +130,7 @@ def test_gemm_requires_preparation_and_workspace(be, oracle):
 
 
 def test_gemm_config5_full_shape_bit_exact(be, oracle):
-    """BASELINE configs[4]: Q8_K activations [512 x 4096] x Q5_K [12288 x 4096]."""
+    """Q8_K activations [512 x 4096] x Q5_K [12288 x 4096]."""
     rows, k, n = 12288, 4096, 512
     w = synth.random_matrix(Q5_K, rows, k, seed=41)
     q8 = q8_rows(oracle, np.random.default_rng(42).standard_normal((n, k)).astype(np.float32))

@@ -51,7 +51,7 @@ def small(be, oracle):
 
 @pytest.fixture(scope="module")
 def config3(be, oracle):
-    # BASELINE configs[2] shapes with 16 experts (the per-token work of top-8 is the same).
+    # The 192-expert layer's shapes with 16 experts (the per-token work of top-8 is the same).
     return Layer(be, oracle, 16, 4096, 1536, 4096, (IQ2_S, IQ3_S, Q4_K, Q5_K), seed=23)
 
 

@@ -1,12 +1,12 @@
 """GPU parity of the MoE paths on 192-expert layers, the router's summation
 order and bounded waits, and the largest single-token down launch.
 
-* 192 routed experts (the BASELINE configs[2]/[3] expert count) at hidden 4096
-  with the configs' shared expert (Q4_K/Q5_K, ffn 4096) and a reduced routed
+* 192 routed experts at hidden 4096
+  with the full layer's shared expert (Q4_K/Q5_K, ffn 4096) and a reduced routed
   ffn of 512 so the layer uploads in seconds: the device-router block decode
   (lbh_moe_block_forward) and the 64-token batched decode over Zipf(1.1)
   routes, where most of the ~120 experts hit get chunks of 1-3 tokens (the
-  engine mix the configs[3] bench times), every token bit-exact against the
+  mix that the bench's batched step times), every token bit-exact against the
   oracle's moe_routed_by_id (crates/bridge-kernels-reference/src/moe.rs:64-147).
 * The router logit is one sequential f32 chain (dot_f32_row,
   crates/bridge-kernels-reference/src/gemv.rs:286-303): for inputs

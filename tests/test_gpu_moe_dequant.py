@@ -4,7 +4,7 @@ ReferenceExecutionMode::DequantF32: every matvec is dot_dequant_row,
 gemv.rs:33-41) through lbh_moe_routed_by_id_dequant_f32_into.  Outputs and
 error payloads are compared bit for bit with the oracle run in the same mode
 (oracle/lb_oracle.c lbo_moe_routed_by_id with LBO_MODE_DEQUANT_F32): random
-routes at small and at the configs[2] shapes, the routing errors, a non-finite
+routes at small and at the full layer's shapes, the routing errors, a non-finite
 input, a SwiGLU overflow and an accumulation overflow (output left as the
 reference leaves it)."""
 import numpy as np
@@ -74,7 +74,7 @@ def test_dequant_moe_bit_exact(be, oracle, small, seed):
 
 
 def test_dequant_moe_configs2_shapes_bit_exact(be, oracle):
-    """configs[2] widths (hidden 4096, routed ffn 1536, Q4_K/Q5_K shared ffn 4096), top-8 of 12 experts."""
+    """The full layer's widths (hidden 4096, routed ffn 1536, Q4_K/Q5_K shared ffn 4096), top-8 of 12 experts."""
     layer = Layer(be, oracle, 12, 4096, 1536, 4096, (IQ2_S, IQ3_S, Q4_K, Q5_K), seed=71)
     rng = np.random.default_rng(72)
     ids = np.sort(rng.choice(12, 8, replace=False)).astype(np.uint32)

@@ -1,4 +1,4 @@
-"""The MoE layer at its production size (BASELINE configs[2]/[3]): 192 routed
+"""The MoE layer at its production size: 192 routed
 experts, IQ2_S gate/up 1536x4096 and IQ3_S down 4096x1536, a Q4_K/Q5_K shared
 expert with ffn 4096, an F32 router 4096x192 with softmax top-8.  Every output
 is compared bit for bit with the oracle's moe_routed_by_id
