@@ -1601,6 +1601,11 @@ static hipError_t mx_down_launch(const BatchArgs &a, hipStream_t s) {
 template <int TY, bool SHARED>
 static hipError_t mx_gate_up_launches(const BatchArgs &a, hipStream_t s) {
     if constexpr (SHARED) {
+        // Gate and up apart while that takes no more than a workgroup per CU (whole
+        // steps, apart / together, shared width 4096: 16 tokens, 64 workgroups, 80 /
+        // 87 us, 48 tokens, 192 workgroups, 99.6 / 95.4; width 1536: 64 tokens, 96
+        // workgroups, 144 / 145, 96 tokens, 144 workgroups, 174 / 167).
+        if (cdiv(a.n_tokens, a.tc) * cdiv(a.ffn_s, a.mx_rows_gu) <= 128) return mx_gate_up_launch<TY, true, false, 1>(a, s);
         return mx_gate_up_launch<TY, true, false, 2>(a, s);
     } else {
         hipError_t e = hipSuccess;
@@ -1623,7 +1628,13 @@ static hipError_t mx_gate_up_launches(const BatchArgs &a, hipStream_t s) {
 template <int TY, bool SHARED>
 static hipError_t mx_down_launches(const BatchArgs &a, hipStream_t s) {
     if constexpr (SHARED) {
-        return mx_down_launch<TY, true, false>(a, s);
+        // A tile per wave instead of four, one after the other, while the default
+        // rows give less than a workgroup per CU (hidden 4096 from IQ3_S 1536: 16
+        // workgroups for up to 16 tokens; step of 5 tokens with copies 90 -> 81 us,
+        // from 4096 105 -> 78).
+        BatchArgs b = a;
+        if (cdiv(a.n_tokens, a.tc) * cdiv(a.hidden, a.mx_rows_d) < 256 && a.mx_rows_d > 64) b.mx_rows_d = 64;
+        return mx_down_launch<TY, true, false>(b, s);
     } else {
         hipError_t e = hipSuccess;
         bool kt = a.shared_kt;

@@ -155,6 +155,11 @@ def test_batch_type_sets(be, oracle, types, ffn_s):
     want = oracle_batch(oracle, layer, ids, coefs, xs)
     got = run_checked(be, layer, ids, coefs, xs)
     assert all(_same(got[t], want[t]) for t in range(11))
+    # 48 to 816 workgroups: the wider shared gate and up in one launch, not apart
+    layer.moe.set_batch_engine(1, 16, 16)
+    layer.moe.set_batch_tiles(4)
+    got = run_checked(be, layer, ids, coefs, xs)
+    assert all(_same(got[t], want[t]) for t in range(11))
 
 
 def test_batch_device_routing_softmax_and_sigmoid(be, oracle, small):
